@@ -10,16 +10,18 @@
 // Rows of up to 1024 values: a segment of G lanes (G = 4, 16 or 64, the smallest that holds
 // the row in at most 16 values per lane) owns one row and keeps it in registers, so every
 // statistic (max, sums, mean, variance) is a segment reduction over registers and no value is
-// read twice.  Lane s of a segment holds chunks s, s + G, s + 2G, ... of the row (a chunk is 4
-// values with 16-byte loads when C % 4 == 0 and the pointers are 16-byte aligned, else 1), so
-// one load instruction covers G consecutive chunks of every row in the wave.
+// read twice.  Lane s of a segment holds chunks s, s + G, s + 2G, ... of the row, so one load
+// instruction covers G consecutive chunks of every row in the wave.
+// Rows of up to 32768 values: one work-group per row holds it the same way (see row_block).
 // Longer rows: one 256-thread work-group per row, streaming the row from L2 once per pass.
+//
+// A chunk is 4 values, loaded and stored as one 16-byte access that needs only the 4-byte
+// alignment every row has: rows of any C and any pointer take the same path, and only the
+// chunk that holds a row's end goes value by value.
 #include "dh_common.hpp"
 
 namespace dh {
 namespace {
-
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 template <int G>
 __device__ inline float seg_sum(float v) {
@@ -34,40 +36,40 @@ __device__ inline float seg_max(float v) {
     return v;
 }
 
-// NV chunks of VEC values of one row, chunk t of lane s at element VEC (t G + s).
-template <int G, int NV, int VEC>
+// 16-byte access at 4-byte alignment.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// NV chunks of 4 values of one row over g lanes, chunk t of lane s at element 4 (t g + s).
+template <int NV>
 struct Row {
-    float v[NV][VEC];
-    __device__ void load(const float* __restrict__ p, int C, int s, float fill) {
+    float v[NV][4];
+    __device__ void load(const float* __restrict__ p, int C, int s, int g, float fill) {
 #pragma unroll
         for (int t = 0; t < NV; ++t) {
-            const int e = VEC * (t * G + s);
-            if (VEC == 4) {
-                if (e < C) {
-                    const f4 x = *reinterpret_cast<const f4*>(p + e);
+            const int e = 4 * (t * g + s);
+            if (e + 4 <= C) {
+                const f4u x = *reinterpret_cast<const f4u*>(p + e);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[t][q] = x[q];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) v[t][q] = fill;
-                }
+                for (int q = 0; q < 4; ++q) v[t][q] = x[q];
             } else {
-                v[t][0] = e < C ? p[e] : fill;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[t][q] = e + q < C ? p[e + q] : fill;
             }
         }
     }
     // Non-temporal: the output row is streamed out and not read again here, and keeping it
     // out of the caches leaves them to the inputs.
-    __device__ void store(float* __restrict__ p, int C, int s) const {
+    __device__ void store(float* __restrict__ p, int C, int s, int g) const {
 #pragma unroll
         for (int t = 0; t < NV; ++t) {
-            const int e = VEC * (t * G + s);
-            if (e >= C) continue;
-            if (VEC == 4) {
-                __builtin_nontemporal_store(f4{v[t][0], v[t][1], v[t][2], v[t][3]},
-                                            reinterpret_cast<f4*>(p + e));
+            const int e = 4 * (t * g + s);
+            if (e + 4 <= C) {
+                __builtin_nontemporal_store(f4u{v[t][0], v[t][1], v[t][2], v[t][3]},
+                                            reinterpret_cast<f4u*>(p + e));
             } else {
-                __builtin_nontemporal_store(v[t][0], p + e);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (e + q < C) __builtin_nontemporal_store(v[t][q], p + e + q);
             }
         }
     }
@@ -75,143 +77,223 @@ struct Row {
 
 #define ROW_LOOP(stmt)                              \
     _Pragma("unroll") for (int t = 0; t < NV; ++t)  \
-        _Pragma("unroll") for (int q = 0; q < VEC; ++q) { stmt; }
+        _Pragma("unroll") for (int q = 0; q < 4; ++q) { stmt; }
 
-// Common prologue: 256 threads = 256 / G rows per work-group; a row index past R exits the
-// whole segment (segments never straddle a wave, so the reductions stay within live lanes).
+// Reductions over the lanes that hold a row: a segment of G lanes within a wave, or a whole
+// work-group (wave sums through LDS, added in wave order).
+template <int G>
+struct SegLanes {
+    __device__ float sum(float v) const { return seg_sum<G>(v); }
+    __device__ float max(float v) const { return seg_max<G>(v); }
+};
+
+template <typename Op>
+__device__ inline float block_reduce(float v, Op op, float* red) {
+    v = wave_reduce(v, op);
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    __syncthreads();   // red[] may still be read from a previous reduction
+    if ((threadIdx.x & 63) == 0) red[w] = v;
+    __syncthreads();
+    v = red[0];
+    for (int i = 1; i < nw; ++i) v = op(v, red[i]);
+    return v;
+}
+
+struct BlockLanes {
+    float* red;   // 16 floats of LDS
+    __device__ float sum(float v) const { return block_reduce(v, OpSum(), red); }
+    __device__ float max(float v) const { return block_reduce(v, OpMax(), red); }
+};
+
+// The four row operations on a row held by g lanes, lane s (`L` reduces over them); off is the
+// row's first element.
+template <int NV, typename L>
+__device__ inline void softmax_row(const float* __restrict__ X, float* __restrict__ Y, size_t off,
+                                   int C, int s, int g, L lanes, int logsm) {
+    Row<NV> x;
+    x.load(X + off, C, s, g, -INFINITY);
+    float mx = -INFINITY;
+    ROW_LOOP(mx = fmaxf(mx, x.v[t][q]));
+    mx = lanes.max(mx);
+    float sum = 0.f;
+    if (logsm) {
+        ROW_LOOP(sum += __expf(x.v[t][q] - mx));
+        const float lse = mx + __logf(lanes.sum(sum));
+        ROW_LOOP(x.v[t][q] -= lse);
+    } else {
+        ROW_LOOP(x.v[t][q] = __expf(x.v[t][q] - mx); sum += x.v[t][q]);
+        const float inv = 1.f / lanes.sum(sum);
+        ROW_LOOP(x.v[t][q] *= inv);
+    }
+    x.store(Y + off, C, s, g);
+}
+
+// softmax:     gx (+)= y (g - sum(g y))
+// log_softmax: gx (+)= g - exp(y) sum(g)      (y = log_softmax(x), so exp(y) = softmax(x))
+template <int NV, typename L>
+__device__ inline void softmax_bwd_row(const float* __restrict__ Yf, const float* __restrict__ Gr,
+                                       float* __restrict__ GX, size_t off, int C, int s, int g,
+                                       L lanes, int logsm, int acc) {
+    Row<NV> y, d;
+    y.load(Yf + off, C, s, g, 0.f);
+    d.load(Gr + off, C, s, g, 0.f);
+    float red = 0.f;
+    if (logsm) {
+        ROW_LOOP(red += d.v[t][q]);
+    } else {
+        ROW_LOOP(red += d.v[t][q] * y.v[t][q]);
+    }
+    red = lanes.sum(red);
+    if (logsm) {
+        ROW_LOOP(y.v[t][q] = d.v[t][q] - __expf(y.v[t][q]) * red);
+    } else {
+        ROW_LOOP(y.v[t][q] = y.v[t][q] * (d.v[t][q] - red));
+    }
+    if (acc) {
+        Row<NV> o;
+        o.load(GX + off, C, s, g, 0.f);
+        ROW_LOOP(y.v[t][q] += o.v[t][q]);
+    }
+    y.store(GX + off, C, s, g);
+}
+
+// Per-row mean and inverse standard deviation (biased variance, eps 1e-5) from registers;
+// padding chunks hold 0 and are excluded from the variance by the element count.
+template <int NV, typename L>
+__device__ inline void row_stats(const Row<NV>& x, int C, int s, int g, L lanes, float& mu,
+                                 float& inv_std) {
+    float sum = 0.f;
+    ROW_LOOP(sum += x.v[t][q]);
+    mu = lanes.sum(sum) / (float)C;
+    float var = 0.f;
+#pragma unroll
+    for (int t = 0; t < NV; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float d = 4 * (t * g + s) + q < C ? x.v[t][q] - mu : 0.f;
+            var += d * d;
+        }
+    var = lanes.sum(var) / (float)C;
+    inv_std = rsqrtf(var + 1e-5f);
+}
+
+template <int NV, typename L>
+__device__ inline void layer_norm_row(const float* __restrict__ X, float* __restrict__ Y,
+                                      size_t off, int C, int s, int g, L lanes) {
+    Row<NV> x;
+    x.load(X + off, C, s, g, 0.f);
+    float mu, inv_std;
+    row_stats(x, C, s, g, lanes, mu, inv_std);
+    ROW_LOOP(x.v[t][q] = (x.v[t][q] - mu) * inv_std);
+    x.store(Y + off, C, s, g);
+}
+
+// gx (+)= inv_std / C (C dy - sum(dy) - y sum(dy y)), inv_std recomputed from x.
+template <int NV, typename L>
+__device__ inline void layer_norm_bwd_row(const float* __restrict__ X, const float* __restrict__ Yf,
+                                          const float* __restrict__ DY, float* __restrict__ GX,
+                                          size_t off, int C, int s, int g, L lanes, int acc) {
+    float mu, inv_std;
+    {
+        Row<NV> x;
+        x.load(X + off, C, s, g, 0.f);
+        row_stats(x, C, s, g, lanes, mu, inv_std);
+    }
+    Row<NV> y, dy;
+    y.load(Yf + off, C, s, g, 0.f);
+    dy.load(DY + off, C, s, g, 0.f);
+    float sdy = 0.f, sdyy = 0.f;
+    ROW_LOOP(sdy += dy.v[t][q]; sdyy += dy.v[t][q] * y.v[t][q]);
+    sdy = lanes.sum(sdy);
+    sdyy = lanes.sum(sdyy);
+    const float k = inv_std / (float)C, fc = (float)C;
+    ROW_LOOP(y.v[t][q] = k * (fc * dy.v[t][q] - sdy - y.v[t][q] * sdyy));
+    if (acc) {
+        Row<NV> o;
+        o.load(GX + off, C, s, g, 0.f);
+        ROW_LOOP(y.v[t][q] += o.v[t][q]);
+    }
+    y.store(GX + off, C, s, g);
+}
+
+// Segment kernels, rows of at most 16 G values: 256 threads = 256 / G rows per work-group; a
+// row index past R exits the whole segment (segments never straddle a wave, so the reductions
+// stay within live lanes).
 #define SEG_PROLOGUE()                                                    \
     const int s = threadIdx.x & (G - 1);                                  \
     const int row = blockIdx.x * (256 / G) + threadIdx.x / G;             \
     if (row >= R) return;                                                 \
     const size_t off = (size_t)row * C;
 
-template <int G, int NV, int VEC>
+template <int G>
 __global__ void __launch_bounds__(256) softmax_seg(const float* __restrict__ X,
                                                    float* __restrict__ Y, int R, int C, int logsm) {
     SEG_PROLOGUE();
-    Row<G, NV, VEC> x;
-    x.load(X + off, C, s, -INFINITY);
-    float mx = -INFINITY;
-    ROW_LOOP(mx = fmaxf(mx, x.v[t][q]));
-    mx = seg_max<G>(mx);
-    float sum = 0.f;
-    ROW_LOOP(sum += __expf(x.v[t][q] - mx));
-    sum = seg_sum<G>(sum);
-    if (logsm) {
-        const float lse = mx + __logf(sum);
-        ROW_LOOP(x.v[t][q] -= lse);
-    } else {
-        const float inv = 1.f / sum;
-        ROW_LOOP(x.v[t][q] = __expf(x.v[t][q] - mx) * inv);
-    }
-    x.store(Y + off, C, s);
+    softmax_row<4>(X, Y, off, C, s, G, SegLanes<G>(), logsm);
 }
-
-// softmax:     gx (+)= y (g - sum(g y))
-// log_softmax: gx (+)= g - exp(y) sum(g)      (y = log_softmax(x), so exp(y) = softmax(x))
-template <int G, int NV, int VEC>
+template <int G>
 __global__ void __launch_bounds__(256) softmax_bwd_seg(const float* __restrict__ Yf,
                                                        const float* __restrict__ Gr,
                                                        float* __restrict__ GX, int R, int C,
                                                        int logsm, int acc) {
     SEG_PROLOGUE();
-    Row<G, NV, VEC> y, g;
-    y.load(Yf + off, C, s, 0.f);
-    g.load(Gr + off, C, s, 0.f);
-    float red = 0.f;
-    if (logsm) {
-        ROW_LOOP(red += g.v[t][q]);
-    } else {
-        ROW_LOOP(red += g.v[t][q] * y.v[t][q]);
-    }
-    red = seg_sum<G>(red);
-    if (logsm) {
-        ROW_LOOP(y.v[t][q] = g.v[t][q] - __expf(y.v[t][q]) * red);
-    } else {
-        ROW_LOOP(y.v[t][q] = y.v[t][q] * (g.v[t][q] - red));
-    }
-    if (acc) {
-        Row<G, NV, VEC> o;
-        o.load(GX + off, C, s, 0.f);
-        ROW_LOOP(y.v[t][q] += o.v[t][q]);
-    }
-    y.store(GX + off, C, s);
+    softmax_bwd_row<4>(Yf, Gr, GX, off, C, s, G, SegLanes<G>(), logsm, acc);
 }
-
-// Per-row mean and inverse standard deviation (biased variance, eps 1e-5) from registers;
-// padding chunks hold 0 and are excluded from the variance by the element count.
-template <int G, int NV, int VEC>
-__device__ inline void row_stats(const Row<G, NV, VEC>& x, int C, int s, float& mu,
-                                 float& inv_std) {
-    float sum = 0.f;
-    ROW_LOOP(sum += x.v[t][q]);
-    mu = seg_sum<G>(sum) / (float)C;
-    float var = 0.f;
-#pragma unroll
-    for (int t = 0; t < NV; ++t)
-#pragma unroll
-        for (int q = 0; q < VEC; ++q) {
-            const float d = VEC * (t * G + s) + q < C ? x.v[t][q] - mu : 0.f;
-            var += d * d;
-        }
-    var = seg_sum<G>(var) / (float)C;
-    inv_std = rsqrtf(var + 1e-5f);
-}
-
-template <int G, int NV, int VEC>
+template <int G>
 __global__ void __launch_bounds__(256) layer_norm_seg(const float* __restrict__ X,
                                                       float* __restrict__ Y, int R, int C) {
     SEG_PROLOGUE();
-    Row<G, NV, VEC> x;
-    x.load(X + off, C, s, 0.f);
-    float mu, inv_std;
-    row_stats(x, C, s, mu, inv_std);
-    ROW_LOOP(x.v[t][q] = (x.v[t][q] - mu) * inv_std);
-    x.store(Y + off, C, s);
+    layer_norm_row<4>(X, Y, off, C, s, G, SegLanes<G>());
 }
-
-// gx (+)= inv_std / C (C dy - sum(dy) - y sum(dy y)), inv_std recomputed from x.
-template <int G, int NV, int VEC>
+template <int G>
 __global__ void __launch_bounds__(256) layer_norm_bwd_seg(const float* __restrict__ X,
                                                           const float* __restrict__ Yf,
                                                           const float* __restrict__ DY,
                                                           float* __restrict__ GX, int R, int C,
                                                           int acc) {
     SEG_PROLOGUE();
-    float mu, inv_std;
-    {
-        Row<G, NV, VEC> x;
-        x.load(X + off, C, s, 0.f);
-        row_stats(x, C, s, mu, inv_std);
-    }
-    Row<G, NV, VEC> y, dy;
-    y.load(Yf + off, C, s, 0.f);
-    dy.load(DY + off, C, s, 0.f);
-    float sdy = 0.f, sdyy = 0.f;
-    ROW_LOOP(sdy += dy.v[t][q]; sdyy += dy.v[t][q] * y.v[t][q]);
-    sdy = seg_sum<G>(sdy);
-    sdyy = seg_sum<G>(sdyy);
-    const float k = inv_std / (float)C, fc = (float)C;
-    ROW_LOOP(y.v[t][q] = k * (fc * dy.v[t][q] - sdy - y.v[t][q] * sdyy));
-    if (acc) {
-        Row<G, NV, VEC> o;
-        o.load(GX + off, C, s, 0.f);
-        ROW_LOOP(y.v[t][q] += o.v[t][q]);
-    }
-    y.store(GX + off, C, s);
+    layer_norm_bwd_row<4>(X, Yf, DY, GX, off, C, s, G, SegLanes<G>(), acc);
 }
 
-// ---- long rows: one work-group of 256 threads per row, streaming ---------------------------
-template <typename Op>
-__device__ inline float block_reduce(float v, Op op, float* red) {
-    v = wave_reduce(v, op);
-    const int w = threadIdx.x >> 6;
-    __syncthreads();   // red[] may still be read from a previous reduction
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    return op(op(red[0], red[1]), op(red[2], red[3]));
+// row_block: one work-group per row of 1025 to 32768 values, held in registers at 4 NV values
+// per lane (NV = 4 up to 16384, then 8; blockDim.x = the fewest whole waves that hold it).
+// Bound by HBM: each input is read once and the output written once, where the streaming
+// kernels below read the row once per pass.  Same box, 4096 x 5000 log_softmax, streaming /
+// registers: forward 62.6 / 25.5 us, backward 59.9 / 38.2 us (6.4 and 6.4 TB/s).
+template <int NV>
+__global__ void __launch_bounds__(1024) softmax_block(const float* __restrict__ X,
+                                                      float* __restrict__ Y, int C, int logsm) {
+    __shared__ float red[16];
+    softmax_row<NV>(X, Y, (size_t)blockIdx.x * C, C, threadIdx.x, blockDim.x, BlockLanes{red},
+                    logsm);
+}
+template <int NV>
+__global__ void __launch_bounds__(1024) softmax_bwd_block(const float* __restrict__ Yf,
+                                                          const float* __restrict__ Gr,
+                                                          float* __restrict__ GX, int C, int logsm,
+                                                          int acc) {
+    __shared__ float red[16];
+    softmax_bwd_row<NV>(Yf, Gr, GX, (size_t)blockIdx.x * C, C, threadIdx.x, blockDim.x,
+                        BlockLanes{red}, logsm, acc);
+}
+template <int NV>
+__global__ void __launch_bounds__(1024) layer_norm_block(const float* __restrict__ X,
+                                                         float* __restrict__ Y, int C) {
+    __shared__ float red[16];
+    layer_norm_row<NV>(X, Y, (size_t)blockIdx.x * C, C, threadIdx.x, blockDim.x, BlockLanes{red});
+}
+template <int NV>
+__global__ void __launch_bounds__(1024) layer_norm_bwd_block(const float* __restrict__ X,
+                                                             const float* __restrict__ Yf,
+                                                             const float* __restrict__ DY,
+                                                             float* __restrict__ GX, int C,
+                                                             int acc) {
+    __shared__ float red[16];
+    layer_norm_bwd_row<NV>(X, Yf, DY, GX, (size_t)blockIdx.x * C, C, threadIdx.x, blockDim.x,
+                           BlockLanes{red}, acc);
 }
 
+// ---- rows above 32768 values: one work-group of 256 threads per row, streaming --------------
 __global__ void __launch_bounds__(256) softmax_blk(const float* __restrict__ X,
                                                    float* __restrict__ Y, int C, int logsm) {
     __shared__ float red[4];
@@ -337,42 +419,28 @@ __global__ void __launch_bounds__(256) bias_grad_final(const float* __restrict__
 }
 
 // ---- dispatch --------------------------------------------------------------------------------
-constexpr int SEG_MAX_C = 1024;
+constexpr int SEG_MAX_C = 1024, BLOCK_MAX_C = 32768;
 
-bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
-template <int G>
-constexpr unsigned seg_grid(int R) { return (unsigned)((R + 256 / G - 1) / (256 / G)); }
-
-template <int G, int NV, int VEC>
-int launch_softmax(const float* X, float* Y, int R, int C, int lg) {
-    softmax_seg<G, NV, VEC><<<seg_grid<G>(R), 256, 0, stream()>>>(X, Y, R, C, lg);
-    return check_launch("dh_row_softmax");
-}
-template <int G, int NV, int VEC>
-int launch_softmax_bwd(const float* Y, const float* Gr, float* GX, int R, int C, int lg, int acc) {
-    softmax_bwd_seg<G, NV, VEC><<<seg_grid<G>(R), 256, 0, stream()>>>(Y, Gr, GX, R, C, lg, acc);
-    return check_launch("dh_row_softmax_bwd");
-}
-template <int G, int NV, int VEC>
-int launch_layer_norm(const float* X, float* Y, int R, int C) {
-    layer_norm_seg<G, NV, VEC><<<seg_grid<G>(R), 256, 0, stream()>>>(X, Y, R, C);
-    return check_launch("dh_layer_norm");
-}
-template <int G, int NV, int VEC>
-int launch_layer_norm_bwd(const float* X, const float* Y, const float* DY, float* GX, int R, int C,
-                          int acc) {
-    layer_norm_bwd_seg<G, NV, VEC><<<seg_grid<G>(R), 256, 0, stream()>>>(X, Y, DY, GX, R, C, acc);
-    return check_launch("dh_layer_norm_bwd");
-}
-
-// The smallest segment that holds a row of C values in at most 16 values per lane (chunks of 4
-// when `vec`).
-#define SEG_DISPATCH(C, vec, FN, ...)                                                      \
-    ((vec) ? ((C) / 4 <= 16 ? FN<4, 4, 4>(__VA_ARGS__)                                     \
-                            : (C) / 4 <= 64 ? FN<16, 4, 4>(__VA_ARGS__) : FN<64, 4, 4>(__VA_ARGS__)) \
-           : ((C) <= 64 ? FN<4, 16, 1>(__VA_ARGS__)                                        \
-                        : (C) <= 256 ? FN<16, 16, 1>(__VA_ARGS__) : FN<64, 16, 1>(__VA_ARGS__)))
+// Launches the segment, row_block or streaming form of a row operation for R rows of C values:
+// KERNEL_seg<G>(ARGS, R, C, ...), KERNEL_block<NV>(ARGS, C, ...) or KERNEL_blk(ARGS, C, ...).
+#define ROW_LAUNCH(KERNEL, WHAT, R, C, ARGS, ...)                                               \
+    do {                                                                                        \
+        if ((C) <= 64) KERNEL##_seg<4><<<((R) + 63) / 64, 256, 0, stream()>>>(                  \
+            UNPAREN ARGS, R, C __VA_OPT__(, ) __VA_ARGS__);                                     \
+        else if ((C) <= 256) KERNEL##_seg<16><<<((R) + 15) / 16, 256, 0, stream()>>>(           \
+            UNPAREN ARGS, R, C __VA_OPT__(, ) __VA_ARGS__);                                     \
+        else if ((C) <= SEG_MAX_C) KERNEL##_seg<64><<<((R) + 3) / 4, 256, 0, stream()>>>(       \
+            UNPAREN ARGS, R, C __VA_OPT__(, ) __VA_ARGS__);                                     \
+        else if ((C) <= BLOCK_MAX_C / 2) KERNEL##_block<4><<<R, 64 * (((C) + 1023) / 1024), 0,  \
+                                                             stream()>>>(                       \
+            UNPAREN ARGS, C __VA_OPT__(, ) __VA_ARGS__);                                        \
+        else if ((C) <= BLOCK_MAX_C) KERNEL##_block<8><<<R, 64 * (((C) + 2047) / 2048), 0,      \
+                                                         stream()>>>(                           \
+            UNPAREN ARGS, C __VA_OPT__(, ) __VA_ARGS__);                                        \
+        else KERNEL##_blk<<<R, 256, 0, stream()>>>(UNPAREN ARGS, C __VA_OPT__(, ) __VA_ARGS__); \
+        return check_launch(WHAT);                                                              \
+    } while (0)
+#define UNPAREN(...) __VA_ARGS__
 
 int check_rows(const char* op, int R, int C) {
     if (R < 0 || C < 0) return set_error(DH_ERR_INVALID, "%s: negative shape", op);
@@ -391,12 +459,7 @@ int dh_row_softmax(const float* X, float* Y, int R, int C, int log_softmax) {
     DH_TRY(check_rows("dh_row_softmax", R, C));
     if (R == 0 || C == 0) return DH_OK;
     if (!X || !Y) return set_error(DH_ERR_INVALID, "dh_row_softmax: null pointer");
-    if (C > SEG_MAX_C) {
-        softmax_blk<<<R, 256, 0, stream()>>>(X, Y, C, log_softmax);
-        return check_launch("dh_row_softmax");
-    }
-    return SEG_DISPATCH(C, C % 4 == 0 && aligned16(X) && aligned16(Y), launch_softmax, X, Y, R, C,
-                        log_softmax);
+    ROW_LAUNCH(softmax, "dh_row_softmax", R, C, (X, Y), log_softmax);
 }
 
 int dh_row_softmax_bwd(const float* Y, const float* G, float* GX, int R, int C, int log_softmax,
@@ -405,12 +468,7 @@ int dh_row_softmax_bwd(const float* Y, const float* G, float* GX, int R, int C, 
     DH_TRY(check_rows("dh_row_softmax_bwd", R, C));
     if (R == 0 || C == 0) return DH_OK;
     if (!Y || !G || !GX) return set_error(DH_ERR_INVALID, "dh_row_softmax_bwd: null pointer");
-    if (C > SEG_MAX_C) {
-        softmax_bwd_blk<<<R, 256, 0, stream()>>>(Y, G, GX, C, log_softmax, accumulate);
-        return check_launch("dh_row_softmax_bwd");
-    }
-    return SEG_DISPATCH(C, C % 4 == 0 && aligned16(Y) && aligned16(G) && aligned16(GX),
-                        launch_softmax_bwd, Y, G, GX, R, C, log_softmax, accumulate);
+    ROW_LAUNCH(softmax_bwd, "dh_row_softmax_bwd", R, C, (Y, G, GX), log_softmax, accumulate);
 }
 
 int dh_layer_norm(const float* X, float* Y, int R, int C) {
@@ -418,12 +476,7 @@ int dh_layer_norm(const float* X, float* Y, int R, int C) {
     DH_TRY(check_rows("dh_layer_norm", R, C));
     if (R == 0 || C == 0) return DH_OK;
     if (!X || !Y) return set_error(DH_ERR_INVALID, "dh_layer_norm: null pointer");
-    if (C > SEG_MAX_C) {
-        layer_norm_blk<<<R, 256, 0, stream()>>>(X, Y, C);
-        return check_launch("dh_layer_norm");
-    }
-    return SEG_DISPATCH(C, C % 4 == 0 && aligned16(X) && aligned16(Y), launch_layer_norm, X, Y, R,
-                        C);
+    ROW_LAUNCH(layer_norm, "dh_layer_norm", R, C, (X, Y));
 }
 
 int dh_layer_norm_bwd(const float* X, const float* Y, const float* DY, float* GX, int R, int C,
@@ -432,13 +485,7 @@ int dh_layer_norm_bwd(const float* X, const float* Y, const float* DY, float* GX
     DH_TRY(check_rows("dh_layer_norm_bwd", R, C));
     if (R == 0 || C == 0) return DH_OK;
     if (!X || !Y || !DY || !GX) return set_error(DH_ERR_INVALID, "dh_layer_norm_bwd: null pointer");
-    if (C > SEG_MAX_C) {
-        layer_norm_bwd_blk<<<R, 256, 0, stream()>>>(X, Y, DY, GX, C, accumulate);
-        return check_launch("dh_layer_norm_bwd");
-    }
-    return SEG_DISPATCH(C, C % 4 == 0 && aligned16(X) && aligned16(Y) && aligned16(DY) &&
-                               aligned16(GX),
-                        launch_layer_norm_bwd, X, Y, DY, GX, R, C, accumulate);
+    ROW_LAUNCH(layer_norm_bwd, "dh_layer_norm_bwd", R, C, (X, Y, DY, GX), accumulate);
 }
 
 int dh_linear_bias_grad(const float* Y, float* dY, float* db, int N, int out, int relu,

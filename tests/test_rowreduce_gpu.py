@@ -135,6 +135,45 @@ def test_row_ops_reference_golden_vectors():
     assert np.abs(LdX - GOLD["layer_norm_dX"]).max() <= _tol(GOLD["layer_norm_dX"], C)
 
 
+@pytest.mark.parametrize("C", [1025, 1088, 4099, 16384, 16385, 20002, 32768, 32769])
+@pytest.mark.parametrize("off", [0, 1])
+def test_row_ops_wide_rows(C, off):
+    # Rows held by one work-group (4 values per chunk, 16 or 32 values per lane), its edges,
+    # the streaming form above it, and buffers that start one float past a 16-byte boundary.
+    # Bounds as above, times 4 for the layer norm's two chained reductions.
+    R = 3
+    rng = np.random.default_rng(C + off)
+    X = (rng.standard_normal((R, C)) * 3 + 0.5).astype(np.float32)
+    G = rng.standard_normal((R, C)).astype(np.float32)
+
+    def at(buf):
+        return buf.ptr + 4 * off
+
+    def run(fn, *ins):
+        bufs = []
+        for x in ins:
+            b = DB.from_numpy(np.concatenate([np.zeros(off, np.float32), x.ravel()]))
+            bufs.append(b)
+        out = DB.empty(R * C + off, np.float32)
+        fn(*[at(b) for b in bufs], at(out))
+        return out.numpy()[off:].reshape(R, C)
+
+    X64, G64 = X.astype(np.float64), G.astype(np.float64)
+    for log in (False, True):
+        ref = O.log_softmax_rows(X64) if log else O.softmax_rows(X64)
+        Y = run(lambda x, y: hip.row_softmax(x, y, R, C, log), X)
+        assert np.abs(Y - ref).max() <= _tol(ref, C)
+        gref = O.log_softmax_bwd(X64, G64) if log else O.softmax_bwd(Y.astype(np.float64), G64)
+        got = run(lambda y, g, gx: hip.row_softmax_bwd(y, g, gx, R, C, log), Y, G)
+        assert np.abs(got - gref).max() <= _tol(gref, C)
+    ref = O.layer_norm(X64)
+    Y = run(lambda x, y: hip.layer_norm(x, y, R, C), X)
+    assert np.abs(Y - ref).max() <= 4 * _tol(ref, C)
+    gref = O.layer_norm_bwd(X64, ref, G64)
+    got = run(lambda x, y, dy, gx: hip.layer_norm_bwd(x, y, dy, gx, R, C), X, Y, G)
+    assert np.abs(got - gref).max() <= 4 * _tol(gref, C)
+
+
 def test_row_ops_large_rows_count():
     # Many short rows (the segment kernels' multi-row work-groups with a ragged last group)
     # and the properties that hold at any size: softmax rows sum to 1, layer-norm rows have
