@@ -174,6 +174,22 @@ def test_row_ops_wide_rows(C, off):
     assert np.abs(got - gref).max() <= 4 * _tol(gref, C)
 
 
+@pytest.mark.parametrize("N,out", [(1, 1), (63, 64), (65, 65), (2049, 3), (4096, 257), (20000, 40)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_linear_bias_grad_row_and_partial_remainders(N, out, relu):
+    # Rows taken 8 at a time per wave and partials 16 at a time: remainders of both, one row,
+    # one column.  The mask is exact; sums of N values within 1e-6 sqrt(N) of max |dY| ~ 4.
+    rng = np.random.default_rng(N + out)
+    Y = np.maximum(rng.standard_normal((N, out)), 0).astype(np.float32)
+    dY = rng.standard_normal((N, out)).astype(np.float32)
+    dy, db = DB.from_numpy(dY), DB.from_numpy(np.full(out, 0.5, np.float32))
+    y = DB.from_numpy(Y) if relu else None
+    hip.linear_bias_grad(y, dy, db, N, out, relu=relu, accumulate=True)
+    want = np.where(Y > 0, dY, 0) if relu else dY
+    assert np.array_equal(dy.numpy(), want)
+    assert np.abs(db.numpy() - (0.5 + want.astype(np.float64).sum(0))).max() <= 4e-6 * np.sqrt(N)
+
+
 def test_row_ops_large_rows_count():
     # Many short rows (the segment kernels' multi-row work-groups with a ragged last group)
     # and the properties that hold at any size: softmax rows sum to 1, layer-norm rows have
