@@ -22,112 +22,246 @@
 // (one batched NT product per chunk of slices), a row kernel applies the scale, the causal
 // mask and the softmax (max, exp, sum, divide), O = P V; the backward
 // (runtime/ops/autograd.inc:675-778) recomputes P, then dV += P^T dO, dP = dO V^T,
-// dS = P (dP - rowsum(dP P)), dQ += scale dS K, dK += scale dS^T Q.  Score buffers come from
-// the pool in chunks of slices (at most 256 MB per buffer).
+// dS = P (dP - rowsum(dP P)), dQ += scale dS K, dK += scale dS^T Q.  Causal products leave out
+// what the mask zeroes (F64_SCORES ...).  Score buffers come from the pool in chunks of slices
+// (at most 256 MB per buffer).
+//
+// Bound by the fp64 matrix cores.  16 causal slices of 1024 x 256, forward + backward: 1520 ->
+// 721 us (30 GFLOP visible, 42 TFLOP/s); 4096^3 53.5 -> 60.8 (NN), 65.0 (TN) TFLOP/s of the
+// 70 that a library product reaches here.
 #include "dh_common.hpp"
 
 #include <math.h>
 #include <cstdlib>
+#include <type_traits>
 
 namespace dh {
 namespace {
 
-constexpr int F64_KT = 16;        // k per LDS stage
 constexpr int F64_KC = 256;       // the reference's KC: chains restart every 256 k
 constexpr int F64_THREADS = 256;  // four waves as 2 x 2, each WB x WB blocks of 16 x 16
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 
-template <int WB>
+// Which part of a product a causal attention needs (query row0 + m or key k visible up to the
+// diagonal), so that masked blocks are neither computed nor read:
+//   F64_SCORES     C[m][n]: tiles whose keys n all lie past their queries row0 + m are left out;
+//   F64_TO_DIAG    A[m][k] masked past k = row0 + m: k stops at the end of the tile's queries;
+//   F64_FROM_DIAG  A^T[m][k] (m a key, k a query row0 + k): k starts at the tile's first key.
+// A masked product is an exact zero, and adding it changes no chain, so the results are those
+// of the full product.  The row kernels write zeros up to F64_PAD keys past the diagonal, as
+// far as a tile's edge and a stage's start reach.
+enum { F64_ALL = 0, F64_SCORES, F64_TO_DIAG, F64_FROM_DIAG };
+constexpr int F64_PAD = 80;       // 64-wide tile + 16-deep stage (or 32 + 32)
+
+// Explicitly global pointers: through the argument struct they would become flat loads.
+typedef const double __attribute__((address_space(1)))* GlobalF64;
+typedef const char __attribute__((address_space(1)))* GlobalBytes;
+__device__ double g_zero64;   // zero-initialised, never written
+
+__device__ inline __amdgpu_buffer_rsrc_t f64_rsrc(GlobalBytes p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)p, 0, bytes, 0x00020000);
+}
+// Two doubles at byte offset off; words past the resource's range (F64_OOB always is) read zero.
+// The opaque offset keeps the four 32-bit loads at constant distances, so that the backend
+// merges them into one 128-bit load.
+constexpr int F64_OOB = -16;
+__device__ inline f64x2 f64_load2(__amdgpu_buffer_rsrc_t rs, int off) {
+    asm volatile("" : "+v"(off));
+    float v[4];
+    buf_load_floats<4>(rs, off, v);
+    return __builtin_bit_cast(f64x2, f32x4{v[0], v[1], v[2], v[3]});
+}
+
+struct F64Args {
+    int M, N, K;
+    double alpha;
+    const double* A;
+    int lda;
+    long long sA;
+    const double* B;
+    int ldb;
+    long long sB;
+    double beta;
+    double* C;
+    int ldc;
+    long long sC;
+    int tilesN;
+    double* part;                 // split mode: the chain sums' buffer
+    int causal, row0, snake;
+};
+
+template <int WB, int KT>
 struct F64Cfg {
-    static constexpr int TILE = 32 * WB;                       // work-group tile side
-    static constexpr int NLD = TILE * F64_KT / F64_THREADS;    // A (and B) values per thread
+    static constexpr int TILE = 32 * WB;                    // work-group tile side
+    static constexpr int NLD = TILE * KT / 2 / F64_THREADS; // A (and B) pairs per thread
     // LDS copy of an operand tile in its global order, so the stores from global memory
     // are conflict-free as well as the MFMA operand reads (16 consecutive rows or columns
     // of one k, times 4 k, per wave):
-    //   k-contiguous (A untransposed, B transposed): [row][k], row pitch KT + 1 doubles;
-    //   row-contiguous (A transposed, B untransposed): [k][row], k pitch TILE + 16 doubles
-    //   (128 bytes past a multiple of the 256-byte bank sweep).
-    static constexpr int KP = F64_KT + 1, RP = TILE + 16;
-    static constexpr int SZ_K = TILE * KP, SZ_R = F64_KT * RP;
+    //   k-contiguous (A untransposed, B transposed): [row][k], row pitch KT + 2 doubles (16
+    //   rows start 4 banks apart, the 2 k of a half-wave fill the gaps);
+    //   row-contiguous (A transposed, B untransposed): [k][row], odd k with halves of 16 rows
+    //   swapped (the 2 k of a half-wave on opposite halves of the 64 banks).
+    static constexpr int KP = KT + 2, RP = TILE;
+    __device__ static int at_k(int row, int k) { return row * KP + k; }
+    __device__ static int at_r(int row, int k) { return k * RP + (row ^ (16 * (k & 1))); }
+    static constexpr int SZ_K = TILE * KP, SZ_R = KT * RP;
 };
 
-// One TILE x TILE output tile over the k range [kbeg, kend): all of K, or (split mode,
-// part != null) the single 256-deep block blockIdx.z, whose chain sum goes to the partial
-// buffer.  Products run on v_mfma_f64_16x16x4f64, which performs its four products of an
-// output as sequential IEEE fused multiply-adds in k order (a GPU probe over 7 M outputs --
-// integers, N(0,1), exponents over 2^+-30, subnormals, infinities and NaNs, 64-step chains --
-// found it bitwise equal to the fma chain), so each accumulator is exactly the reference's
-// chain.  Operand layout: lane l holds A[l % 16][k0 + l / 16] and B[k0 + l / 16][l % 16];
-// result register r holds D[l / 16 + 4 r][l % 16].  k past the range is zero in both
-// operands, and fma(0, 0, c) = c for every chain value (a chain started at +0 never holds
-// -0), so the padded k-steps of a last partial stage change nothing.  Stages of 16 k are
-// double-buffered in LDS; the next stage's global loads are issued before the current
-// stage's products.
-template <int TA, int TB, int WB>
-__global__ __launch_bounds__(F64_THREADS) void gemm_f64_kernel(
-    int M, int N, int K, double alpha, const double* __restrict__ A, int lda, long long sA,
-    const double* __restrict__ B, int ldb, long long sB, double beta, double* __restrict__ C,
-    int ldc, long long sC, int tilesN, double* __restrict__ part) {
-    using Cf = F64Cfg<WB>;
-    constexpr int TILE = Cf::TILE, NLD = Cf::NLD, KP = Cf::KP, RP = Cf::RP;
-    __shared__ double As[2][TA == 0 ? Cf::SZ_K : Cf::SZ_R];
-    __shared__ double Bs[2][TB == 1 ? Cf::SZ_K : Cf::SZ_R];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+// One TILE x TILE output tile.  Products run on v_mfma_f64_16x16x4f64, which performs its four
+// products of an output as sequential IEEE fused multiply-adds in k order (a GPU probe over 7 M
+// outputs -- integers, N(0,1), exponents over 2^+-30, subnormals, infinities and NaNs, 64-step
+// chains -- found it bitwise equal to the fma chain), so each accumulator is exactly the
+// reference's chain.  Operand layout: lane l holds A[l % 16][k0 + l / 16] and
+// B[k0 + l / 16][l % 16]; result register r holds D[l / 16 + 4 r][l % 16].  k past the range
+// is zero in both operands, and fma(0, 0, c) = c for every chain value (a chain started at +0
+// never holds -0), so padded k-steps change nothing.
+//
+// G groups of four waves share the tile: group g runs the chains of the 256-deep blocks
+// g, g + G, ... and the chain sums meet in LDS, where group 0 adds them in k order.  A
+// small grid is bound by the chain of memory latencies of a work-group's k-stages; G groups
+// run G such chains at a time without a second launch and its partials.  Each group stages its
+// own operands: KT k per stage, double-buffered in LDS, two stages in flight in registers (a
+// load has two stages' products to land).  With `part`, blockIdx.z takes G blocks and every
+// group writes its chain sum there instead.
+template <int TA, int TB, int WB, int KT, int G, bool WIDE>
+__global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_kernel(F64Args ar) {
+    using Cf = F64Cfg<WB, KT>;
+    constexpr int TILE = Cf::TILE, NLD = Cf::NLD;
+    constexpr int SZA = TA == 0 ? Cf::SZ_K : Cf::SZ_R, SZB = TB == 1 ? Cf::SZ_K : Cf::SZ_R;
+    constexpr int SPB = F64_KC / KT;             // stages per block
+    static_assert(SPB % 2 == 0, "stages run in pairs");
+    static_assert(G == 1 || SZA + SZB >= TILE * TILE, "a stage buffer holds a group's chain sums");
+    __shared__ __attribute__((aligned(16))) double lds[G][2][SZA + SZB];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int g = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int t = tid & (F64_THREADS - 1);
     const int wr = 16 * WB * (wave & 1), wc = 16 * WB * (wave >> 1);   // wave's sub-tile
-    const int tile = blockIdx.x;
-    const int m0 = (tile / tilesN) * TILE, n0 = (tile % tilesN) * TILE;
-    const long long b = blockIdx.y;
-    int kbeg = 0, kend = K;
-    if (part) {
-        kbeg = blockIdx.z * F64_KC;
-        kend = min(K, kbeg + F64_KC);
+    const int M = ar.M, N = ar.N, K = ar.K;
+    int tile = blockIdx.x;
+    long long b = blockIdx.y;
+    if (ar.causal >= F64_TO_DIAG) {
+        // Unequal k-ranges: the tiles of every member by length, longest first, in runs of
+        // `snake` (the CU count) that alternate direction, so that the work-groups a CU is dealt
+        // (one of each run) add up to about the same length.  Causal P V of 16 slices
+        // of 1024 x 256, same box: 142 us in tile order, 100 us so.
+        const int lin = blockIdx.y * gridDim.x + blockIdx.x, all = gridDim.x * gridDim.y;
+        const int run = lin / ar.snake, base = run * ar.snake;
+        const int len = min(ar.snake, all - base);
+        const int rank = run & 1 ? base + len - 1 - (lin - base) : lin;
+        tile = rank / gridDim.y;
+        b = rank - tile * gridDim.y;
+        if (ar.causal == F64_TO_DIAG) tile = gridDim.x - 1 - tile;
     }
-    const int ns = (kend - kbeg + F64_KT - 1) / F64_KT;
+    int tm, tn;
+    if (ar.causal == F64_SCORES) {
+        // the grid holds the visible tiles only: tile row tm has tm + 1 + o of them (the last one
+        // may lie past N), tm (tm + 1) / 2 + tm o before it
+        const int o = (ar.row0 + TILE - 1) / TILE;
+        const float h = o + 0.5f;
+        tm = (int)(sqrtf(h * h + 2.f * tile) - h);
+        while (tm * (tm + 1) / 2 + tm * o > tile) --tm;
+        while ((tm + 1) * (tm + 2) / 2 + (tm + 1) * o <= tile) ++tm;
+        tn = tile - (tm * (tm + 1) / 2 + tm * o);
+        if (tn >= ar.tilesN) return;
+    } else if (ar.causal == F64_ALL) {
+        // each XCD a 4-row block of tiles: its work-groups share operand rows in its L2
+        xcd_tile_order(tile, gridDim.x, (M + TILE - 1) / TILE, ar.tilesN, 4, tm, tn);
+    } else {
+        tm = tile / ar.tilesN;
+        tn = tile % ar.tilesN;
+    }
+    // scalar registers (the tile search goes through the vector ALU)
+    const int m0 = __builtin_amdgcn_readfirstlane(tm) * TILE;
+    const int n0 = __builtin_amdgcn_readfirstlane(tn) * TILE;
+    int kbeg = 0, kend = K;
+    if (ar.causal == F64_TO_DIAG) kend = min(K, ar.row0 + m0 + TILE);
+    if (ar.causal == F64_FROM_DIAG) kbeg = max(0, m0 - ar.row0) / KT * KT;
+    // blocks from blk0 on, G of them a round; stage q of group g starts at k_of(q)
+    int blk0 = kbeg / F64_KC * F64_KC;
+    if (ar.part) {
+        blk0 = blockIdx.z * (G * F64_KC);
+        kend = min(kend, blk0 + G * F64_KC);
+    }
+    const int left = kend - blk0;
+    const int rounds = left > 0 ? (left + G * F64_KC - 1) / (G * F64_KC) : 0;
+    const int last = left - (rounds - 1) * (G * F64_KC);     // k of the last round
+    const int nq = rounds ? (rounds - 1) * SPB + (min(last, F64_KC) + KT - 1) / KT : 0;
+    const int q0 = G == 1 && kbeg > blk0 ? (kbeg - blk0) / KT & ~1 : 0;
+    auto k_of = [&](int q) { return blk0 + (q / SPB * G + g) * F64_KC + q % SPB * KT; };
 
-    // Element (row, k) of an operand tile in LDS.
-    auto a_at = [&](int buf, int row, int k) -> double& {
-        return TA == 0 ? As[buf][row * KP + k] : As[buf][k * RP + row];
-    };
-    auto b_at = [&](int buf, int row, int k) -> double& {
-        return TB == 1 ? Bs[buf][row * KP + k] : Bs[buf][k * RP + row];
-    };
-    // This thread's NLD (row, k) positions per operand, read along the contiguous index
-    // (k-contiguous: 16 lanes per 128-byte row piece; row-contiguous: TILE lanes), with a
-    // loop-invariant pointer to k = kbeg + the position's k and the row's validity.
-    int arow[NLD], ak[NLD], brow[NLD], bk[NLD];
-    const double* ap[NLD];
-    const double* bp[NLD];
-    bool aok[NLD], bok[NLD];
+    // This thread's NLD pairs of values per operand, two consecutive along the contiguous index
+    // (a load instruction costs its issue whatever its width), as loop-invariant byte offsets
+    // from a base that moves with the stage: a stage spends next to no vector ALU time, which
+    // fp64 products need, on addresses.  k outside the range (the ragged last stage, a stage past
+    // the end, masked values before kbeg that nobody wrote) reads zero through an offset or a
+    // buffer range that excludes it, or is dropped by stash(): no branch, so nothing waits for
+    // a load before its stash.  kbeg is a multiple of KT: no stage straddles it.  A row past the
+    // edge reads the last row: its values reach only results that are not stored.  The buffer
+    // range ends with the operand's last valid value.
+    int ak[NLD], bk[NLD], arow[NLD], brow[NLD];
+    size_t ao[NLD], bo[NLD];
+    const int ma = min(TILE, M - m0), nb = min(TILE, N - n0);   // valid rows of the tile
 #pragma unroll
     for (int r = 0; r < NLD; ++r) {
-        if (TA == 0) { ak[r] = t & 15; arow[r] = (t >> 4) + 16 * r; }
-        else         { arow[r] = t % TILE; ak[r] = t / TILE + (F64_THREADS / TILE) * r; }
-        if (TB == 1) { bk[r] = t & 15; brow[r] = (t >> 4) + 16 * r; }
-        else         { brow[r] = t % TILE; bk[r] = t / TILE + (F64_THREADS / TILE) * r; }
-        const int gm = m0 + arow[r], gn = n0 + brow[r];
-        aok[r] = gm < M;
-        bok[r] = gn < N;
-        const long long ka = kbeg + ak[r], kb = kbeg + bk[r];
-        ap[r] = A + b * sA + (aok[r] ? (TA == 0 ? (long long)gm * lda + ka : ka * lda + gm) : 0);
-        bp[r] = B + b * sB + (bok[r] ? (TB == 1 ? (long long)gn * ldb + kb : kb * ldb + gn) : 0);
+        const int f = t + F64_THREADS * r;
+        ak[r] = TA == 0 ? 2 * (f % (KT / 2)) : f / (TILE / 2);
+        arow[r] = TA == 0 ? f / (KT / 2) : 2 * (f % (TILE / 2));
+        bk[r] = TB == 1 ? 2 * (f % (KT / 2)) : f / (TILE / 2);
+        brow[r] = TB == 1 ? f / (KT / 2) : 2 * (f % (TILE / 2));
+        const size_t am = min(arow[r], ma - 1), bn = min(brow[r], nb - 1);
+        ao[r] = 8 * (TA == 0 ? am * ar.lda + ak[r] : ak[r] * (size_t)ar.lda + am);
+        bo[r] = 8 * (TB == 1 ? bn * ar.ldb + bk[r] : bk[r] * (size_t)ar.ldb + bn);
     }
-    const long long astep = TA == 0 ? F64_KT : (long long)F64_KT * lda;   // pointer step per stage
-    const long long bstep = TB == 1 ? F64_KT : (long long)F64_KT * ldb;
-    double ra[NLD], rb[NLD];
-    auto fetch = [&](int s) {           // stage s: k = kbeg + 16 s + position
-        const int kleft = kend - kbeg - F64_KT * s;   // valid k in this stage (may exceed 16)
+    const GlobalBytes abase = (GlobalBytes)(ar.A + b * ar.sA + (TA == 0 ? (long long)m0 * ar.lda : m0));
+    const GlobalBytes bbase = (GlobalBytes)(ar.B + b * ar.sB + (TB == 1 ? (long long)n0 * ar.ldb : n0));
+    auto valid_of = [&](int q) {   // k of stage q inside the range
+        const int k0 = k_of(q);
+        return q < nq && k0 >= kbeg && k0 < kend ? min(kend - k0, KT) : 0;
+    };
+    f64x2 ra[2][NLD], rb[2][NLD];
+    auto fetch = [&](auto set_c, int q) {
+        constexpr int set = decltype(set_c)::value;
+        const int k0 = k_of(q), valid = valid_of(q);
+        const GlobalBytes pa = abase + 8LL * (TA == 0 ? k0 : (long long)k0 * ar.lda);
+        const GlobalBytes pb = bbase + 8LL * (TB == 1 ? k0 : (long long)k0 * ar.ldb);
+        if constexpr (WIDE) {   // 64-bit offsets, value by value
+            const GlobalBytes zero = (GlobalBytes)&g_zero64;
 #pragma unroll
-        for (int r = 0; r < NLD; ++r) {
-            ra[r] = aok[r] && ak[r] < kleft ? ap[r][s * astep] : 0.0;
-            rb[r] = bok[r] && bk[r] < kleft ? bp[r][s * bstep] : 0.0;
+            for (int r = 0; r < NLD; ++r)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const bool ain = TA == 0 ? ak[r] + e < valid : ak[r] < valid && arow[r] + e < ma;
+                    const bool bin = TB == 1 ? bk[r] + e < valid : bk[r] < valid && brow[r] + e < nb;
+                    ra[set][r][e] = *(GlobalF64)(ain ? pa + ao[r] + 8 * e : zero);
+                    rb[set][r][e] = *(GlobalF64)(bin ? pb + bo[r] + 8 * e : zero);
+                }
+        } else {
+            const int lasta = TA == 0 ? (ma - 1) * ar.lda + valid : (valid - 1) * ar.lda + ma;
+            const int lastb = TB == 1 ? (nb - 1) * ar.ldb + valid : (valid - 1) * ar.ldb + nb;
+            const __amdgpu_buffer_rsrc_t sa = f64_rsrc(pa, __builtin_amdgcn_readfirstlane(valid ? 8 * lasta : 0));
+            const __amdgpu_buffer_rsrc_t sb = f64_rsrc(pb, __builtin_amdgcn_readfirstlane(valid ? 8 * lastb : 0));
+#pragma unroll
+            for (int r = 0; r < NLD; ++r) {
+                ra[set][r] = f64_load2(sa, TA == 1 || ak[r] < valid ? (int)ao[r] : F64_OOB);
+                rb[set][r] = f64_load2(sb, TB == 0 || bk[r] < valid ? (int)bo[r] : F64_OOB);
+            }
         }
     };
-    auto stash = [&](int buf) {
+    auto stash = [&](auto set_c, int q) {
+        constexpr int set = decltype(set_c)::value;
+        double* d = lds[g][set];
+        const int valid = valid_of(q);
 #pragma unroll
         for (int r = 0; r < NLD; ++r) {
-            a_at(buf, arow[r], ak[r]) = ra[r];
-            b_at(buf, brow[r], bk[r]) = rb[r];
+            f64x2 va = ra[set][r], vb = rb[set][r];
+            // k along a row: the pair that holds the range's end read the next value with it
+            if (TA == 0) va[1] = ak[r] + 1 < valid ? va[1] : 0.0;
+            if (TB == 1) vb[1] = bk[r] + 1 < valid ? vb[1] : 0.0;
+            *reinterpret_cast<f64x2*>(d + (TA == 0 ? Cf::at_k(arow[r], ak[r]) : Cf::at_r(arow[r], ak[r]))) = va;
+            *reinterpret_cast<f64x2*>(d + SZA + (TB == 1 ? Cf::at_k(brow[r], bk[r]) : Cf::at_r(brow[r], bk[r]))) = vb;
         }
     };
 
@@ -138,63 +272,119 @@ __global__ __launch_bounds__(F64_THREADS) void gemm_f64_kernel(
         for (int j = 0; j < WB; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) tot[i][j][r] = acc[i][j][r] = 0.0;
-    auto step = [&](int buf, int k4) {
-        const int kr = 4 * k4 + (lane >> 4), c = lane & 15;
-        double a[WB], bb[WB];
+    const int kr0 = lane >> 4, c0 = lane & 15;
+    auto step = [&](auto set_c, int q) {   // stage q from LDS buffer q % 2 = set
+        constexpr int set = decltype(set_c)::value;
+        fetch(set_c, q + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        const double* as = lds[g][set];
+        const double* bs = as + SZA;
+        double a[KT / 4][WB], bb[KT / 4][WB];
 #pragma unroll
-        for (int i = 0; i < WB; ++i) a[i] = a_at(buf, wr + 16 * i + c, kr);
+        for (int k4 = 0; k4 < KT / 4; ++k4) {
+            const int kr = 4 * k4 + kr0;
 #pragma unroll
-        for (int j = 0; j < WB; ++j) bb[j] = b_at(buf, wc + 16 * j + c, kr);
+            for (int i = 0; i < WB; ++i) {
+                const int row = wr + 16 * i + c0, col = wc + 16 * i + c0;
+                a[k4][i] = as[TA == 0 ? Cf::at_k(row, kr) : Cf::at_r(row, kr)];
+                bb[k4][i] = bs[TB == 1 ? Cf::at_k(col, kr) : Cf::at_r(col, kr)];
+            }
+        }
+        // One block per wave: a dependent chain of products; with the reads between them each
+        // pair waited for its own LDS latency (200 cycles a product instead of 64), so a
+        // stage's reads all go first.
+        if (WB == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < WB; ++i)
+        for (int k4 = 0; k4 < KT / 4; ++k4)
 #pragma unroll
-            for (int j = 0; j < WB; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bb[j], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < WB; ++i)
+#pragma unroll
+                for (int j = 0; j < WB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k4][i], bb[k4][j], acc[i][j], 0, 0, 0);
+        // stage q + 1, fetched a step ago; kept behind the products (the scheduler would move its
+        // wait to the front, and the loads would have one stage to land instead of two)
+        __builtin_amdgcn_sched_barrier(0);
+        stash(std::integral_constant<int, set ^ 1>{}, q + 1);
+        __syncthreads();
     };
-
-    // Every stage runs its four k-steps (zeros past kend), so the loop has no branch around
-    // the accumulators; a fetch past the last stage loads nothing and its stash lands in the
-    // buffer no later stage reads.  Blocks of 256 k (kbeg is a multiple of 256): the chain
-    // sum of each is added to tot in k order.
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int s = 0; s < ns;) {
-        const int s_end = min(ns, s + F64_KC / F64_KT);
-        for (; s < s_end; ++s) {
-            const int buf = s & 1;
-            fetch(s + 1);
+    // Stages run in pairs (a pair's second stage past the end multiplies zeros), so the loop
+    // has no branch around the accumulators; the blocks of 256 k are an outer loop, which adds
+    // their chain sums in k order.
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    if (q0 < nq) {
+        fetch(even, q0);
+        fetch(odd, q0 + 1);
+        stash(even, q0);
+        __syncthreads();
+    }
+    for (int q = q0; q < nq;) {
+        const int qe = min(nq, (q / SPB + 1) * SPB);
+        for (; q < qe; q += 2) {
+            step(even, q);
+            step(odd, q + 1);
+        }
+        if (G > 1 && !ar.part) {
+            // lds[.][1] was read in the last step and is not written before the next round
+            auto at = [&](int grp, int i, int j, int r) -> double& {
+                return lds[grp][1][(((wave * WB + i) * WB + j) * 4 + r) * 64 + lane];
+            };
+            if (g > 0) {
 #pragma unroll
-            for (int k4 = 0; k4 < F64_KT / 4; ++k4) step(buf, k4);
-            stash(buf ^ 1);   // the buffer stage s - 1 read, released below
+                for (int i = 0; i < WB; ++i)
+#pragma unroll
+                    for (int j = 0; j < WB; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) at(g, i, j, r) = acc[i][j][r];
+            }
             __syncthreads();
+            if (g == 0) {
+#pragma unroll
+                for (int i = 0; i < WB; ++i)
+#pragma unroll
+                    for (int j = 0; j < WB; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            double s = tot[i][j][r] + acc[i][j][r];
+                            for (int x = 1; x < G; ++x) s = s + at(x, i, j, r);
+                            tot[i][j][r] = s;
+                        }
+            }
+            __syncthreads();
+        } else {
+#pragma unroll
+            for (int i = 0; i < WB; ++i)
+#pragma unroll
+                for (int j = 0; j < WB; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) tot[i][j][r] = tot[i][j][r] + acc[i][j][r];
         }
 #pragma unroll
         for (int i = 0; i < WB; ++i)
 #pragma unroll
             for (int j = 0; j < WB; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    tot[i][j][r] = tot[i][j][r] + acc[i][j][r];
-                    acc[i][j][r] = 0.0;
-                }
+                for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0;
     }
+    const int block = blockIdx.z * G + g;   // split mode: this group's block
+    if (ar.part ? block * F64_KC >= K : g > 0) return;
     // lane l, register r of block (i, j): row wr + 16 i + l / 16 + 4 r, column wc + 16 j + l % 16
-    double* out = part ? part + ((long long)blockIdx.z * gridDim.y + b) * ((long long)M * N)
-                       : C + b * sC;
-    const long long ld = part ? N : ldc;
+    double* out = ar.part ? ar.part + ((long long)block * gridDim.y + b) * ((long long)M * N)
+                          : ar.C + b * ar.sC;
+    const long long ld = ar.part ? N : ar.ldc;
+    const double alpha = ar.alpha, beta = ar.beta;
 #pragma unroll
     for (int i = 0; i < WB; ++i)
 #pragma unroll
         for (int j = 0; j < WB; ++j) {
-            const int gn = n0 + wc + 16 * j + (lane & 15);
+            const int gn = n0 + wc + 16 * j + c0;
             if (gn >= N) continue;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int gm = m0 + wr + 16 * i + (lane >> 4) + 4 * r;
+                const int gm = m0 + wr + 16 * i + kr0 + 4 * r;
                 if (gm >= M) continue;
                 double* c = out + (long long)gm * ld + gn;
-                if (part) {             // this block's chain sum, compact M x N per (block, member)
+                if (ar.part) {          // this block's chain sum, compact M x N per (block, member)
                     *c = tot[i][j][r];
                 } else {
                     const double v = alpha == 1.0 ? tot[i][j][r] : alpha * tot[i][j][r];
@@ -225,10 +415,13 @@ __global__ __launch_bounds__(256) void gemm_f64_reduce(int M, int N, int nkb, in
 
 // Row softmax of one chunk of attention scores, in place: row r is query i = r mod S of its
 // slice; x_j = s_j * scale over the row's visible keys (j <= i when causal), then
-// p_j = exp(x_j - max x) / sum exp(x - max x), and exact zeros for masked keys
-// (training.inc:193-201, 240-247).  One wave per row.
-// P holds `rows` score rows of S keys: consecutive groups of R rows are query rows
+// p_j = exp(x_j - max x) / sum exp(x - max x), and exact zeros for masked keys (up to F64_PAD
+// past the diagonal: no product reads further) (training.inc:193-201, 240-247).  One wave per
+// row.  P holds `rows` score rows of S keys: consecutive groups of R rows are query rows
 // row0 .. row0 + R - 1 of a slice (R = S, row0 = 0 for whole slices).
+// Bound by memory: with NV > 0 (S <= 64 NV) the row stays in registers, so it is read and
+// written once.
+template <int NV>
 __global__ __launch_bounds__(256) void attn_softmax_f64(double* __restrict__ P, int S,
                                                         long long rows, int R, int row0,
                                                         double scale, int causal) {
@@ -238,25 +431,53 @@ __global__ __launch_bounds__(256) void attn_softmax_f64(double* __restrict__ P, 
     if (r >= rows) return;
     const int lane = threadIdx.x & 63;
     const int i = row0 + (int)(r % R);
-    const int n = causal ? i + 1 : S;
+    const int n = causal ? i + 1 : S, fill = causal ? min(S, i + F64_PAD) : S;
     double* row = P + r * (long long)S;
-    double mx = -1e30;
-    for (int j = lane; j < n; j += 64) mx = fmax(mx, row[j] * scale);
+    double mx = -1e30, sum = 0.0;
+    if constexpr (NV > 0) {
+        double x[NV];
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) mx = fmax(mx, __shfl_xor(mx, d));
-    double sum = 0.0;
-    for (int j = lane; j < n; j += 64) {
-        const double e = exp(row[j] * scale - mx);
-        row[j] = e;
-        sum += e;
+        for (int t = 0; t < NV; ++t) {
+            x[t] = row[min(lane + 64 * t, n - 1)] * scale;   // no branch: the loads overlap
+        }
+#pragma unroll
+        for (int t = 0; t < NV; ++t)
+            if (lane + 64 * t < n) mx = fmax(mx, x[t]);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) mx = fmax(mx, __shfl_xor(mx, d));
+#pragma unroll
+        for (int t = 0; t < NV; ++t) {
+            if (64 * t >= n) continue;   // wave-uniform
+            if (lane + 64 * t < n) {
+                x[t] = exp(x[t] - mx);
+                sum += x[t];
+            }
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+#pragma unroll
+        for (int t = 0; t < NV; ++t) {
+            const int j = lane + 64 * t;
+            if (j < fill) row[j] = j < n ? x[t] / sum : 0.0;
+        }
+    } else {
+        for (int j = lane; j < n; j += 64) mx = fmax(mx, row[j] * scale);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) mx = fmax(mx, __shfl_xor(mx, d));
+        for (int j = lane; j < n; j += 64) {
+            const double e = exp(row[j] * scale - mx);
+            row[j] = e;
+            sum += e;
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+        for (int j = lane; j < fill; j += 64) row[j] = j < n ? row[j] / sum : 0.0;
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
-    for (int j = lane; j < S; j += 64) row[j] = j < n ? row[j] / sum : 0.0;
 }
 
-// dS = P o (dP - rowsum(dP o P)) in place of dP, zeros on masked keys (the softmax JVP of
-// autograd.inc:711-714, 758-761).
+// dS = P o (dP - rowsum(dP o P)) in place of dP, zeros on masked keys up to F64_PAD past the
+// diagonal (the softmax JVP of autograd.inc:711-714, 758-761).
+template <int NV>
 __global__ __launch_bounds__(256) void attn_softmax_bwd_f64(const double* __restrict__ P,
                                                             double* __restrict__ dP, int S,
                                                             long long rows, int R, int row0,
@@ -265,23 +486,40 @@ __global__ __launch_bounds__(256) void attn_softmax_bwd_f64(const double* __rest
     if (r >= rows) return;
     const int lane = threadIdx.x & 63;
     const int i = row0 + (int)(r % R);
-    const int n = causal ? i + 1 : S;
+    const int n = causal ? i + 1 : S, fill = causal ? min(S, i + F64_PAD) : S;
     const double* p = P + r * (long long)S;
     double* g = dP + r * (long long)S;
     double rd = 0.0;
-    for (int j = lane; j < n; j += 64) rd = __builtin_fma(g[j], p[j], rd);
+    if constexpr (NV > 0) {
+        double pv[NV], gv[NV];
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) rd += __shfl_xor(rd, d);
-    for (int j = lane; j < S; j += 64) g[j] = j < n ? p[j] * (g[j] - rd) : 0.0;
+        for (int t = 0; t < NV; ++t) {
+            const int j = min(lane + 64 * t, n - 1);   // no branch: the loads overlap
+            pv[t] = p[j];
+            gv[t] = g[j];
+        }
+#pragma unroll
+        for (int t = 0; t < NV; ++t)
+            if (lane + 64 * t < n) rd = __builtin_fma(gv[t], pv[t], rd);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) rd += __shfl_xor(rd, d);
+#pragma unroll
+        for (int t = 0; t < NV; ++t) {
+            const int j = lane + 64 * t;
+            if (j < fill) g[j] = j < n ? pv[t] * (gv[t] - rd) : 0.0;
+        }
+    } else {
+        for (int j = lane; j < n; j += 64) rd = __builtin_fma(g[j], p[j], rd);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) rd += __shfl_xor(rd, d);
+        for (int j = lane; j < fill; j += 64) g[j] = j < n ? p[j] * (g[j] - rd) : 0.0;
+    }
 }
 
-template <int WB>
-void launch_f64(int transA, int transB, dim3 grid, int M, int N, int K, double alpha,
-                const double* A, int lda, long long sA, const double* B, int ldb, long long sB,
-                double beta, double* C, int ldc, long long sC, int tilesN, double* part) {
-#define DH_F64_LAUNCH(TA, TB)                                                                  \
-    gemm_f64_kernel<TA, TB, WB><<<grid, F64_THREADS, 0, stream()>>>(                           \
-        M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, tilesN, part)
+template <int WB, int KT, int G, bool WIDE = false>
+void launch_f64(int transA, int transB, dim3 grid, const F64Args& ar) {
+#define DH_F64_LAUNCH(TA, TB) \
+    gemm_f64_kernel<TA, TB, WB, KT, G, WIDE><<<grid, F64_THREADS * G, 0, stream()>>>(ar)
     if (!transA && !transB) DH_F64_LAUNCH(0, 0);
     else if (!transA) DH_F64_LAUNCH(0, 1);
     else if (!transB) DH_F64_LAUNCH(1, 0);
@@ -291,26 +529,42 @@ void launch_f64(int transA, int transB, dim3 grid, int M, int N, int K, double a
 
 int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, const double* A,
                     int lda, long long sA, const double* B, int ldb, long long sB, double beta,
-                    double* C, int ldc, long long sC, int batch) {
+                    double* C, int ldc, long long sC, int batch, int causal = F64_ALL,
+                    int row0 = 0) {
     // 64 x 64 tiles (2 x 2 blocks per wave) when they fill the chip twice over, else 32 x 32.
-    // Grids still too small split K at the reference's 256-deep block boundaries (one
-    // work-group per block, each block's chain sum stored, then summed in k order by
-    // gemm_f64_reduce), which leaves every result bit-identical.
-    const long long fill = 2LL * num_cus();
-    const int wb = ((M + 63) / 64) * (long long)((N + 63) / 64) * batch >= fill ? 2 : 1;
+    // A small grid is bound by the latencies of its work-groups' k-stages, so it runs the
+    // 256-deep blocks of k side by side: up to four groups of waves in a work-group, as many as
+    // bring a CU about 16 waves (same box, us, one group / chosen: 511^3 13.6 / 12.5, 512^2 x
+    // 1024 22.6 / 17.9, 256 x 1023 x 4096 81.9 / 58.4), or, where the tiles leave half the CUs
+    // idle, one work-group per block, whose chain sums gemm_f64_reduce adds in k order (64^2 x
+    // 4096 77.7 / 15.3, 300^2 x 1000 21.8 / 15.6; with groups 56.7 and 17.5).  Every form leaves
+    // the results bit-identical.  Leading dimensions past 2^22 need 64-bit offsets within a
+    // tile: one form has them.
+    const long long cus = num_cus();
+    const bool wide = lda > (1 << 22) || ldb > (1 << 22);
+    const int wb = !wide && ((M + 63) / 64) * (long long)((N + 63) / 64) * batch >= 2 * cus ? 2 : 1;
     const long long tilesM = (M + 32 * wb - 1) / (32 * wb), tilesN = (N + 32 * wb - 1) / (32 * wb);
+    const long long tiles = tilesM * tilesN * batch;
     const long long nkb = ((long long)K + F64_KC - 1) / F64_KC;
     const size_t pbytes = (size_t)nkb * batch * M * N * sizeof(double);
     double* part = nullptr;
-    if (nkb > 1 && nkb <= 65535 && tilesM * tilesN * batch < fill && pbytes <= ((size_t)512 << 20))
+    if (nkb > 1 && nkb <= 65535 && 2 * tiles <= cus && pbytes <= ((size_t)512 << 20))
         part = static_cast<double*>(dh_malloc(pbytes));   // none: the unsplit grid
-    const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)batch, part ? (unsigned)nkb : 1u);
-    if (wb == 2)
-        launch_f64<2>(transA, transB, grid, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc,
-                      sC, (int)tilesN, part);
-    else
-        launch_f64<1>(transA, transB, grid, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc,
-                      sC, (int)tilesN, part);
+    int G = 1;
+    if (wb == 1 && !wide && !part)
+        while (G < 4 && G < nkb && tiles * G < 4 * cus) G *= 2;
+    const long long o = (row0 + 32 * wb - 1) / (32 * wb);   // F64_SCORES: visible tiles only
+    const dim3 grid((unsigned)(causal == F64_SCORES ? tilesM * (tilesM + 1) / 2 + tilesM * o
+                                                    : tilesM * tilesN),
+                    (unsigned)batch,
+                    part ? (unsigned)nkb : 1u);
+    const F64Args ar{M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, (int)tilesN, part,
+                     causal, row0, (int)cus};
+    if (wide) launch_f64<1, 32, 1, true>(transA, transB, grid, ar);
+    else if (wb == 2) launch_f64<2, 16, 1>(transA, transB, grid, ar);
+    else if (G == 1) launch_f64<1, 32, 1>(transA, transB, grid, ar);
+    else if (G == 2) launch_f64<1, 32, 2>(transA, transB, grid, ar);
+    else launch_f64<1, 32, 4>(transA, transB, grid, ar);
     if (part) {
         const long long total = (long long)M * N * batch;
         long long blocks = (total + 255) / 256;
@@ -384,14 +638,18 @@ int check_attn_f64(const char* op, int BH, int S, int D) {
 
 void launch_softmax(double* P, int S, long long rows, int R, int row0, double scale,
                     int causal) {
-    attn_softmax_f64<<<(unsigned)((rows + 3) / 4), 256, 0, stream()>>>(P, S, rows, R, row0,
-                                                                      scale, causal);
+    const unsigned grid = (unsigned)((rows + 3) / 4);
+    if (S <= 256) attn_softmax_f64<4><<<grid, 256, 0, stream()>>>(P, S, rows, R, row0, scale, causal);
+    else if (S <= 1024) attn_softmax_f64<16><<<grid, 256, 0, stream()>>>(P, S, rows, R, row0, scale, causal);
+    else attn_softmax_f64<0><<<grid, 256, 0, stream()>>>(P, S, rows, R, row0, scale, causal);
 }
 
 void launch_softmax_bwd(const double* P, double* G, int S, long long rows, int R, int row0,
                         int causal) {
-    attn_softmax_bwd_f64<<<(unsigned)((rows + 3) / 4), 256, 0, stream()>>>(P, G, S, rows, R,
-                                                                          row0, causal);
+    const unsigned grid = (unsigned)((rows + 3) / 4);
+    if (S <= 256) attn_softmax_bwd_f64<4><<<grid, 256, 0, stream()>>>(P, G, S, rows, R, row0, causal);
+    else if (S <= 1024) attn_softmax_bwd_f64<16><<<grid, 256, 0, stream()>>>(P, G, S, rows, R, row0, causal);
+    else attn_softmax_bwd_f64<0><<<grid, 256, 0, stream()>>>(P, G, S, rows, R, row0, causal);
 }
 
 }  // namespace
@@ -442,14 +700,14 @@ int dh_attention_f64_fwd(int BH, int S, int D, double scale, int causal, const d
             const long long off = (long long)b0 * SD, qoff = off + (long long)r0 * D;
             // scores of query rows r0 .. r0 + nr - 1 = Q K^T
             st = gemm_f64_launch(0, 1, nr, S, D, 1.0, d_Q + qoff, D, SD, d_K + off, D, SD, 0.0,
-                                 P, S, RS, nb);
+                                 P, S, RS, nb, causal ? F64_SCORES : F64_ALL, r0);
             if (st != DH_OK) break;
             launch_softmax(P, S, (long long)nb * nr, nr, r0, scale, causal);
             st = check_launch("dh_attention_f64_fwd");
             if (st != DH_OK) break;
             // O = P V
             st = gemm_f64_launch(0, 0, nr, D, S, 1.0, P, S, RS, d_V + off, D, SD, 0.0,
-                                 d_O + qoff, D, SD, nb);
+                                 d_O + qoff, D, SD, nb, causal ? F64_TO_DIAG : F64_ALL, r0);
         }
     }
     dh_free(P);   // pooled: stream order keeps the buffer alive for the queued work
@@ -469,8 +727,11 @@ int dh_attention_f64_bwd(int BH, int S, int D, double scale, int causal, const d
     const long long SD = (long long)S * D;
     const size_t gbytes = (size_t)BH * SD * sizeof(double);
     // Shared gradient buffers (one tensor passed as several of Q, K, V) receive the sum of
-    // their gradients: every product below adds into its output, after one clearing pass.
-    if (!accumulate) {
+    // their gradients: every product then adds into its output, after one clearing pass.
+    // Buffers of their own are written by the first product that reaches them.
+    const bool shared = d_dQ == d_dK || d_dQ == d_dV || d_dK == d_dV;
+    const bool add = accumulate || shared;
+    if (!accumulate && shared) {
         double* outs[3] = {d_dQ, d_dK, d_dV};
         for (int x = 0; x < 3; ++x) {
             bool seen = false;
@@ -497,26 +758,29 @@ int dh_attention_f64_bwd(int BH, int S, int D, double scale, int causal, const d
         for (int r0 = 0; r0 < S && st == DH_OK; r0 += ps.rows) {
             const int nr = S - r0 < ps.rows ? S - r0 : ps.rows;
             const long long ro = (long long)r0 * D;
+            const double beta = add || r0 > 0 ? 1.0 : 0.0;   // dV, dK: summed over the passes
             // P recomputed from Q, K exactly as the forward computes it
-            st = gemm_f64_launch(0, 1, nr, S, D, 1.0, Q + ro, D, SD, K, D, SD, 0.0, P, S, RS, nb);
+            st = gemm_f64_launch(0, 1, nr, S, D, 1.0, Q + ro, D, SD, K, D, SD, 0.0, P, S, RS, nb,
+                                 causal ? F64_SCORES : F64_ALL, r0);
             if (st != DH_OK) break;
             launch_softmax(P, S, (long long)nb * nr, nr, r0, scale, causal);
             if ((st = check_launch("dh_attention_f64_bwd")) != DH_OK) break;
             // dV += P^T dO
-            st = gemm_f64_launch(1, 0, S, D, nr, 1.0, P, S, RS, dO + ro, D, SD, 1.0, d_dV + off,
-                                 D, SD, nb);
+            st = gemm_f64_launch(1, 0, S, D, nr, 1.0, P, S, RS, dO + ro, D, SD, beta, d_dV + off,
+                                 D, SD, nb, causal ? F64_FROM_DIAG : F64_ALL, r0);
             if (st != DH_OK) break;
             // dP = dO V^T, then dS in its place
-            st = gemm_f64_launch(0, 1, nr, S, D, 1.0, dO + ro, D, SD, V, D, SD, 0.0, G, S, RS, nb);
+            st = gemm_f64_launch(0, 1, nr, S, D, 1.0, dO + ro, D, SD, V, D, SD, 0.0, G, S, RS, nb,
+                                 causal ? F64_SCORES : F64_ALL, r0);
             if (st != DH_OK) break;
             launch_softmax_bwd(P, G, S, (long long)nb * nr, nr, r0, causal);
             if ((st = check_launch("dh_attention_f64_bwd")) != DH_OK) break;
             // dQ += scale dS K ;  dK += scale dS^T Q
-            st = gemm_f64_launch(0, 0, nr, D, S, scale, G, S, RS, K, D, SD, 1.0,
-                                 d_dQ + off + ro, D, SD, nb);
+            st = gemm_f64_launch(0, 0, nr, D, S, scale, G, S, RS, K, D, SD, add ? 1.0 : 0.0,
+                                 d_dQ + off + ro, D, SD, nb, causal ? F64_TO_DIAG : F64_ALL, r0);
             if (st != DH_OK) break;
-            st = gemm_f64_launch(1, 0, S, D, nr, scale, G, S, RS, Q + ro, D, SD, 1.0,
-                                 d_dK + off, D, SD, nb);
+            st = gemm_f64_launch(1, 0, S, D, nr, scale, G, S, RS, Q + ro, D, SD, beta,
+                                 d_dK + off, D, SD, nb, causal ? F64_FROM_DIAG : F64_ALL, r0);
         }
     }
     dh_free(P);

@@ -243,3 +243,60 @@ def test_attention_f64_query_row_blocks(causal, monkeypatch):
         assert maxrel(g, r + i) <= 1e-11
     shared = sum(O.attention_bwd(Q, Q, Q, G, B, S, D, causal))
     assert maxrel(attn64_bwd(Q, Q, Q, G, B, S, D, causal, alias=True)[0], shared) <= 1e-11
+
+
+@pytest.mark.parametrize("M,N,K", [(511, 511, 511), (500, 330, 1030), (256, 257, 2051),
+                                   (65, 31, 1300), (1, 1, 513), (33, 64, 33), (32, 96, 32),
+                                   (1450, 1500, 47), (1500, 1450, 271)])
+def test_gemm_f64_forms_are_bit_identical(M, N, K):
+    # One, two and four groups of waves per tile, blocks of k over work-groups, 64-wide tiles;
+    # ragged stages, odd leading dimensions (pairs across a row's end), rows past the edge.
+    # Every layout runs the reference's chains, so all four equal the oracle bit for bit.
+    rng = np.random.default_rng(M * N + K)
+    A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    ref = O.gemm_d(A, B)
+    for ta in (0, 1):
+        for tb in (0, 1):
+            a, b = (A.T if ta else A), (B.T if tb else B)
+            pa, pb = 1 + 2 * ta, 3 - 2 * tb   # padding columns hold NaN: they must not be used
+            pad = lambda x, n: np.concatenate([x, np.full((x.shape[0], n), np.nan)], axis=1)
+            dA, dB = DB.from_numpy(pad(a, pa)), DB.from_numpy(pad(b, pb))
+            dC = DB.empty((M, N), np.float64)
+            hip.gemm_f64(ta, tb, M, N, K, dA, a.shape[1] + pa, dB, b.shape[1] + pb, 0.0, dC, N)
+            assert np.array_equal(dC.numpy(), ref), (ta, tb)
+
+
+def test_gemm_f64_huge_leading_dimension():
+    # a leading dimension past 2^22: the form with 64-bit offsets
+    ld, M, N, K = (1 << 22) + 3, 5, 7, 300
+    rng = np.random.default_rng(22)
+    A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    wide = np.zeros((M - 1) * ld + K)
+    for i in range(M):
+        wide[i * ld:i * ld + K] = A[i]
+    dA, dB, dC = DB.from_numpy(wide), DB.from_numpy(B), DB.empty((M, N), np.float64)
+    hip.gemm_f64(0, 0, M, N, K, dA, ld, dB, N, 0.0, dC, N)
+    assert np.array_equal(dC.numpy(), O.gemm_d(A, B))
+
+
+@pytest.mark.parametrize("B,S,D,rows", [(2, 63, 40, 0), (1, 64, 8, 0), (3, 65, 130, 0),
+                                        (2, 257, 33, 0), (40, 300, 64, 0), (1, 1030, 16, 0),
+                                        (2, 330, 24, 77), (1, 200, 136, 1)])
+def test_attention_f64_causal_leaves_masked_scores_alone(B, S, D, rows, monkeypatch):
+    """Causal attention neither computes nor reads scores past the diagonal's tile.  The score
+    buffers come out of the pool filled with NaN, so a read of one that was not written shows;
+    rows = query rows per pass (0: whole slices).  Bounds as the tests above."""
+    n = B * S * S
+    if rows:
+        monkeypatch.setenv("DH_ATTN_F64_SCORE_BYTES", str(rows * S * 8))
+        n = rows * S
+    held = [DB(8 * n) for _ in range(2)]
+    for h in held:
+        hip.check(hip.load().dh_memset(h.ptr, 0xFF, h.nbytes))
+        h.free()
+    rng = np.random.default_rng(S + D + rows)
+    Q, K, V, G = (rng.standard_normal((B, S * D)) for _ in range(4))
+    assert maxrel(attn64(Q, K, V, B, S, D, True), O.attention(Q, K, V, B, S, D, True)) <= 1e-12
+    ref = O.attention_bwd(Q, K, V, G, B, S, D, True)
+    for g, r in zip(attn64_bwd(Q, K, V, G, B, S, D, True), ref):
+        assert maxrel(g, r) <= 1e-11

@@ -154,7 +154,7 @@ def test_row_ops_wide_rows(C, off):
         for x in ins:
             b = DB.from_numpy(np.concatenate([np.zeros(off, np.float32), x.ravel()]))
             bufs.append(b)
-        out = DB.empty(R * C + off, np.float32)
+        out = DB.empty((R * C + off,), np.float32)
         fn(*[at(b) for b in bufs], at(out))
         return out.numpy()[off:].reshape(R, C)
 
