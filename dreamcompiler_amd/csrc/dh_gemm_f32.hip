@@ -30,6 +30,15 @@ namespace {
 
 constexpr int BK = 16, NTHREADS = 256;
 
+// How an operand is read, 4 consecutive elements at a time:
+//   LD_VEC     16-byte aligned rows and a contiguous extent divisible by 4;
+//   LD_BUF     any alignment and extent, leading dimensions up to LD_BUF_MAX (32-bit offsets):
+//              16-byte buffer loads at 4-byte alignment, see Slice;
+//   LD_BUF4    the same for K divisible by 4, so no load straddles the end of K;
+//   LD_SCALAR  anything, element by element.
+enum { LD_SCALAR = 0, LD_VEC = 1, LD_BUF = 2, LD_BUF4 = 3 };
+constexpr int LD_BUF_MAX = 1 << 20;
+
 // Four consecutive elements of one row of a row-major matrix:
 // row r, columns c..c+3 of a rows x cols matrix with leading dimension ld.
 // VEC: 16-byte aligned rows and cols % 4 == 0, so a chunk (c % 4 == 0) is wholly inside or
@@ -62,15 +71,48 @@ __device__ inline f32x4 load4(const float* __restrict__ p, int ld, int rows, int
 // halves) overlaps on 28 banks.  An XOR swizzle like store_swz's for these tiles measured +1%
 // at 4096^3 but -3% for 64 x 512^3 batched products: it breaks the paired ds_read2 /
 // ds_write2 forms the padded layout gets.
-template <bool KCONTIG, bool VEC, int TILE, int BKT = BK, int NT = NTHREADS>
+//
+// LD_BUF reads a chunk with one 128-bit buffer load wherever it starts (element-wise loads cost
+// four issues and, guarded, were each waited for at once): rows past the tile's edge repeat its
+// last one, and what a chunk reads past the end of its row reaches only results that are not
+// stored or, along k, is zeroed on the way to LDS (LD_BUF4: takes an offset past the buffer).
+// The buffer range ends with the operand's last value in the tile.  The offsets are loop
+// invariant, so aligned operands gain too (LD_VEC builds a 64-bit address per load).  Same box,
+// before / with it, ms: 4095^3 1.542 / 1.012, 4096^3 NN 1.053 / 1.010, TN 1.056 / 0.961; us: 4096 x
+// 784 x 257 35.5 / 27.3, 300 x 3000 x 3001 91 / 66.
+template <bool KCONTIG, int LD, int TILE, int BKT = BK, int NT = NTHREADS>
 struct Slice {
+    static constexpr bool VEC = LD == LD_VEC;
     static constexpr int CH = TILE * BKT / 4 / NT;   // float4 per thread per slice
     f32x4 v[CH];
+    int left;   // LD_BUF along k: valid k of the slice in v
 
     // base/ld describe the stored matrix; t0 = first index along the tile dimension,
     // k0 = first k; extent_t / extent_k bound the valid region.
     __device__ void fetch(const float* __restrict__ base, int ld, int t0, int k0, int extent_t,
                           int extent_k, int tid) {
+        if constexpr (LD == LD_BUF || LD == LD_BUF4) {
+            left = extent_k - k0;
+            const int rows = min(KCONTIG ? extent_t - t0 : left, KCONTIG ? TILE : BKT);
+            const int cols = KCONTIG ? left : min(extent_t - t0, TILE);
+            const int bytes = left > 0 ? 4 * ((rows - 1) * ld + cols) : 0;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(base) + (KCONTIG ? (size_t)t0 * ld + k0 : (size_t)k0 * ld + t0), 0,
+                __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+#pragma unroll
+            for (int r = 0; r < CH; ++r) {
+                const int f = tid + r * NT;
+                const int row = KCONTIG ? min(f / (BKT / 4), rows - 1) : f / (TILE / 4);
+                const int c = 4 * (KCONTIG ? f % (BKT / 4) : f % (TILE / 4));
+                int off = 4 * (row * ld + c);
+                if (LD == LD_BUF4 && KCONTIG) off = c < left ? off : -16;
+                asm volatile("" : "+v"(off));   // one 128-bit load: constant distances from off
+                float x[4];
+                buf_load_floats<4>(rs, off, x);
+                v[r] = f32x4{x[0], x[1], x[2], x[3]};
+            }
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < CH; ++r) {
             const int f = tid + r * NT;
@@ -83,6 +125,10 @@ struct Slice {
             }
         }
     }
+    // Element e of chunk r, whose first k is kq4 within the slice.
+    __device__ float at(int r, int e, int kq4) const {
+        return LD == LD_BUF && KCONTIG && kq4 + e >= left ? 0.f : v[r][e];
+    }
     __device__ void store(float* lds, int stride, int tid) const {
 #pragma unroll
         for (int r = 0; r < CH; ++r) {
@@ -90,7 +136,7 @@ struct Slice {
             if (KCONTIG) {
                 const int t = f / (BKT / 4), kq = f % (BKT / 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) lds[(4 * kq + e) * stride + t] = v[r][e];
+                for (int e = 0; e < 4; ++e) lds[(4 * kq + e) * stride + t] = at(r, e, 4 * kq);
             } else {
                 const int k = f / (TILE / 4), tq = f % (TILE / 4);
                 *reinterpret_cast<f32x4*>(&lds[k * stride + 4 * tq]) = v[r];
@@ -115,7 +161,7 @@ struct Slice {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int k = 4 * kq + e;
-                    lds[k * 64 + swz64(k, t)] = v[r][e];
+                    lds[k * 64 + swz64(k, t)] = at(r, e, 4 * kq);
                 }
             } else {
                 const int k = f / (TILE / 4), tq = f % (TILE / 4);
@@ -128,7 +174,7 @@ struct Slice {
 // One work-group tile TBM x TBN of C (128 x 128, or 64 x 256 / 256 x 64 for products with M
 // or N at most 64) at the origin tile_of(m0, n0) sets; the 4 waves tile it in 64 x 64
 // sub-tiles.
-template <bool TA, bool TB, bool VA, bool VB, int TBM, int TBN, typename TileOf>
+template <bool TA, bool TB, int VA, int VB, int TBM, int TBN, typename TileOf>
 __device__ __forceinline__ void gemm_f32_tile(int M, int N, int K, const float* __restrict__ A,
                                               int lda, const float* __restrict__ B, int ldb,
                                               float beta, float* __restrict__ C, int ldc,
@@ -246,7 +292,7 @@ __device__ __forceinline__ void gemm_f32_tile(int M, int N, int K, const float* 
 // The kernel body: batch member blockIdx.y (strides in elements; 0 for a single product).  In
 // a split-K launch the members are the chunks of K, and the last one takes the ragged rest,
 // k_last (= K otherwise).
-template <bool TA, bool TB, bool VA, bool VB, int TBM, int TBN>
+template <bool TA, bool TB, int VA, int VB, int TBM, int TBN>
 __device__ __forceinline__ void gemm_f32_grid_tile(int M, int N, int K, const float* __restrict__ A,
                                                    int lda, const float* __restrict__ B, int ldb,
                                                    float beta, float* __restrict__ C, int ldc,
@@ -267,7 +313,7 @@ __device__ __forceinline__ void gemm_f32_grid_tile(int M, int N, int K, const fl
     });
 }
 
-template <bool TA, bool TB, bool VA, bool VB, int TBM, int TBN>
+template <bool TA, bool TB, int VA, int VB, int TBM, int TBN>
 __global__ void __launch_bounds__(NTHREADS)
 gemm_f32_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
                 const float* __restrict__ B, int ldb, float beta, float* __restrict__ C, int ldc,
@@ -283,7 +329,7 @@ gemm_f32_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
 // same box, fp32 4096^3 NN 1.080 -> 1.055 ms, TN 1.094-1.099 -> 1.062-1.066, 8192 x 8192 x 2048
 // 1-3% faster; with fewer tiles per CU the default form is faster (2048^3, one per CU: 175 ->
 // 184 us; 3000^3 NN 520 -> 535-543 us).
-template <bool TA, bool TB, bool VA, bool VB>
+template <bool TA, bool TB, int VA, int VB>
 __global__ void __launch_bounds__(NTHREADS)
 __attribute__((amdgpu_waves_per_eu(4, 4)))
 gemm_f32_occ4_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
@@ -302,7 +348,7 @@ gemm_f32_occ4_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
 // of it (TM = 128 at D = 128; two 64 x 64 blocks per tile at D = 64); the tiles go heaviest
 // first, and consecutive work-groups take consecutive slices, so with BH a multiple of 8 each
 // XCD reads the K rows of its own slices.
-template <bool VA, bool VB, int D>
+template <int VA, int VB, int D>
 __global__ void __launch_bounds__(NTHREADS)
 flash_dq_from_ds_kernel(int BH, int S, int T, int causal, const float* __restrict__ dS,
                         long long slice, const float* __restrict__ Kr, float beta,
@@ -332,7 +378,7 @@ flash_dq_from_ds_kernel(int BH, int S, int T, int causal, const float* __restric
 // loop runs in groups of PF slices and the zero slices past K in a last group cost products.
 constexpr int KS_NT = 512, KS_BK = 32;
 
-template <bool TA, bool TB, bool VA, bool VB, int PF>
+template <bool TA, bool TB, int VA, int VB, int PF>
 __global__ void __launch_bounds__(KS_NT)
 gemm_f32_ks_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
                    const float* __restrict__ B, int ldb, float beta, float* __restrict__ C, int ldc,
@@ -427,6 +473,157 @@ gemm_f32_ks_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
         if (row < M) {
             float* c = C + (size_t)row * ldc + col;
             float v = (beta == 0.f ? acc[r] : acc[r] + beta * *c) + (row_bias ? bias[row] : bcol);
+            if (relu) v = v < 0.f ? 0.f : v;
+            *c = v;
+        }
+    }
+}
+
+// ---- small and middling grids: a 32 x 32 tile's k split over the waves of a work-group ---------
+// Bound by latency: a grid of large tiles leaves CUs idle and each work-group alone with its chain
+// of slice loads, LDS stores, barriers and operand reads.  Here a work-group of NW waves owns a
+// 32 x 32 tile and wave w takes the 32-wide k slices w, w + NW, ...; a wave stages its own operands
+// in its own LDS, so nothing waits at a barrier until the partial tiles meet in LDS at the end
+// (added in wave order).  Twice the operand traffic of a 64 x 64 tile, which is why larger grids
+// keep those.  Same box, us, before / now: 512^3 24.8 / 6.4, 513 x 517 x 301 45.5 / 7.9, 700^3
+// 20.9 / 12.7, 4096 x 257 x 784 NT 38.0 / 26.8, 8192 x 64 x 512 17.2 / 10.4.
+// LDS per wave: a k-contiguous operand as [row][k], pitch 36 floats (16-byte stores, and one
+// 16-byte read gives a lane 4 k of its row; 16 rows start on distinct groups of 4 banks); the
+// other as [k][32], rows k and k + 4 side by side, so the two halves of an operand read fall in
+// opposite halves of the banks.  Products take k = 8 s + 4 (l / 32) + j at step (s, j): the order
+// of k within a slice is free as long as both operands agree.  Two slices are in flight in
+// registers while a third is multiplied.  All loads are LD_BUF's.  Measured and not kept: the next
+// half slice's operands read under the products of this one (more registers: 512^3 6.4 -> 8.6 us),
+// and 64 x 32 or 64 x 64 tiles a wave.
+constexpr int WV_BK = 32, WV_PITCH = 36;
+
+template <bool KCONTIG>
+struct WaveSlice {
+    f32x4 v[4];
+    int left;
+    // rows / columns t0 .. t0 + 31 and k0 .. k0 + 31 of the operand (see Slice::fetch)
+    __device__ void fetch(const float* __restrict__ base, int ld, int t0, int k0, int extent_t,
+                          int extent_k, int lane) {
+        left = extent_k - k0;
+        const int rows = min(KCONTIG ? extent_t - t0 : left, 32);
+        const int cols = KCONTIG ? left : min(extent_t - t0, 32);
+        const int bytes = left > 0 ? 4 * ((rows - 1) * ld + cols) : 0;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(base) + (KCONTIG ? (size_t)t0 * ld + k0 : (size_t)k0 * ld + t0), 0,
+            __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = KCONTIG ? min(8 * r + (lane >> 3), rows - 1) : 8 * r + (lane >> 3);
+            int off = 4 * (row * ld + 4 * (lane & 7));
+            asm volatile("" : "+v"(off));
+            float x[4];
+            buf_load_floats<4>(rs, off, x);
+            v[r] = f32x4{x[0], x[1], x[2], x[3]};
+        }
+    }
+    __device__ static int krow(int k) { return (k & ~7) + 2 * (k & 3) + ((k >> 2) & 1); }
+    __device__ void store(float* lds, int lane) const {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 8 * r + (lane >> 3), q = 4 * (lane & 7);
+            if (KCONTIG) {
+                f32x4 x = v[r];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = q + e < left ? x[e] : 0.f;
+                *reinterpret_cast<f32x4*>(lds + row * WV_PITCH + q) = x;
+            } else {
+                *reinterpret_cast<f32x4*>(lds + krow(row) * 32 + q) = v[r];
+            }
+        }
+    }
+    // x[s][j] = this lane's operand at k = 8 s + 4 h + j (row or column l32)
+    __device__ static void read(const float* lds, int l32, int h, float (&x)[4][4]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (KCONTIG) {
+                const f32x4 t = *reinterpret_cast<const f32x4*>(lds + l32 * WV_PITCH + 8 * s + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[s][j] = t[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[s][j] = lds[krow(8 * s + 4 * h + j) * 32 + l32];
+            }
+        }
+    }
+};
+
+template <bool TA, bool TB, int NW>
+__global__ void __launch_bounds__(64 * NW)
+gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
+                     const float* __restrict__ B, int ldb, float beta, float* __restrict__ C,
+                     int ldc, long long sA, long long sB, long long sC,
+                     const float* __restrict__ bias, int epi, int k_last) {
+    constexpr int SZ = 32 * WV_PITCH;
+    __shared__ __attribute__((aligned(16))) float lds[NW][2 * SZ];
+    if (blockIdx.y == gridDim.y - 1) K = k_last;
+    A += blockIdx.y * sA;
+    B += blockIdx.y * sB;
+    C += blockIdx.y * sC;
+    int tm, tn;
+    xcd_tile_order(blockIdx.x, gridDim.x, (M + 31) / 32, (N + 31) / 32, 8, tm, tn);
+    const int m0 = tm * 32, n0 = tn * 32;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float* la = lds[wave];
+    float* lb = la + SZ;
+    WaveSlice<!TA> sa[2];
+    WaveSlice<TB> sb[2];
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int nk = (K + WV_BK - 1) / WV_BK;
+    auto fetch = [&](auto set_c, int i) {   // the wave's slice i (past K: zeros)
+        constexpr int set = decltype(set_c)::value;
+        const int k0 = (wave + NW * i) * WV_BK;
+        sa[set].fetch(A, lda, m0, k0, M, K, lane);
+        sb[set].fetch(B, ldb, n0, k0, N, K, lane);
+    };
+    auto step = [&](auto set_c, int i) {
+        constexpr int set = decltype(set_c)::value;
+        sa[set].store(la, lane);   // behind the last slice's reads: a wave's LDS accesses are in order
+        sb[set].store(lb, lane);
+        fetch(set_c, i + 2);
+        float a[4][4], b[4][4];
+        WaveSlice<!TA>::read(la, l32, h, a);
+        WaveSlice<TB>::read(lb, l32, h, b);
+        __builtin_amdgcn_sched_barrier(0);   // all reads first: one LDS latency per slice
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], acc, 0, 0, 0);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    const int n = nk > wave ? (nk - wave + NW - 1) / NW : 0;   // this wave's slices
+    if (n > 0) {
+        fetch(even, 0);
+        fetch(odd, 1);
+        for (int i = 0; i < n; i += 2) {
+            step(even, i);
+            if (i + 1 < n) step(odd, i + 1);
+        }
+    }
+    // partial tiles, lane-major, in the waves' own LDS
+#pragma unroll
+    for (int r = 0; r < 16; ++r) la[r * 64 + lane] = acc[r];
+    __syncthreads();
+    const bool row_bias = bias && (epi & DH_EPI_ROW_BIAS), relu = epi & DH_EPI_RELU;
+#pragma unroll
+    for (int i = 0; i < 16 / NW; ++i) {
+        const int r = wave + NW * i;   // register r of every wave
+        float v = lds[0][r * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += lds[w][r * 64 + lane];
+        const int row = m0 + 8 * (r >> 2) + 4 * h + (r & 3), col = n0 + l32;
+        if (row < M && col < N) {
+            float* c = C + (size_t)row * ldc + col;
+            v = (beta == 0.f ? v : v + beta * *c) + (bias ? bias[row_bias ? row : col] : 0.f);
             if (relu) v = v < 0.f ? 0.f : v;
             *c = v;
         }
@@ -528,7 +725,7 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     const int l32 = lane & 31, h = lane >> 5;
     const int wm = (wave / WN) * WT, wn = (wave % WN) * WT;
 
-    Slice<true, VA, TBM> sa[2];
+    Slice<true, VA ? LD_VEC : LD_SCALAR, TBM> sa[2];
     ConvSlice<TBN> sb[2];
     sb[0].init(g, n0, P, tid);
     sb[1].init(g, n0, P, tid);
@@ -632,7 +829,15 @@ __global__ void __launch_bounds__(256) splitk_reduce(const float* __restrict__ p
     const size_t MN = (size_t)M * N;
     for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < MN; e += (size_t)gridDim.x * 256) {
         float v = 0.f;
-        for (int s = 0; s < S; ++s) v += part[s * MN + e];
+        int s = 0;
+        for (; s + 8 <= S; s += 8) {   // eight loads in flight (one at a time: 16 us for S = 32)
+            float p[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) p[u] = part[(s + u) * MN + e];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += p[u];
+        }
+        for (; s < S; ++s) v += part[s * MN + e];
         const int r = (int)(e / N), c = (int)(e % N);
         float* o = C + (size_t)r * ldc + c;
         v = (beta == 0.f ? v : v + beta * *o) + (bias ? bias[(epi & DH_EPI_ROW_BIAS) ? r : c] : 0.f);
@@ -735,7 +940,7 @@ conv_wgrad_kernel(int Cout, int P, int R, const float* __restrict__ dY, const fl
 
     ColTGeom<TBN> cg;
     cg.init(g, R, n0, tid);
-    Slice<true, VA, TBM> sa[2];
+    Slice<true, VA ? LD_VEC : LD_SCALAR, TBM> sa[2];
     ColTSlice<TBN> sb[2];
     // slice kt of the chunk: image n, positions p0 ..; past the chunk's end: zeros
     auto fetch = [&](auto set_c, int kt) {
@@ -883,17 +1088,21 @@ auto pick_kernel(int M, int N, int K, const float* A, int lda, long long sA, con
     const int ca = TA ? M : K, cb = TB ? K : N;
     const bool va = ((uintptr_t)A % 16 == 0) && (lda % 4 == 0) && (sA % 4 == 0) && (ca % 4 == 0);
     const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 4 == 0) && (sB % 4 == 0) && (cb % 4 == 0);
+    const bool buf = lda <= LD_BUF_MAX && ldb <= LD_BUF_MAX, k4 = K % 4 == 0;
     if constexpr (TBM == 128 && TBN == 128) {
         static const bool occ4 = [] {
             const char* e = std::getenv("DH_GEMM_F32_OCC4");   // tuning knob: 0 or 1
             return !e || std::atoi(e) != 0;
         }();
-        if (occ4 && va && vb && wgs >= 4LL * num_cus()) return gemm_f32_occ4_kernel<TA, TB, true, true>;
+        if (occ4 && wgs >= 4LL * num_cus() && (buf || (va && vb)))
+            return buf && k4 ? gemm_f32_occ4_kernel<TA, TB, LD_BUF4, LD_BUF4>
+                 : buf       ? gemm_f32_occ4_kernel<TA, TB, LD_BUF, LD_BUF>
+                             : gemm_f32_occ4_kernel<TA, TB, LD_VEC, LD_VEC>;
     }
-    return va && vb ? gemm_f32_kernel<TA, TB, true, true, TBM, TBN>
-         : va       ? gemm_f32_kernel<TA, TB, true, false, TBM, TBN>
-         : vb       ? gemm_f32_kernel<TA, TB, false, true, TBM, TBN>
-                    : gemm_f32_kernel<TA, TB, false, false, TBM, TBN>;
+    return buf && k4  ? gemm_f32_kernel<TA, TB, LD_BUF4, LD_BUF4, TBM, TBN>
+         : buf        ? gemm_f32_kernel<TA, TB, LD_BUF, LD_BUF, TBM, TBN>
+         : va && vb   ? gemm_f32_kernel<TA, TB, LD_VEC, LD_VEC, TBM, TBN>
+                      : gemm_f32_kernel<TA, TB, LD_SCALAR, LD_SCALAR, TBM, TBN>;
 }
 
 // One grid of the tiled kernel; gridDim.y carries the batch member, in chunks of 65535 (the
@@ -917,10 +1126,10 @@ int launch_grid(int M, int N, int K, const float* A, int lda, const float* B, in
 // One product (bt.count == 1) with K cut into about S chunks (multiples of BK) run as gridDim.y
 // members writing fp32 partials, which splitk_reduce adds in order with the epilogue.
 // DH_ERR_UNSUPPORTED, with nothing launched, when no workspace can be had.
-template <bool TA, bool TB, int TBM, int TBN>
-int launch_split_k(int M, int N, int K, int S, const float* A, int lda, const float* B, int ldb,
-                   float beta, float* C, int ldc, const Batch& bt) {
-    const int tiles = ((M + TBM - 1) / TBM) * ((N + TBN - 1) / TBN);
+// pick(sA, sB): the kernel, of `threads` threads on a grid of `tiles`.
+template <bool TA, bool TB, typename Pick>
+int launch_split(int M, int N, int K, int S, const float* A, int lda, const float* B, int ldb,
+                 float beta, float* C, int ldc, const Batch& bt, int tiles, int threads, Pick pick) {
     hipStream_t s = stream();
     const int Kc = ((K + S - 1) / S + BK - 1) / BK * BK;   // chunk of K, multiple of BK
     S = (K + Kc - 1) / Kc;
@@ -931,9 +1140,9 @@ int launch_split_k(int M, int N, int K, int S, const float* A, int lda, const fl
     // the whole K: 16-byte loads along k only where K is a multiple of 4, so that a ragged last
     // chunk has no 4-wide group crossing its end.
     const long long sA = TA ? (long long)Kc * lda : Kc, sB = TB ? Kc : (long long)Kc * ldb;
-    auto kern = pick_kernel<TA, TB, TBM, TBN>(M, N, K, A, lda, sA, B, ldb, sB);
-    kern<<<dim3(tiles, S), NTHREADS, 0, s>>>(M, N, Kc, A, lda, B, ldb, 0.f, part, N, sA, sB,
-                                             (long long)M * N, nullptr, 0, K - (S - 1) * Kc);
+    auto kern = pick(sA, sB);
+    kern<<<dim3(tiles, S), threads, 0, s>>>(M, N, Kc, A, lda, B, ldb, 0.f, part, N, sA, sB,
+                                            (long long)M * N, nullptr, 0, K - (S - 1) * Kc);
     int st = check_launch("dh_gemm_f32(split-K)");
     if (st == DH_OK) {
         const int cus = num_cus();
@@ -944,6 +1153,24 @@ int launch_split_k(int M, int N, int K, int S, const float* A, int lda, const fl
     }
     dh_free(part);   // pooled; later users of the buffer are ordered on the stream
     return st;
+}
+
+template <bool TA, bool TB, int TBM, int TBN>
+int launch_split_k(int M, int N, int K, int S, const float* A, int lda, const float* B, int ldb,
+                   float beta, float* C, int ldc, const Batch& bt) {
+    return launch_split<TA, TB>(M, N, K, S, A, lda, B, ldb, beta, C, ldc, bt,
+                                ((M + TBM - 1) / TBM) * ((N + TBN - 1) / TBN), NTHREADS,
+                                [&](long long sA, long long sB) {
+        return pick_kernel<TA, TB, TBM, TBN>(M, N, K, A, lda, sA, B, ldb, sB);
+    });
+}
+template <bool TA, bool TB>
+int launch_split_wave(int M, int N, int K, int S, const float* A, int lda, const float* B, int ldb,
+                      float beta, float* C, int ldc, const Batch& bt) {
+    return launch_split<TA, TB>(M, N, K, S, A, lda, B, ldb, beta, C, ldc, bt,
+                                ((M + 31) / 32) * ((N + 31) / 32), 512, [](long long, long long) {
+        return gemm_f32_wave_kernel<TA, TB, 8>;
+    });
 }
 
 template <bool TA, bool TB, int TBM, int TBN>
@@ -1189,14 +1416,14 @@ int launch_ks(int M, int N, int K, const float* A, int lda, const float* B, int 
     const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 4 == 0) && (bt.sB % 4 == 0) && (cb % 4 == 0);
     const int nk = (K + KS_BK - 1) / KS_BK;
     const bool deep = (nk % 4 == 0 && nk >= 8) || nk >= 40;   // a last group wastes < 10%
-    auto kern = deep ? (va && vb ? gemm_f32_ks_kernel<TA, TB, true, true, 4>
-                        : va     ? gemm_f32_ks_kernel<TA, TB, true, false, 4>
-                        : vb     ? gemm_f32_ks_kernel<TA, TB, false, true, 4>
-                                 : gemm_f32_ks_kernel<TA, TB, false, false, 4>)
-                     : (va && vb ? gemm_f32_ks_kernel<TA, TB, true, true, 2>
-                        : va     ? gemm_f32_ks_kernel<TA, TB, true, false, 2>
-                        : vb     ? gemm_f32_ks_kernel<TA, TB, false, true, 2>
-                                 : gemm_f32_ks_kernel<TA, TB, false, false, 2>);
+    const bool buf = lda <= LD_BUF_MAX && ldb <= LD_BUF_MAX, k4 = K % 4 == 0;
+    auto kern = buf && k4 ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_BUF4, LD_BUF4, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_BUF4, LD_BUF4, 2>)
+              : buf       ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_BUF, LD_BUF, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_BUF, LD_BUF, 2>)
+              : va && vb  ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_VEC, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_VEC, 2>)
+                          : gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_SCALAR, 2>;
     const int tiles = ((M + 63) / 64) * ((N + 63) / 64);
     for (int b0 = 0; b0 < bt.count; b0 += 65535) {
         const int nb = bt.count - b0 < 65535 ? bt.count - b0 : 65535;
@@ -1206,6 +1433,52 @@ int launch_ks(int M, int N, int K, const float* A, int lda, const float* B, int 
         DH_TRY(check_launch("dh_gemm_f32(64x64, 8 waves)"));
     }
     return DH_OK;
+}
+
+// The 32 x 32 tiles of gemm_f32_wave_kernel where they are the faster form; DH_ERR_UNSUPPORTED
+// otherwise, with nothing launched.  Times in us, fitted to measurements on both sides (30 shapes
+// from 128 x 128 x 64 to 1500^3): a CU takes 0.16 us per tile and 32-deep slice, 0.185 with
+// several tiles on it, a work-group's slices rounded up to its waves; a 64 x 64 tile takes
+// 0.0185 us per k, and the grid as many as its fullest CU (past one 128 x 128 tile per CU the
+// larger tiles are always better).  Few tiles with a long K also split K over work-groups (6 us
+// for the second launch), where the 64 x 64 form does the same at about 0.6 of the matrix rate.
+template <bool TA, bool TB>
+int launch_wave(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta,
+                float* C, int ldc, const Batch& bt) {
+    const long long cus = num_cus();
+    const long long tiles = (long long)((M + 31) / 32) * ((N + 31) / 32);
+    const long long t32 = tiles * bt.count;
+    const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * bt.count;
+    const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * bt.count;
+    if (K < 1 || lda > LD_BUF_MAX || ldb > LD_BUF_MAX || bt.count > 65535 || t128 >= cus)
+        return DH_ERR_UNSUPPORTED;
+    auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
+    auto wave_us = [&](int S, int nw) {
+        const int slices = (K / S + 31) / 32;
+        return rounds(t32 * S) * nw * ((slices + nw - 1) / nw) * (t32 * S > cus ? 0.185 : 0.16);
+    };
+    const int nw = t32 > cus && wave_us(1, 4) <= wave_us(1, 8) ? 4 : 8;
+    int S = 1;
+    if (bt.count == 1 && 2 * t32 <= cus && K >= 1024) {
+        S = (int)(cus / t32);
+        S = S > K / 512 ? K / 512 : S;
+        if (S < 2 || 6.0 + wave_us(S, 8) >= wave_us(1, 8)) S = 1;
+    }
+    const double here = S > 1 ? 6.0 + wave_us(S, 8) : wave_us(1, nw);
+    // at most half the CUs busy with 64 x 64 tiles: only their split over K is ever better
+    const double there = 2 * t64 > cus ? rounds(t64) * K * 0.0185
+                       : bt.count == 1 && K >= 512 ? 7.0 + (double)t64 * K * 8192 / 157e6 / 0.6
+                                                   : INFINITY;
+    if (here >= there) return DH_ERR_UNSUPPORTED;
+    if (S > 1) return launch_split_wave<TA, TB>(M, N, K, S, A, lda, B, ldb, beta, C, ldc, bt);
+    const dim3 grid((unsigned)tiles, (unsigned)bt.count);
+    if (nw == 4)
+        gemm_f32_wave_kernel<TA, TB, 4><<<grid, 256, 0, stream()>>>(
+            M, N, K, A, lda, B, ldb, beta, C, ldc, bt.sA, bt.sB, bt.sC, bt.bias, bt.epi, K);
+    else
+        gemm_f32_wave_kernel<TA, TB, 8><<<grid, 512, 0, stream()>>>(
+            M, N, K, A, lda, B, ldb, beta, C, ldc, bt.sA, bt.sB, bt.sC, bt.bias, bt.epi, K);
+    return check_launch("dh_gemm_f32(32 x 32)");
 }
 
 template <bool TA, bool TB>
@@ -1219,6 +1492,8 @@ int launch(int M, int N, int K, const float* A, int lda, const float* B, int ldb
         const int st = launch_skinny<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
         if (st != DH_ERR_UNSUPPORTED) return st;   // no workspace: the tiled kernels below
     }
+    const int wst = launch_wave<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
+    if (wst != DH_ERR_UNSUPPORTED) return wst;   // else a larger tile is the better form
     const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * bt.count;
     if ((M <= 64 && N > 64) || (N <= 64 && M > 64)) {
         const long long tn = (long long)((M <= 64 ? N : M) + 255) / 256 * bt.count;
@@ -1296,10 +1571,10 @@ int launch_dq_from_ds(int BH, int S, int causal, const float* dS, long long slic
     // 16-byte loads of dS rows need every tile's K extent (a multiple of 128, or S) to be a
     // multiple of 4; K rows (D floats) need an aligned base
     const bool va = S % 4 == 0, vb = (uintptr_t)K % 16 == 0;
-    auto kern = va && vb ? flash_dq_from_ds_kernel<true, true, D>
-              : va       ? flash_dq_from_ds_kernel<true, false, D>
-              : vb       ? flash_dq_from_ds_kernel<false, true, D>
-                         : flash_dq_from_ds_kernel<false, false, D>;
+    auto kern = S > LD_BUF_MAX - 128 ? (va && vb ? flash_dq_from_ds_kernel<LD_VEC, LD_VEC, D>
+                                                 : flash_dq_from_ds_kernel<LD_SCALAR, LD_SCALAR, D>)
+              : va ? flash_dq_from_ds_kernel<LD_BUF4, LD_BUF4, D>
+                   : flash_dq_from_ds_kernel<LD_BUF, LD_BUF, D>;
     kern<<<(unsigned)(T * BH * (D == 128 ? 1 : 2)), NTHREADS, 0, stream()>>>(BH, S, T, causal, dS,
                                                                             slice, K, beta, dQ);
     return check_launch("flash backward dQ from dS");

@@ -749,3 +749,53 @@ def test_bf16_mid_shapes_on_the_general_kernel():
                        capture_output=True, text=True, timeout=110)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.count("general") == 12, r.stdout
+
+
+# 32 x 32 tiles (one slice, ragged slices, split K), 64 x 64 tiles, their 8-wave form, 128 x 128
+# tiles with and without four work-groups per CU
+@pytest.mark.parametrize("M,N,K", [(17, 33, 1), (33, 47, 35), (64, 64, 64), (513, 130, 301),
+                                   (200, 200, 4001), (90, 3000, 260), (1000, 1001, 301),
+                                   (1300, 1300, 71), (2100, 2050, 67), (4100, 4097, 19)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_fp32_unaligned_rows_read_nothing_outside(M, N, K, ta, tb):
+    # Rows of any alignment are read 16 bytes at a time.  Every stored row is followed by 1 or
+    # 3 padding values of NaN (odd and even leading dimensions) and the operands start 4 bytes
+    # past a 16-byte boundary: a value taken from outside the matrix would show.  K = 4n and
+    # 4n + 1, 4n + 3 end rows at every position of a load.  Bound: 1e-5 sqrt(K), as check_f32.
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+
+    def stored(X, pad):
+        X = np.concatenate([X, np.full((X.shape[0], pad), np.nan)], axis=1).astype(np.float32)
+        return hip.DeviceBuffer.from_numpy(np.concatenate([[np.float32(np.nan)], X.ravel()])), X.shape[1]
+
+    dA, lda = stored(A.T if ta else A, 1 + 2 * tb)
+    dB, ldb = stored(B.T if tb else B, 3 - 2 * ta)
+    dC = hip.DeviceBuffer.from_numpy(C0)
+    hip.gemm_f32(ta, tb, M, N, K, dA.ptr + 4, lda, dB.ptr + 4, ldb, 1.0, dC, N)
+    ref = f32(A).astype(np.float64) @ f32(B).astype(np.float64) + C0
+    assert maxrel(dC.numpy(), ref) <= 1e-5 * np.sqrt(max(K, 4))
+
+
+@pytest.mark.parametrize("Bt,M,N,K", [(3, 33, 40, 97), (7, 100, 70, 64), (1, 100, 100, 2500)])
+@pytest.mark.parametrize("relu,row_bias", [(False, False), (True, False), (True, True)])
+def test_fp32_32x32_tiles_batched_epilogue(Bt, M, N, K, relu, row_bias):
+    for ta, tb, beta in ((0, 1, 0.5), (1, 0, 0.0)):
+        got, ref = _ex("f32", ta, tb, Bt, M, N, K, beta=beta, relu=relu, row_bias=row_bias)
+        assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)
+
+
+def test_fp32_leading_dimensions_past_32_bit_offsets():
+    # above 2^20: element by element, or (aligned) with 64-bit addresses
+    for ld in ((1 << 20) + 1, (1 << 20) + 4):
+        M, N, K = 20, 24, 36
+        rng = np.random.default_rng(ld)
+        A, B = f32(rng.standard_normal((M, K))), f32(rng.standard_normal((K, N)))
+        wide = np.zeros((M - 1) * ld + K, np.float32)
+        for i in range(M):
+            wide[i * ld:i * ld + K] = A[i]
+        dA, dB = hip.DeviceBuffer.from_numpy(wide), hip.DeviceBuffer.from_numpy(B)
+        dC = hip.DeviceBuffer.empty((M, N), np.float32)
+        hip.gemm_f32(0, 0, M, N, K, dA, ld, dB, N, 0.0, dC, N)
+        assert maxrel(dC.numpy(), A.astype(np.float64) @ B.astype(np.float64)) <= 1e-5 * np.sqrt(K)
