@@ -558,6 +558,20 @@ __device__ inline void store_tile(int M, int N, float beta, float* __restrict__ 
         // are not stored; bias indices are clamped so nothing outside C or the bias is read.
         const int row0 = m0 + wm + 4 * h, col0 = n0 + wn + l32;
         const bool row_bias = bias && (epi & DH_EPI_ROW_BIAS);
+        if (beta == 0.f && !bias && !(epi & DH_EPI_RELU)) {
+            // A store and its bounds only: with the loads and selects of the general form below a
+            // 128-wide tile's edge took ~8 us more.  Same box, us: 1000 x 1000 x 1024 21.7 -> 14.2
+            // (on 128 x 128 tiles), 4095^3 192 -> 175, 8000^3 812 -> 775.
+#pragma unroll
+            for (int a = 0; a < FM; ++a)
+#pragma unroll
+                for (int b = 0; b < FN; ++b)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (row0 + 32 * a + 8 * (r >> 2) + (r & 3) < M && col0 + 32 * b < N)
+                            __builtin_nontemporal_store(acc[a][b][r], at(a, b, r));
+            return;
+        }
 #pragma unroll
         for (int a = 0; a < FM; ++a)
 #pragma unroll
@@ -1001,6 +1015,156 @@ gemm_bf16_mid_kernel(int M, int N, int K, const uint16_t* __restrict__ A, int ld
     store_tile<FM, FN, 128>(M, N, beta, C, ldc, bias, epi, m0, n0, wm, wn, lane, acc);
 }
 
+// ---------------------------------------------------------------------------------
+// Few tiles per CU (stage64_tiles): 64 x 64 tiles, 64-k stages, 4 waves of 32 x 32.  Bound by the
+// chain of a work-group's stages: with one or two on a CU little covers its barriers and LDS
+// latencies (a 32-k stage of the 128 x 128 kernel above takes 690 cycles alone on a CU, 256 of
+// them products; 128-wide tiles of 64-k stages were no faster), so a stage is twice as deep: one
+// barrier and one DMA wait per four 16-k steps, every step's operands read under the step before,
+// rows of a k-contiguous operand fetched as whole 128-byte lines, and four times the work-groups.
+// A ring of NS stages (16 KB each), DMA NS - 1 ahead.
+// ---------------------------------------------------------------------------------
+template <bool KCONTIG>
+struct StageOperand {
+    // One stage is 8 DMA blocks of 1 KB, 2 per wave.  LDS tile, 16-byte chunks:
+    //   k-contiguous [64 rows][64 k]: chunk c of row r at c ^ (r/2 % 8) (see DeepKOperand);
+    //   otherwise [64 k][64]: chunk c of row k at c ^ 4 (k/2 % 2) (two rows per 64 banks), so the
+    //   four rows of a transposing read's half-wave fall on distinct banks.
+    static constexpr int T = 64, PER = 2, ELEMS = 64 * T;
+    uint32_t off[PER], step, bytes;   // as FastOperand's
+    uint32_t last[KCONTIG ? PER : 1];   // offsets in the last stage: chunks at or past K read zeros
+
+    __device__ static int swz(int k) { return 4 * ((k >> 1) & 1); }
+    // rows x cols: the stored operand; klast: k of its last stage that lie below K.  The buffer
+    // range ends with its last value (an odd last column with its dword).
+    __device__ void init(int ld, int rows, int cols, int t0, int klast, int wave, int lane) {
+#pragma unroll
+        for (int t = 0; t < PER; ++t) {
+            const int b = PER * wave + t;
+            if (KCONTIG) {
+                const int row = 8 * b + (lane >> 3);
+                const int c = (lane & 7) ^ ((row >> 1) & 7);
+                off[t] = 2u * ((uint32_t)(t0 + row) * ld + 8 * c);
+                last[t] = 8 * c < klast ? off[t] : 0xFFFFFFF0u;
+            } else {
+                const int k = 8 * b + (lane >> 3);
+                const int c = (lane & 7) ^ swz(k);
+                off[t] = 2u * ((uint32_t)k * ld + t0 + 8 * c);
+            }
+        }
+        step = KCONTIG ? 128u : 128u * (uint32_t)ld;
+        // (a k-contiguous row ends with its last chunk: K is a multiple of 8, or the row is padded)
+        bytes = 2u * ((uint32_t)(rows - 1) * (uint32_t)ld + (KCONTIG ? (cols + 7) & ~7 : (cols + 1) & ~1));
+    }
+    __device__ void issue(const uint16_t* __restrict__ g, int kt, bool at_end, uint16_t* lds,
+                          int wave) const {
+        const uint32_t soff = __builtin_amdgcn_readfirstlane((uint32_t)kt * step);
+        const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(lds) + 1024u * PER * wave);
+        const u32x4 rs = make_rsrc(g, bytes);
+#pragma unroll
+        for (int t = 0; t < PER; ++t)
+            lds_dma16_buf_so(KCONTIG && at_end ? last[KCONTIG ? t : 0] : off[t], rs, soff,
+                             base + 1024u * t);
+    }
+    // MFMA operand for tile rows / columns o .. o + 31, 16-k step kk of the stage.
+    __device__ static bf16x8 frag(const uint16_t* lds, int o, int kk, int lane) {
+        const int h = lane >> 5;
+        if (KCONTIG) {
+            const int row = o + (lane & 31);
+            const int p = (2 * kk + h) ^ ((row >> 1) & 7);
+            return *reinterpret_cast<const bf16x8*>(lds + row * 64 + 8 * p);
+        } else {
+            const int G = (lane & 31) >> 4, i = lane & 15;
+            const int n = o + 16 * G + 4 * (i & 3);
+            s16x4 r[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int k = 16 * kk + 8 * h + 4 * q + (i >> 2);
+                r[q] = ds_read_tr(lds + k * T + 8 * ((n >> 3) ^ swz(k)) + 4 * ((n >> 2) & 1));
+            }
+            return __builtin_bit_cast(bf16x8, __builtin_shufflevector(r[0], r[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+};
+
+// A k-contiguous operand has K a multiple of 8 (the host pads copies with zeros): past it whole
+// chunks of the last stage take an offset outside the buffer and land as zeros, as do k rows past
+// the end of the other kind, so no tail steps follow.
+template <bool TA, bool TB, int NS>
+__global__ void __launch_bounds__(256)
+gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
+                         const uint16_t* __restrict__ B, int ldb, float beta,
+                         float* __restrict__ C, int ldc, long long sA, long long sB, long long sC,
+                         const float* __restrict__ bias, int epi, int k_last) {
+    using OA = StageOperand<!TA>;
+    using OB = StageOperand<TB>;
+    constexpr int T = OA::T, FM = 1, FN = 1;
+    __shared__ __attribute__((aligned(16))) uint16_t ring[NS * 2 * OA::ELEMS];
+    if (blockIdx.y == gridDim.y - 1) K = k_last;   // the rest of K (= K but for chunks of it)
+    A += blockIdx.y * sA;   // batch member, or chunk of K
+    B += blockIdx.y * sB;
+    C += blockIdx.y * sC;
+    int tm, tn;
+    xcd_tile_order(blockIdx.x, gridDim.x, (M + T - 1) / T, (N + T - 1) / T, 4, tm, tn);
+    const int m0 = tm * T, n0 = tn * T;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+
+    OA oa;
+    OB ob;
+    const int nk = (K + 63) / 64;   // >= 1
+    oa.init(lda, TA ? K : M, TA ? M : K, m0, K - 64 * (nk - 1), wave, lane);
+    ob.init(ldb, TB ? N : K, TB ? K : N, n0, K - 64 * (nk - 1), wave, lane);
+    f32x16 acc[FM][FN];
+#pragma unroll
+    for (int a = 0; a < FM; ++a)
+#pragma unroll
+        for (int b = 0; b < FN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+
+    auto stage_ptr = [&](int kt) { return ring + (kt % NS) * 2 * OA::ELEMS; };
+    auto issue = [&](int kt) {
+        uint16_t* st = stage_ptr(kt);
+        oa.issue(A, kt, kt == nk - 1, st, wave);
+        ob.issue(B, kt, kt == nk - 1, st + OA::ELEMS, wave);
+    };
+    const int pre = nk < NS - 1 ? nk : NS - 1;
+    for (int s = 0; s < pre; ++s) issue(s);
+    wait_dma_stages<2 * OA::PER>(pre - 1);
+    __syncthreads();
+    asm volatile("" ::"s"(C), "s"(ldc), "s"(beta), "s"(bias), "s"(epi));
+    bf16x8 f0a[FM], f0b[FN], f1a[FM], f1b[FN];
+    auto read = [&](int kt, int kk, bf16x8 (&fa)[FM], bf16x8 (&fb)[FN]) {
+        load_frags<OA, OB, FM, FN, OA::ELEMS>(stage_ptr(kt), kk, wm, wn, lane, fa, fb);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mma = [&](bf16x8 (&fa)[FM], bf16x8 (&fb)[FN]) {
+        mfma_block<FM, FN>(fa, fb, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    read(0, 0, f0a, f0b);
+    for (int kt = 0; kt < nk; ++kt) {
+        if (kt + NS - 1 < nk) issue(kt + NS - 1);
+        read(kt, 1, f1a, f1b);
+        mma(f0a, f0b);
+        read(kt, 2, f0a, f0b);
+        mma(f1a, f1b);
+        read(kt, 3, f1a, f1b);
+        mma(f0a, f0b);
+        if (kt + 1 < nk) {
+            // this wave's reads of stage kt are done, stage kt + 1 has landed
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            wait_dma_stages<2 * OA::PER>(min(nk - 1, kt + NS - 1) - (kt + 1));
+            __syncthreads();
+            read(kt + 1, 0, f0a, f0b);
+        }
+        mma(f1a, f1b);
+    }
+    store_tile<FM, FN, T>(M, N, beta, C, ldc, bias, epi, m0, n0, wm, wn, lane, acc);
+}
+
 template <bool TA, bool TB>
 int launch_fast(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
                 float beta, float* C, int ldc, const Batch& bt) {
@@ -1083,8 +1247,8 @@ int launch_fast(int M, int N, int K, const uint16_t* A, int lda, const uint16_t*
 }
 
 template <bool TA, bool TB>
-int launch_mid_grid(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
-                    float beta, float* C, int ldc, const Batch& bt) {
+int launch_mid(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+               float beta, float* C, int ldc, const Batch& bt) {
     for (int b0 = 0; b0 < bt.count; b0 += 65535) {   // gridDim.y = batch member
         const int nb = bt.count - b0 < 65535 ? bt.count - b0 : 65535;
         gemm_bf16_mid_kernel<TA, TB><<<dim3(((M + 127) / 128) * ((N + 127) / 128), nb), 256, 0,
@@ -1096,45 +1260,62 @@ int launch_mid_grid(int M, int N, int K, const uint16_t* A, int lda, const uint1
     return DH_OK;
 }
 
-// One product whose 128 x 128 tiles fill at most half the CUs with a long contraction (weight
-// gradients, K = the batch; 512 x 512 x 8192) splits K into S chunks of Kc (a multiple of 32,
-// the last chunk taking the rest) run as batch members of the same kernel, each writing an fp32
-// partial, which splitk_reduce_launch adds in a fixed order (reruns stay bit-identical) with
-// beta, the bias and ReLU.  The partials cost 8 S M N bytes of HBM traffic, so S aims at only
-// 2 work-groups per CU, at most 16 chunks of at least 256, and K below 2048 is not split
-// (1024^3: 13.4 us unsplit against 27.7 us in 8 chunks; 512^2 x 8192: 79 us unsplit, 34 us in
-// 32 chunks).
+// Whether 64-wide tiles of 64-k stages are the better form: up to two work-groups per CU (rings of
+// four stages, 64 KB), and up to three (rings of three) unless the contraction is long enough
+// for the 128 x 128 tiles' better reuse.  Same box, us, 128 x 128 / these: 512^3 7.9 / 4.7,
+// 1024^3 13.3 / 7.8, 1024 x 1536 x 2048 30.9 / 15.5, 1000^3 (K tail) 15.3 / 8.2, 2880 x 960 x 704
+// 11.8 / 9.2, 1536 x 2048 x 1024 14.7 / 12.5; but 1024 x 3072 x 4096 44.9 / 48.2, 2048 x 2048 x 1024
+// 15.9 / 17.7, 3072 x 2048 x 1024 21.8 / 24.2.
+bool stage64_tiles(int M, int N, int K, int count) {
+    const long long t = (long long)((M + 63) / 64) * ((N + 63) / 64) * count, cus = num_cus();
+    return t <= 2 * cus || (t <= 3 * cus && K <= 2048);
+}
+
+// 64-wide tiles of 64-k stages.  One product whose tiles fill at most half the CUs with a long
+// contraction (weight gradients, K = the batch; 512 x 512 x 8192) splits K into S chunks of Kc (a
+// multiple of 64, the last chunk taking the rest), one grid of S rows, each writing an fp32
+// partial, which splitk_reduce_launch adds in a fixed order (reruns stay bit-identical) with beta,
+// the bias and ReLU.  The partials cost 8 S M N bytes of HBM traffic and a launch, so S aims at
+// only 2 work-groups per CU, at most 16 chunks of at least 256, and K below 2048 is not split
+// (4096 x 128 x 1024: 6.9 us unsplit, 12.1 us in 4 chunks; 128 x 128 x 4096 10.0 us in 16 and
+// 512 x 512 x 8192 14.6 us in 8, where the 128 x 128 kernel's split took 14.8 and 23.6).
 template <bool TA, bool TB>
-int launch_mid(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
-               float beta, float* C, int ldc, const Batch& bt) {
-    const int tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    const int cus = num_cus();
+int launch_stage64(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+                   float beta, float* C, int ldc, const Batch& bt) {
+    const int tiles = ((M + 63) / 64) * ((N + 63) / 64), cus = num_cus();
     static const bool split_on = [] {
         const char* e = std::getenv("DH_GEMM_BF16_SPLITK");   // tuning knob: 0 or 1
         return !e || std::atoi(e) != 0;
     }();
+    const bool three = (long long)tiles * bt.count > 2LL * cus;   // see stage64_tiles
+    auto kern = three ? gemm_bf16_stage64_kernel<TA, TB, 3> : gemm_bf16_stage64_kernel<TA, TB, 4>;
     if (split_on && bt.count == 1 && 2 * tiles <= cus && K >= 2048) {
         int S = 2 * cus / tiles;
         S = S > 16 ? 16 : S;
         S = S > K / 256 ? K / 256 : S;
-        const int Kc = K / S / 32 * 32;
-        float* part = static_cast<float*>(dh_malloc((size_t)S * M * N * sizeof(float)));
+        const int Kc = ((K + S - 1) / S + 63) / 64 * 64;
+        S = (K + Kc - 1) / Kc;
+        const long long MN = (long long)M * N;
+        float* part = static_cast<float*>(dh_malloc((size_t)S * MN * sizeof(float)));
         if (part) {
-            const long long MN = (long long)M * N;
-            const Batch pb{TA ? (long long)Kc * lda : Kc, TB ? Kc : (long long)Kc * ldb, MN, S - 1,
-                           nullptr, 0};
-            int st = launch_mid_grid<TA, TB>(M, N, Kc, A, lda, B, ldb, 0.f, part, N, pb);
-            if (st == DH_OK)
-                st = launch_mid_grid<TA, TB>(M, N, K - (S - 1) * Kc, A + (S - 1) * pb.sA, lda,
-                                             B + (S - 1) * pb.sB, ldb, 0.f, part + (S - 1) * MN, N,
-                                             Batch{0, 0, 0, 1, nullptr, 0});
+            kern<<<dim3(tiles, S), 256, 0, stream()>>>(
+                M, N, Kc, A, lda, B, ldb, 0.f, part, N, TA ? (long long)Kc * lda : Kc,
+                TB ? Kc : (long long)Kc * ldb, MN, nullptr, 0, K - (S - 1) * Kc);
+            int st = check_launch("dh_gemm_bf16(64-k stages, split K)");
             if (st == DH_OK) st = splitk_reduce_launch(part, S, M, N, beta, C, ldc, bt.bias, bt.epi);
             dh_free(part);   // pooled; later users of the buffer are ordered on the stream
             return st;
         }
         // no workspace: the one-pass grid
     }
-    return launch_mid_grid<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
+    for (int b0 = 0; b0 < bt.count; b0 += 65535) {   // gridDim.y = batch member
+        const int nb = bt.count - b0 < 65535 ? bt.count - b0 : 65535;
+        kern<<<dim3(tiles, nb), 256, 0, stream()>>>(
+            M, N, K, A + b0 * bt.sA, lda, B + b0 * bt.sB, ldb, beta, C + b0 * bt.sC, ldc, bt.sA,
+            bt.sB, bt.sC, bt.bias, bt.epi, K);
+        DH_TRY(check_launch("dh_gemm_bf16(64-k stages)"));
+    }
+    return DH_OK;
 }
 
 template <bool TA, bool TB>
@@ -1148,39 +1329,53 @@ int launch_general(int M, int N, int K, const uint16_t* A, int lda, const uint16
     return launch_vec<TA, TB, false, false>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
 }
 
-// Rows of cols bf16 values at leading dimension ld -> rows at ldo (a multiple of 8, dst
-// 16-byte aligned), zero-filled to ldo: 16 bytes per thread and store, grid-stride.
-__global__ __launch_bounds__(256) void copy_rows_bf16(const uint16_t* __restrict__ src, int ld,
-                                                     uint16_t* __restrict__ dst, int ldo,
-                                                     int rows, int cols) {
-    const int chunks = ldo / 8;
-    const long long total = (long long)rows * chunks;
+// Operand blockIdx.y: rows of cols bf16 values at leading dimension ld -> rows at ldo (a multiple
+// of 8, dst 16-byte aligned), zero-filled to ldo: 16 bytes per thread, load and store (the load at
+// 2-byte alignment, value by value where it would pass the row's end), grid-stride.
+struct RowCopy {
+    const uint16_t* src;
+    uint16_t* dst;
+    int ld, ldo, rows, cols;
+};
+
+__global__ __launch_bounds__(256) void copy_rows_bf16(RowCopy c0, RowCopy c1) {
+    typedef short s16x8u __attribute__((ext_vector_type(8), aligned(2)));
+    const RowCopy cp = blockIdx.y ? c1 : c0;
+    const int chunks = cp.ldo / 8;
+    const long long total = (long long)cp.rows * chunks;
     for (long long x = (long long)blockIdx.x * 256 + threadIdx.x; x < total;
          x += (long long)gridDim.x * 256) {
         const int r = (int)(x / chunks), c = (int)(x - (long long)r * chunks) * 8;
-        const uint16_t* sp = src + (size_t)r * ld + c;
+        const uint16_t* sp = cp.src + (size_t)r * cp.ld + c;
         s16x8 v;
+        if (c + 8 <= cp.cols) {
+            v = *reinterpret_cast<const s16x8u*>(sp);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = c + e < cols ? (short)sp[e] : (short)0;
-        *reinterpret_cast<s16x8*>(dst + (size_t)r * ldo + c) = v;
+            for (int e = 0; e < 8; ++e) v[e] = c + e < cp.cols ? (short)sp[e] : (short)0;
+        }
+        *reinterpret_cast<s16x8*>(cp.dst + (size_t)r * cp.ldo + c) = v;
     }
 }
 
-// A stored operand (rows x cols, leading dimension ld) copied to pool memory with 16-byte
-// aligned rows (leading dimension cols rounded up to 8, zero-padded).
-uint16_t* aligned_copy(const uint16_t* src, int rows, int cols, int ld, int& ld_out) {
-    ld_out = (cols + 7) & ~7;
-    uint16_t* d = static_cast<uint16_t*>(dh_malloc((size_t)rows * ld_out * sizeof(uint16_t)));
-    if (!d) return nullptr;
-    const long long total = (long long)rows * (ld_out / 8);
-    long long blocks = (total + 255) / 256;
-    if (blocks > 8LL * num_cus()) blocks = 8LL * num_cus();
-    copy_rows_bf16<<<(unsigned)blocks, 256, 0, stream()>>>(src, ld, d, ld_out, rows, cols);
-    if (check_launch("dh_gemm_bf16(aligned copy)") != DH_OK) {
-        dh_free(d);
-        return nullptr;
+// A stored operand (rows x cols, leading dimension ld) to be copied to pool memory with 16-byte
+// aligned rows (leading dimension cols rounded up to 8, zero-padded); dst = null: no memory.
+RowCopy aligned_copy(const uint16_t* src, int rows, int cols, int ld) {
+    const int ldo = (cols + 7) & ~7;
+    return {src, static_cast<uint16_t*>(dh_malloc((size_t)rows * ldo * sizeof(uint16_t))), ld, ldo,
+            rows, cols};
+}
+
+// The copies (one or both operands) in one launch.
+int launch_copies(const RowCopy* c, int n) {
+    long long blocks = 1;
+    for (int i = 0; i < n; ++i) {
+        const long long b = ((long long)c[i].rows * (c[i].ldo / 8) + 255) / 256;
+        blocks = b > blocks ? b : blocks;
     }
-    return d;
+    if (blocks > 8LL * num_cus()) blocks = 8LL * num_cus();
+    copy_rows_bf16<<<dim3((unsigned)blocks, n), 256, 0, stream()>>>(c[0], c[n - 1]);
+    return check_launch("dh_gemm_bf16(aligned copy)");
 }
 
 template <bool TA, bool TB>
@@ -1188,15 +1383,18 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
            float beta, float* C, int ldc, const Batch& bt) {
     // The direct-to-LDS paths need 16-byte operand rows (aligned bases, leading dimensions
     // and batch strides in multiples of 8 elements): 256 x 256 tiles when there are more of
-    // them than half the CUs, else 128 x 128 (DH_GEMM_BF16_MID=0 sends those shapes to the
-    // general kernel instead).  Between half a round and a round the 256 tiles, one per CU
-    // with some CUs idle, still beat four times as many 128 tiles (same box: 3840^3 125 against
-    // 158 us, 3072^3 79 against 99 us; 2048 x 4096, 128 tiles, 45-50 us either way).  Ragged M and N are edge tiles, a K that is not a multiple of
-    // 32 ends with the kernels' masked tail steps (a DMA'd k-contiguous tile would read the
-    // next row's values, possibly non-finite, past K); rows that are not 16-byte aligned are
-    // copied to aligned ones first (one product, and for the 128 x 128 path one of at least
-    // 2^22 multiply-adds: a pass over the operand and a launch, where the general kernel on
-    // such rows takes ~5-10x the direct-to-LDS time).
+    // them than half the CUs, else 128 x 128 or 64 x 64 (stage64_tiles; DH_GEMM_BF16_MID=0 sends
+    // those shapes to the general kernel instead).  Between half a round and a round the 256
+    // tiles, one per CU with some CUs idle, still beat four times as many 128 tiles (same box:
+    // 3840^3 125 against 158 us, 3072^3 79 against 99 us; 2048 x 4096, 128 tiles, 45-50 us either
+    // way).
+    // Ragged M and N are edge tiles, a K that is not a multiple of 32 ends with the larger tiles'
+    // masked tail steps (a DMA'd k-contiguous tile would read the next row's values, possibly
+    // non-finite, past K; the 64 x 64 kernel leaves out whole 16-byte chunks, so it takes K in
+    // eights of such an operand).  One product's rows that do not fit this are copied to aligned,
+    // zero-padded ones first, both operands in one launch, unless
+    // K <= 16, one step of the general kernel.  Row-major with odd rows, us, general / copied:
+    // 5 x 7 x 9 5.7 / 8.0, 33 x 65 x 17 10.2 / 8.1, 255^3 22.4 / 7.5, 1 x 1000 x 1001 24.7 / 9.0.
     static const bool mid_on = [] {
         const char* e = std::getenv("DH_GEMM_BF16_MID");   // tuning knob: 0 or 1
         return !e || std::atoi(e) != 0;
@@ -1208,29 +1406,41 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     }();
     const bool mid = tiles <= (mid_max >= 0 ? mid_max : num_cus() / 2);
     const int K32 = K - K % 32;
+    if (K < 1) return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
     const long long a_bytes = 2LL * ((TA ? K : M) + 255) * lda,
                     b_bytes = 2LL * ((TB ? N : K) + 255) * ldb;
-    if (K32 == 0 || (mid && !mid_on) || a_bytes >= (1LL << 32) || b_bytes >= (1LL << 32))
+    const bool stage64 = mid && mid_on && stage64_tiles(M, N, K, bt.count);
+    if ((K32 == 0 && !stage64) || (mid && !mid_on) || a_bytes >= (1LL << 32) || b_bytes >= (1LL << 32))
         return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
-    const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0);
-    const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0);
+    const bool kmul = !stage64 || K % 8 == 0;
+    const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0) && (TA || kmul);
+    const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0) && (!TB || kmul);
     if (!va || !vb) {
-        if (bt.count > 1 || (mid && (long long)M * N * K < (1LL << 22)))
+        if (bt.count > 1 || K <= 16)
             return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
-        int la = lda, lb = ldb;
-        uint16_t* a2 = va ? nullptr : aligned_copy(A, TA ? K : M, TA ? M : K, lda, la);
-        uint16_t* b2 = vb ? nullptr : aligned_copy(B, TB ? N : K, TB ? K : N, ldb, lb);
+        RowCopy c[2];
+        int n = 0;
+        if (!va) c[n++] = aligned_copy(A, TA ? K : M, TA ? M : K, lda);
+        if (!vb) c[n++] = aligned_copy(B, TB ? N : K, TB ? K : N, ldb);
         int st;
-        if ((!va && !a2) || (!vb && !b2))
+        if (!c[0].dst || !c[n - 1].dst) {
             st = launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
-        else
-            st = launch<TA, TB>(M, N, K, a2 ? a2 : A, la, b2 ? b2 : B, lb, beta, C, ldc, bt);
-        if (a2) dh_free(a2);   // pooled: stream order keeps them alive for the queued work
-        if (b2) dh_free(b2);
+        } else {
+            st = launch_copies(c, n);
+            const uint16_t *a = va ? A : c[0].dst, *b = vb ? B : c[n - 1].dst;
+            const int la = va ? lda : c[0].ldo, lb = vb ? ldb : c[n - 1].ldo;
+            if (st == DH_OK)
+                st = stage64 ? launch_stage64<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
+                   : mid     ? launch_mid<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
+                             : launch_fast<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt);
+        }
+        for (int i = 0; i < n; ++i)
+            if (c[i].dst) dh_free(c[i].dst);   // pooled: stream order keeps them alive
         return st;
     }
-    return mid ? launch_mid<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt)
-               : launch_fast<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
+    return stage64 ? launch_stage64<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt)
+         : mid     ? launch_mid<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt)
+                   : launch_fast<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
 }
 
 }  // namespace

@@ -659,6 +659,36 @@ def test_bf16_mid_path_k_tail_keeps_nonfinite_values_in_their_row():
     assert maxrel(got[ok], A64[ok] @ B64) <= 1e-5 * np.sqrt(K)
 
 
+# The 64 x 64 path (at most two tiles per CU on a ring of four stages, up to three on one of three):
+# K of one chunk, one stage, a stage and a chunk, and ends inside a chunk (a k-contiguous operand is
+# then copied); single, edge and exact tiles, 576 and 768 tiles (ring of three), split K whose last
+# chunk is short.  What lies past a row (aligned or odd leading dimensions) is NaN, C's kept.
+@pytest.mark.parametrize("M,N,K", [(64, 64, 8), (65, 63, 40), (1, 1, 17), (128, 200, 72), (70, 130, 64),
+                                   (257, 64, 191), (130, 70, 16), (1536, 1536, 136), (1530, 2040, 333),
+                                   (1537, 2040, 90), (100, 90, 2061), (512, 257, 4104)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("ldpad", [0, 8, 3])
+def test_bf16_64_wide_tiles(M, N, K, ta, tb, ldpad):
+    rng = np.random.default_rng(M + 3 * N + 7 * K + ta + 2 * tb)
+    A = bf16_bits(rng.standard_normal((K, M) if ta else (M, K), dtype=np.float32))
+    B = bf16_bits(rng.standard_normal((N, K) if tb else (K, N), dtype=np.float32))
+    C0 = rng.standard_normal((M, N), dtype=np.float32)
+    beta = 0.0 if ldpad else -0.5
+    bufs = []
+    for X, pad in ((A, np.uint16(0x7FC0)), (B, np.uint16(0x7FC0)), (C0, np.float32(7))):
+        P = np.full((X.shape[0], X.shape[1] + ldpad), pad, X.dtype)
+        P[:, :X.shape[1]] = X
+        bufs.append(hip.DeviceBuffer.from_numpy(P))
+    hip.gemm_bf16(ta, tb, M, N, K, bufs[0], A.shape[1] + ldpad, bufs[1], B.shape[1] + ldpad, beta,
+                  bufs[2], N + ldpad)
+    out = bufs[2].numpy((M, N + ldpad), np.float32)
+    got = out[:, :N]
+    assert (out[:, N:] == 7).all()
+    A64, B64 = bits_to_f32(A).astype(np.float64), bits_to_f32(B).astype(np.float64)
+    ref = (A64.T if ta else A64) @ (B64.T if tb else B64) + beta * C0
+    assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)      # exact bf16 products, fp32 sums
+
+
 # Between half a round and a round of 256 x 256 tiles the fast kernel runs a partial round
 # (144, 224 and 225 tiles here), at the boundary (128 tiles) the 128 x 128 path.
 @pytest.mark.parametrize("M,N,K", [(3000, 3000, 300), (3500, 4000, 96), (3840, 3840, 33),
