@@ -639,77 +639,101 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
 struct ConvGeom {
     int Cin, H, W, KH, KW, padh, padw, stride, OH, OW;
     FastDiv f_ow, f_kw, f_khkw;   // division by OW, KW and KH*KW
+    FastDiv f_nc;                 // ConvTapSlice: division by its slices per tap
 };
 
-// B slice of the implicit GEMM: rows k0 .. k0 + BK of col_n, columns t0 .. t0 + TILE, laid out
-// like Slice<false, ...> (row k, 4 consecutive columns per chunk).  A thread's chunks all sit
-// in the same 4 columns (tq = tid % (TILE / 4)) and in rows RSTEP apart, so the columns'
-// window origins are computed once per tile and a slice only decomposes its rows.  Every
-// element is one 32-bit-offset buffer load of the image's planes: byte offset = 4 (tap term
-// of its row + pixel term of its column); a tap outside the input takes an offset past the
-// buffer's range, which reads zero.
+// B slice of the implicit GEMM: rows k0 .. k0 + BK of col_n, columns t0 .. t0 + TILE.  A wave's
+// lanes take consecutive columns of one row, so a row's decomposition into (ci, kh, kw) is
+// wave-uniform and runs on the scalar unit, and a thread keeps one column, whose window origin
+// is computed once per tile.  What is left per element for the vector unit, which shares the
+// SIMD's issue with the MFMAs, are two sums, two compares and the offset.  Every element is one
+// 32-bit-offset buffer load of the image's planes: byte offset = 4 (tap term of its row + pixel
+// term of its column); a tap outside the input takes an offset past the buffer's range, which
+// reads zero.
 constexpr uint32_t CONV_OOB = 0xFFFFFFF0u;   // past every image buffer (entries check the size)
 
 template <int TILE>
 struct ConvSlice {
-    static constexpr int CH = TILE * BK / 4 / NTHREADS;
-    static constexpr int RSTEP = NTHREADS / (TILE / 4);
-    f32x4 v[CH];
-    int hb[4], wb[4];   // oh * stride - pad, ow * stride - pad of the thread's 4 columns
-    int pix[4];         // 4 (hb W + wb): the column's part of the byte offset
+    static constexpr int CH = TILE * BK / NTHREADS;
+    static constexpr int RSTEP = NTHREADS / TILE;
+    static_assert(TILE % 64 == 0, "a wave's lanes share a row");
+    float v[CH];
+    int hb, wb;   // oh * stride - pad, ow * stride - pad of the thread's column
+    int pix;      // 4 (hb W + wb): the column's part of the byte offset
+    int row;      // the wave's first row of a slice
 
     __device__ void init(const ConvGeom& g, int t0, int P, int tid) {
-        const int tq = tid % (TILE / 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int p = t0 + 4 * tq + e;
-            const int oh = (int)fdiv((uint32_t)p, g.f_ow), ow = p - oh * g.OW;
-            const int h0 = oh * g.stride - g.padh;
-            wb[e] = ow * g.stride - g.padw;
-            pix[e] = 4 * (h0 * g.W + wb[e]);
-            hb[e] = p < P ? h0 : -(1 << 30);   // a column past P: h < 0
-        }
+        const int p = t0 + tid % TILE;
+        const int oh = (int)fdiv((uint32_t)p, g.f_ow), ow = p - oh * g.OW;
+        const int h0 = oh * g.stride - g.padh;
+        wb = ow * g.stride - g.padw;
+        pix = 4 * (h0 * g.W + wb);
+        hb = p < P ? h0 : -(1 << 30);   // a column past P: h < 0
+        row = __builtin_amdgcn_readfirstlane(tid / TILE);
     }
-    __device__ void fetch(__amdgpu_buffer_rsrc_t rs, const ConvGeom& g, int R, int k0, int tid) {
+    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int R, int k0) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(X), 0, (int)(4u * g.Cin * g.H * g.W), 0x00020000);
 #pragma unroll
         for (int r = 0; r < CH; ++r) {
-            const int k = k0 + tid / (TILE / 4) + RSTEP * r;
+            const int k = k0 + row + RSTEP * r;
             const int q = (int)fdiv((uint32_t)k, g.f_kw), kw = k - q * g.KW;
-            const int ci = (int)fdiv((uint32_t)k, g.f_khkw), kh = q - ci * g.KH;
-            const int tap = 4 * ((ci * g.H + kh) * g.W + kw);
-            const bool kin = k < R;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int h = hb[e] + kh, w = wb[e] + kw;
-                const bool in = kin && (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
-                const uint32_t off = in ? (uint32_t)(tap + pix[e]) : CONV_OOB;
-                v[r][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
-            }
+            const int ci = (int)fdiv((uint32_t)k, g.f_khkw);
+            const int kh = k < R ? q - ci * g.KH : -(1 << 30);   // a row past R: h < 0
+            const int tap = 4 * ((ci * g.H + q - ci * g.KH) * g.W + kw);
+            const bool in = (unsigned)(hb + kh) < (unsigned)g.H && (unsigned)(wb + kw) < (unsigned)g.W;
+            const uint32_t off = in ? (uint32_t)(tap + pix) : CONV_OOB;
+            v[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
         }
     }
     __device__ void store(float* lds, int stride, int tid) const {
 #pragma unroll
-        for (int r = 0; r < CH; ++r) {
-            const int f = tid + r * NTHREADS;
-            *reinterpret_cast<f32x4*>(&lds[(f / (TILE / 4)) * stride + 4 * (f % (TILE / 4))]) = v[r];
+        for (int r = 0; r < CH; ++r) lds[(row + RSTEP * r) * stride + tid % TILE] = v[r];
+    }
+};
+
+// The same slice where the rows of the packed kernel run (kh, kw, ci) with ci padded with zeros
+// to whole slices: a slice is one tap of BK channels, so the window test and the offset inside
+// a plane are computed once per slice for the thread's column, and an element costs one load
+// through a buffer over its own plane (empty past Cin), whose base the scalar unit adds.
+template <int TILE>
+struct ConvTapSlice : ConvSlice<TILE> {
+    using Base = ConvSlice<TILE>;
+    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int R, int k0) {
+        const int t = (int)fdiv((uint32_t)k0 / BK, g.f_nc);
+        const int kq = (int)fdiv((uint32_t)t, g.f_kw), kw = t - kq * g.KW;
+        const int c0 = k0 - t * ((int)g.f_nc.d * BK) + Base::row;
+        const int kh = k0 < R ? kq : -(1 << 30);   // a slice past R: h < 0
+        const bool in = (unsigned)(Base::hb + kh) < (unsigned)g.H &&
+                        (unsigned)(Base::wb + kw) < (unsigned)g.W;
+        const uint32_t off = in ? (uint32_t)(Base::pix + 4 * (kq * g.W + kw)) : CONV_OOB;
+        const int plane = g.H * g.W;
+        const float* xp = X + (size_t)c0 * plane;
+#pragma unroll
+        for (int r = 0; r < Base::CH; ++r) {
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(xp + (size_t)(Base::RSTEP * r) * plane), 0,
+                c0 + Base::RSTEP * r < g.Cin ? 4 * plane : 0, 0x00020000);
+            Base::v[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
         }
     }
 };
 
 // Work-group tile TBM (output channels) x TBN (output positions of image z0 + blockIdx.y);
-// the k-loop is the GEMM kernel's (two register sets, branch-free), A = the kernel matrix
+// the k-loop is the GEMM kernel's (two register sets, branch-free) over kz slices, those of chunk
+// blockIdx.z (one chunk, or partial results that conv_split_reduce adds), A = the kernel matrix
 // Cout x R (k contiguous), epilogue: + bias[co] (+ the old Y with accumulate), stored into
 // Y's (N, Cout, OH OW) layout.
-template <int TBM, int TBN, bool VA>
+template <int TBM, int TBN, int VA, bool TAP>
 __global__ void __launch_bounds__(NTHREADS)
 conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const float* __restrict__ X,
                 ConvGeom g, float* __restrict__ Y, const float* __restrict__ bias, int z0,
-                int accumulate) {
+                int accumulate, int kz) {
     const int n = z0 + blockIdx.y;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(X) + (size_t)n * g.Cin * g.H * g.W, 0, (int)(4u * g.Cin * g.H * g.W),
-        0x00020000);
-    float* Yn = Y + (size_t)n * Cout * P;
+    X += (size_t)n * g.Cin * g.H * g.W;
+    float* Yn = Y + ((size_t)blockIdx.z * gridDim.y + n) * Cout * P;
+    const int kb = blockIdx.z * kz * BK;   // this chunk's rows: kb .. Re
+    const int Re = min(R, kb + kz * BK);
     constexpr int LDS_A = TBM + 4, LDS_B = TBN + 4;
     constexpr int WT = TBM == 64 && TBN == 64 ? 32 : 64, NB = WT / 32;   // wave sub-tile
     constexpr int WN = TBN / WT;
@@ -725,8 +749,8 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     const int l32 = lane & 31, h = lane >> 5;
     const int wm = (wave / WN) * WT, wn = (wave % WN) * WT;
 
-    Slice<true, VA ? LD_VEC : LD_SCALAR, TBM> sa[2];
-    ConvSlice<TBN> sb[2];
+    Slice<true, VA, TBM> sa[2];
+    std::conditional_t<TAP, ConvTapSlice<TBN>, ConvSlice<TBN>> sb[2];
     sb[0].init(g, n0, P, tid);
     sb[1].init(g, n0, P, tid);
 
@@ -738,11 +762,11 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
-    const int nk = (R + BK - 1) / BK;   // R >= 1
-    sa[0].fetch(Kn, R, m0, 0, Cout, R, tid);
-    sb[0].fetch(xr, g, R, 0, tid);
-    sa[1].fetch(Kn, R, m0, BK, Cout, R, tid);
-    sb[1].fetch(xr, g, R, BK, tid);
+    const int nk = (Re - kb + BK - 1) / BK;   // >= 1
+    sa[0].fetch(Kn, R, m0, kb, Cout, Re, tid);
+    sb[0].fetch(X, g, Re, kb);
+    sa[1].fetch(Kn, R, m0, kb + BK, Cout, Re, tid);
+    sb[1].fetch(X, g, Re, kb + BK);
     sa[0].store(As[0], LDS_A, tid);
     sb[0].store(Bs[0], LDS_B, tid);
     __syncthreads();
@@ -764,8 +788,8 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     };
     auto step = [&](auto cur_c, int kt) {
         constexpr int cur = decltype(cur_c)::value;
-        sa[cur].fetch(Kn, R, m0, (kt + 2) * BK, Cout, R, tid);
-        sb[cur].fetch(xr, g, R, (kt + 2) * BK, tid);
+        sa[cur].fetch(Kn, R, m0, kb + (kt + 2) * BK, Cout, Re, tid);
+        sb[cur].fetch(X, g, Re, kb + (kt + 2) * BK);
         mma(As[cur], Bs[cur]);
         sa[cur ^ 1].store(As[cur ^ 1], LDS_A, tid);
         sb[cur ^ 1].store(Bs[cur ^ 1], LDS_B, tid);
@@ -797,17 +821,42 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
         }
 }
 
+// Y (+)= sum_s part[s] + bias over n = N Cout P values, in a fixed order, four loads in flight.
+__global__ void __launch_bounds__(256) conv_split_reduce(const float* __restrict__ part, int S,
+                                                         uint32_t n, uint32_t P, uint32_t Cout,
+                                                         const float* __restrict__ bias,
+                                                         float* __restrict__ Y, int accumulate) {
+    for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+        float v = 0.f;
+        int q = 0;
+        for (; q + 4 <= S; q += 4) {
+            float x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = part[(size_t)(q + u) * n + e];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v += x[u];
+        }
+        for (; q < S; ++q) v += part[(size_t)q * n + e];
+        if (bias) v += bias[e / P % Cout];
+        Y[e] = accumulate ? Y[e] + v : v;
+    }
+}
+
 template <int TBM, int TBN>
 int launch_conv(int N, int Cout, int P, int R, const float* Kn, const float* X,
-                const ConvGeom& g, float* Y, const float* bias, int accumulate) {
-    const bool va = ((uintptr_t)Kn % 16 == 0) && (R % 4 == 0);
+                const ConvGeom& g, float* Y, const float* bias, int accumulate, bool taps, int S) {
+    // kernel rows of any alignment by 16-byte buffer loads; longer than 32-bit offsets reach:
+    // element by element
+    auto kern = taps             ? conv_fwd_kernel<TBM, TBN, LD_BUF4, true>
+              : R > LD_BUF_MAX   ? conv_fwd_kernel<TBM, TBN, LD_SCALAR, false>
+              : R % 4 == 0       ? conv_fwd_kernel<TBM, TBN, LD_BUF4, false>
+                                 : conv_fwd_kernel<TBM, TBN, LD_BUF, false>;
     const int tiles = ((Cout + TBM - 1) / TBM) * ((P + TBN - 1) / TBN);
+    const int nk = (R + BK - 1) / BK, kz = (nk + S - 1) / S;
     for (int z0 = 0; z0 < N; z0 += 65535) {
-        const dim3 grid(tiles, N - z0 < 65535 ? N - z0 : 65535);
-        if (va)
-            conv_fwd_kernel<TBM, TBN, true><<<grid, NTHREADS, 0, stream()>>>(Cout, P, R, Kn, X, g, Y, bias, z0, accumulate);
-        else
-            conv_fwd_kernel<TBM, TBN, false><<<grid, NTHREADS, 0, stream()>>>(Cout, P, R, Kn, X, g, Y, bias, z0, accumulate);
+        const dim3 grid(tiles, N - z0 < 65535 ? N - z0 : 65535,
+                        (nk + kz - 1) / kz);
+        kern<<<grid, NTHREADS, 0, stream()>>>(Cout, P, R, Kn, X, g, Y, bias, z0, accumulate, kz);
         DH_TRY(check_launch("dh_conv2d"));
     }
     return DH_OK;
@@ -854,17 +903,16 @@ __global__ void __launch_bounds__(256) splitk_reduce(const float* __restrict__ p
 // into chunks, one per gridDim.y member, each writing an fp32 partial that splitk_reduce adds
 // in a fixed order.
 
-// The thread's rows of B (kernel taps r): chunk c covers tap t0 + f / (BK / 4), f = tid +
-// c NTHREADS, at output positions p0 + 4 (f % (BK / 4)) + (0..3) -- its tap and hence the
-// input plane and window offset stay fixed across slices.
+// The thread's rows of B (kernel taps r): t0 + tid / BK + RSTEP c, at position tid % BK of a
+// slice -- its taps and hence their input planes and window offsets stay fixed across slices.
 template <int TILE>
 struct ColTGeom {
-    static constexpr int CH = TILE * BK / 4 / NTHREADS;
+    static constexpr int CH = TILE * BK / NTHREADS, RSTEP = NTHREADS / BK;
     int tap[CH], dh[CH], dw[CH];    // 4 (ci H W + dh W + dw); kh - padh (-2^30 past R); kw - padw
     __device__ void init(const ConvGeom& g, int R, int t0, int tid) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const int r = t0 + (tid + c * NTHREADS) / (BK / 4);
+            const int r = t0 + tid / BK + RSTEP * c;
             const int q = (int)fdiv((uint32_t)r, g.f_kw), kw = r - q * g.KW;
             const int ci = (int)fdiv((uint32_t)r, g.f_khkw), kh = q - ci * g.KH;
             dw[c] = kw - g.padw;
@@ -874,48 +922,41 @@ struct ColTGeom {
     }
 };
 
-// A thread's chunks share their 4 positions (f % (BK / 4) = tid % (BK / 4)), so a slice
-// decomposes them once; each element is then one 32-bit-offset buffer load (tap term + pixel
-// term; taps outside the input read zero through an offset past the buffer).
+// A thread's elements of a slice share one position, which is decomposed once (with four
+// positions per thread those divisions took much of the vector unit's time: the bench layer's
+// gradient 185 -> 158-165 us); each element is
+// then one 32-bit-offset buffer load (tap term + pixel term; taps outside the input read zero
+// through an offset past the buffer).  16 lanes read consecutive positions of one tap, and a
+// wave's LDS stores (16 k-rows 4 banks apart, 4 taps) fall on distinct banks.
 template <int TILE>
 struct ColTSlice {
-    static constexpr int CH = TILE * BK / 4 / NTHREADS;
-    f32x4 v[CH];
+    static constexpr int CH = ColTGeom<TILE>::CH, RSTEP = ColTGeom<TILE>::RSTEP;
+    float v[CH];
     // positions p0 .. p0 + BK of the image behind rs; np = number of valid positions (0: zeros)
     __device__ void fetch(__amdgpu_buffer_rsrc_t rs, const ConvGeom& g, const ColTGeom<TILE>& c,
                           int p0, int np, int tid) {
-        const int pq = 4 * (tid % (BK / 4));
+        const int p = p0 + tid % BK;
+        const int oh = (int)fdiv((uint32_t)p, g.f_ow), ow = p - oh * g.OW;
+        const int hs = tid % BK < np ? oh * g.stride : -(1 << 30), ws = ow * g.stride;
+        const int pix = 4 * (oh * g.stride * g.W + ws);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int p = p0 + pq + e;
-            const int oh = (int)fdiv((uint32_t)p, g.f_ow), ow = p - oh * g.OW;
-            const int hs = oh * g.stride, ws = ow * g.stride;
-            const int pix = 4 * (hs * g.W + ws);
-            const bool pin = pq + e < np;
-#pragma unroll
-            for (int k = 0; k < CH; ++k) {
-                const int h = hs + c.dh[k], w = ws + c.dw[k];
-                const bool in = pin && (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
-                const uint32_t off = in ? (uint32_t)(c.tap[k] + pix) : CONV_OOB;
-                v[k][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
-            }
+        for (int k = 0; k < CH; ++k) {
+            const bool in = (unsigned)(hs + c.dh[k]) < (unsigned)g.H &&
+                            (unsigned)(ws + c.dw[k]) < (unsigned)g.W;
+            const uint32_t off = in ? (uint32_t)(c.tap[k] + pix) : CONV_OOB;
+            v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
         }
     }
     __device__ void store(float* lds, int stride, int tid) const {   // transposing, as Slice<true>
 #pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int f = tid + k * NTHREADS;
-            const int t = f / (BK / 4), kq = f % (BK / 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) lds[(4 * kq + e) * stride + t] = v[k][e];
-        }
+        for (int k = 0; k < CH; ++k) lds[(tid % BK) * stride + tid / BK + RSTEP * k] = v[k];
     }
 };
 
 // Work-group: tile TBM (output channels) x TBN (taps) of chunk blockIdx.y, i.e. the slices
 // [y chunk, min((y + 1) chunk, total)) of the flattened (image, slice) contraction, nkp
 // slices per image.  Writes its partial to part + y Cout R.
-template <int TBM, int TBN, bool VA>
+template <int TBM, int TBN, int VA>
 __global__ void __launch_bounds__(NTHREADS)
 conv_wgrad_kernel(int Cout, int P, int R, const float* __restrict__ dY, const float* __restrict__ X,
                   ConvGeom g, int nkp, int total, int chunk, float* __restrict__ part) {
@@ -940,16 +981,18 @@ conv_wgrad_kernel(int Cout, int P, int R, const float* __restrict__ dY, const fl
 
     ColTGeom<TBN> cg;
     cg.init(g, R, n0, tid);
-    Slice<true, VA ? LD_VEC : LD_SCALAR, TBM> sa[2];
+    Slice<true, VA, TBM> sa[2];
     ColTSlice<TBN> sb[2];
-    // slice kt of the chunk: image n, positions p0 ..; past the chunk's end: zeros
+    // slice kt of the chunk, in order: image n, positions p0 ..; past the chunk's end: zeros
+    int nw = sbeg / nkp, pw = (sbeg - nw * nkp) * BK;
     auto fetch = [&](auto set_c, int kt) {
         constexpr int set = decltype(set_c)::value;
-        const int s = sbeg + kt;
         const bool live = kt < ns;
-        const int n = live ? s / nkp : 0;
-        const int p0 = live ? (s - n * nkp) * BK : 0;
+        const int n = live ? nw : 0, p0 = live ? pw : 0;
         const int np = live ? min(BK, P - p0) : 0;
+        const bool wrap = pw + BK >= P;
+        pw = wrap ? 0 : pw + BK;
+        nw += wrap;
         sa[set].fetch(dY + (size_t)n * Cout * P, P, m0, p0, Cout, live ? P : 0, tid);
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float*>(X) + (size_t)n * plane, 0, (int)(4 * plane), 0x00020000);
@@ -1018,7 +1061,7 @@ conv_wgrad_kernel(int Cout, int P, int R, const float* __restrict__ dY, const fl
 // out = beta out + sum_s part[s] for many partials: wave w of a work-group sums partials
 // [w S / 4, (w + 1) S / 4) of 64 consecutive elements, then wave 0 adds the four sums in
 // order (fixed order: bit-identical reruns), so four times as many waves share the loads as
-// in splitk_reduce's one thread per element.
+// in splitk_reduce's one thread per element; 8 loads in flight per thread, added in order.
 __global__ void __launch_bounds__(256) partial_sum4(const float* __restrict__ part, int S,
                                                     size_t n, float beta, float* __restrict__ out) {
     __shared__ float red[3][64];
@@ -1027,8 +1070,17 @@ __global__ void __launch_bounds__(256) partial_sum4(const float* __restrict__ pa
     for (size_t e0 = (size_t)blockIdx.x * 64; e0 < n; e0 += (size_t)gridDim.x * 64) {
         const size_t e = e0 + lane;
         float v = 0.f;
-        if (e < n)
-            for (int q = sb; q < se; ++q) v += part[(size_t)q * n + e];
+        if (e < n) {
+            int q = sb;
+            for (; q + 8 <= se; q += 8) {
+                float x[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) x[u] = part[(size_t)(q + u) * n + e];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v += x[u];
+            }
+            for (; q < se; ++q) v += part[(size_t)q * n + e];
+        }
         if (w > 0) red[w - 1][lane] = v;
         __syncthreads();
         if (w == 0 && e < n) {
@@ -1059,13 +1111,12 @@ int launch_wgrad(int N, int Cout, int P, int R, const float* dY, const float* X,
     S = (total + chunk - 1) / chunk;
     float* part = static_cast<float*>(dh_malloc((size_t)S * Cout * R * sizeof(float)));
     if (!part) return set_error(DH_ERR_OOM, "dh_conv2d_bwd_filter: partials");
-    const bool va = ((uintptr_t)dY % 16 == 0) && (P % 4 == 0);
+    auto kern = P > LD_BUF_MAX ? conv_wgrad_kernel<TBM, TBN, LD_SCALAR>
+              : P % 4 == 0     ? conv_wgrad_kernel<TBM, TBN, LD_BUF4>
+                               : conv_wgrad_kernel<TBM, TBN, LD_BUF>;
     const dim3 grid(tiles, (unsigned)S);
     hipStream_t s = stream();
-    if (va)
-        conv_wgrad_kernel<TBM, TBN, true><<<grid, NTHREADS, 0, s>>>(Cout, P, R, dY, X, g, nkp, (int)total, (int)chunk, part);
-    else
-        conv_wgrad_kernel<TBM, TBN, false><<<grid, NTHREADS, 0, s>>>(Cout, P, R, dY, X, g, nkp, (int)total, (int)chunk, part);
+    kern<<<grid, NTHREADS, 0, s>>>(Cout, P, R, dY, X, g, nkp, (int)total, (int)chunk, part);
     int st = check_launch("dh_conv2d_bwd_filter");
     if (st == DH_OK) {
         const size_t n = (size_t)Cout * R;
@@ -1526,18 +1577,19 @@ int launch(int M, int N, int K, const float* A, int lda, const float* B, int ldb
     return launch_tiles<TA, TB, 128, 128>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
 }
 
-// Tile choice and launch shared by the forward and the data gradient: 64 x 64 tiles for few
-// output channels (the bench layer: 0.271 -> 0.212 ms against 64 x 256 tiles -- 3136
-// work-groups at 8 waves per SIMD instead of 832 at 2) and for small grids; 128 x 128
-// otherwise.
-int run_conv(int N, int Cout, long long P, long long R, const float* Kn, const float* X,
-             const ConvGeom& g, float* Y, const float* bias, int accumulate) {
-    const int cus = num_cus();
-    const long long t128 = (long long)((Cout + 127) / 128) * ((P + 127) / 128) * N;
-    const long long t64 = (long long)((Cout + 63) / 64) * ((P + 63) / 64) * N;
-    if (Cout <= 64 || (t128 < cus && 2 * t64 > cus))
-        return launch_conv<64, 64>(N, Cout, (int)P, (int)R, Kn, X, g, Y, bias, accumulate);
-    return launch_conv<128, 128>(N, Cout, (int)P, (int)R, Kn, X, g, Y, bias, accumulate);
+// Kt[a][t][b] = the kernel of output channel a, tap t and input channel b < B, zero for B <= b <
+// BP.  FLIP is the data gradient's kernel: channels swapped, window flipped.
+template <bool FLIP>
+__global__ void __launch_bounds__(256) conv_pack_kernel(const float* __restrict__ Kn,
+                                                        float* __restrict__ Kt, int A, int B,
+                                                        int BP, int win) {
+    const uint32_t n = (uint32_t)A * BP * win;   // at most 2^30, see run_conv
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const uint32_t b = i % BP, at = i / BP, a = at / win, t = at % win;
+        const size_t src = FLIP ? ((size_t)b * A + a) * win + (win - 1 - t)
+                                : ((size_t)a * B + b) * win + t;
+        Kt[i] = b < (uint32_t)B ? Kn[src] : 0.f;
+    }
 }
 
 // Kt[ci][(co KH + kh) KW + kw] = Kn[co][(ci KH + KH-1-kh) KW + KW-1-kw]: the kernel of the
@@ -1552,6 +1604,84 @@ __global__ void __launch_bounds__(256) conv_flip_kernel(const float* __restrict_
         const int kh = (int)(t / KW), kw = (int)(t % KW);
         Kt[i] = Kn[co * Cin * win + (ci * KH + KH - 1 - kh) * KW + KW - 1 - kw];
     }
+}
+
+unsigned stride_blocks(size_t n) {
+    const size_t blocks = (n + 255) / 256, most = (size_t)num_cus() * 8;
+    return (unsigned)(blocks < most ? blocks : most);
+}
+
+// Tile choice and launch shared by the forward and the data gradient (flip: of a Cout x Cin
+// kernel, here read as Cin x Cout): 64 x 64 tiles for few output channels (the bench layer:
+// 0.271 -> 0.212 ms against 64 x 256 tiles -- 3136 work-groups at 8 waves per SIMD instead of
+// 832 at 2) and for grids of less than one 128 x 128 tile per CU; 128 x 128 otherwise.  At most
+// one 64 x 64 tile for two CUs also splits R into chunks of at least 8 slices, up to two
+// work-groups per CU: a work-group's slices are a serial chain (4 images 256 x 14 x 14 -> 256, 3 x 3:
+// 222 us on 16 work-groups of 128-wide tiles, 26 us split in 8; 2 images 64 x 14 x 14 -> 64: 23.4 /
+// 12.9).  From there to one tile per CU the second launch costs more than it gives (16 images
+// 32 x 28 x 28 -> 64: 14.0 us whole, 19.3 in halves).
+//
+// The kernel is packed to (kh, kw, ci) order where the channels padded to whole slices add at
+// most an eighth of the work and the product is long enough to pay for the 3 to 5 us of the
+// packing launch (the data gradient has a launch for its flip anyway).  Forward, us, packed / as
+// stored: 0.46 GFLOP 19.3 / 19.5, 0.92 24.1 / 25.8 and 26.0 / 25.2, 1.85 30.4 / 35.4, 3.7 48.1 / 57.1 and
+// 53.3 / 64.5, 64 images 64 x 56 x 56 -> 64 (14.8) 146 / 169 (184 with vector-unit row
+// decomposition).
+constexpr double CONV_PACK_FLOPS = 1e9;
+
+int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, ConvGeom g, float* Y,
+             const float* bias, int accumulate, bool flip) {
+    const int cus = num_cus(), win = g.KH * g.KW;
+    long long R = (long long)g.Cin * win;
+    const int cp = (g.Cin + BK - 1) / BK * BK;
+    bool taps = 8ll * (cp - g.Cin) <= g.Cin && (long long)win * cp <= LD_BUF_MAX &&
+                (long long)Cout * win * cp <= 1ll << 30 &&
+                (flip || 2.0 * N * Cout * P * R >= CONV_PACK_FLOPS);
+    float* Kt = nullptr;
+    if (taps || flip) {
+        Kt = static_cast<float*>(dh_malloc((size_t)Cout * (taps ? (long long)win * cp : R) * sizeof(float)));
+        if (!Kt && flip) return set_error(DH_ERR_OOM, "dh_conv2d_bwd_data: flipped kernel");
+        if (!Kt) {   // the forward runs without scratch too
+            taps = false;
+            (void)hipGetLastError();
+        }
+    }
+    if (taps) {
+        R = (long long)win * cp;
+        g.f_nc = make_fastdiv((uint32_t)(cp / BK));
+        (flip ? conv_pack_kernel<true> : conv_pack_kernel<false>)
+            <<<stride_blocks((size_t)Cout * R), 256, 0, stream()>>>(Kn, Kt, Cout, g.Cin, cp, win);
+    } else if (flip) {
+        conv_flip_kernel<<<stride_blocks((size_t)Cout * R), 256, 0, stream()>>>(Kn, Kt, g.Cin, Cout, g.KH, g.KW);
+    }
+    const long long t128 = (long long)((Cout + 127) / 128) * ((P + 127) / 128) * N;
+    const long long t64 = (long long)((Cout + 63) / 64) * ((P + 63) / 64) * N;
+    int S = 1;
+    float* part = nullptr;
+    const size_t n = (size_t)N * Cout * P;
+    if (2 * t64 <= cus && R >= 16 * BK) {
+        S = (int)std::min<long long>(2 * cus / t64, R / (8 * BK));
+        const int nk = (int)((R + BK - 1) / BK), kz = (nk + S - 1) / S;
+        S = (nk + kz - 1) / kz;   // no empty chunks
+        if (S > 1) part = static_cast<float*>(dh_malloc(S * n * sizeof(float)));   // < 9 MB
+        if (!part) {
+            S = 1;
+            (void)hipGetLastError();
+        }
+    }
+    int st = Kt ? check_launch("dh_conv2d(kernel)") : DH_OK;
+    if (st == DH_OK)
+        st = (Cout <= 64 || t128 < cus ? launch_conv<64, 64> : launch_conv<128, 128>)(
+            N, Cout, (int)P, (int)R, Kt ? Kt : Kn, X, g, part ? part : Y, part ? nullptr : bias,
+            part ? 0 : accumulate, taps, S);
+    if (st == DH_OK && part) {
+        conv_split_reduce<<<stride_blocks(n), 256, 0, stream()>>>(part, S, (uint32_t)n, (uint32_t)P,
+                                                                  (uint32_t)Cout, bias, Y, accumulate);
+        st = check_launch("dh_conv2d(reduce)");
+    }
+    dh_free(part);
+    dh_free(Kt);   // pooled; later users of the buffer are ordered on the stream
+    return st;
 }
 
 }  // namespace
@@ -1639,7 +1769,7 @@ extern "C" int dh_conv2d_fwd(const float* X, const float* Kn, const float* bias,
         return set_error(DH_ERR_UNSUPPORTED, "dh_conv2d_fwd: plane or window too large");
     ConvGeom g{Cin, H, W, KH, KW, pad, pad, stride, OH, OW, make_fastdiv((uint32_t)OW),
                make_fastdiv((uint32_t)KW), make_fastdiv((uint32_t)(KH * KW))};
-    return run_conv(N, Cout, P, R, Kn, X, g, Y, bias, 0);
+    return run_conv(N, Cout, P, Kn, X, g, Y, bias, 0, false);
 }
 
 // dX (+)= the input gradient of a stride-1 convolution: for stride 1, col2im(K^T dY) is the
@@ -1666,21 +1796,10 @@ extern "C" int dh_conv2d_bwd_data(const float* dY, const float* Kn, float* dX, i
     if (P >= (1ll << 30) || R >= (1ll << 30) || (long long)OH * OW >= (1ll << 30) ||
         (long long)Cin * P >= (1ll << 31) || 4ll * Cout * OH * OW >= (long long)CONV_OOB)
         return set_error(DH_ERR_UNSUPPORTED, "dh_conv2d_bwd_data: plane or window too large");
-    float* Kt = static_cast<float*>(dh_malloc((size_t)Cin * R * sizeof(float)));
-    if (!Kt) return set_error(DH_ERR_OOM, "dh_conv2d_bwd_data: flipped kernel");
-    const size_t nk = (size_t)Cin * R;
-    size_t blocks = (nk + 255) / 256;
-    if (blocks > (size_t)num_cus() * 8) blocks = (size_t)num_cus() * 8;
-    conv_flip_kernel<<<(unsigned)blocks, 256, 0, stream()>>>(Kn, Kt, Cout, Cin, KH, KW);
-    int st = check_launch("dh_conv2d_bwd_data(flip)");
-    if (st == DH_OK) {
-        ConvGeom g{Cout, OH, OW, KH, KW, KH - 1 - pad, KW - 1 - pad, 1, H, W,
-                   make_fastdiv((uint32_t)W), make_fastdiv((uint32_t)KW),
-                   make_fastdiv((uint32_t)(KH * KW))};
-        st = run_conv(N, Cin, P, R, Kt, dY, g, dX, nullptr, accumulate ? 1 : 0);
-    }
-    dh_free(Kt);   // pooled; later users of the buffer are ordered on the stream
-    return st;
+    ConvGeom g{Cout, OH, OW, KH, KW, KH - 1 - pad, KW - 1 - pad, 1, H, W,
+               make_fastdiv((uint32_t)W), make_fastdiv((uint32_t)KW),
+               make_fastdiv((uint32_t)(KH * KW))};
+    return run_conv(N, Cin, P, Kn, dY, g, dX, nullptr, accumulate ? 1 : 0, true);
 }
 
 // gK (+)= the kernel gradient of a convolution, any pad and stride: sum over images of

@@ -106,6 +106,39 @@ def test_conv2d_fwd_implicit_gemm_against_oracle(shape):
             t.free()
 
 
+@pytest.mark.parametrize("shape", [
+    (20, 30, 47, 45, 70, 3, 3, 1, 1),   # packed kernel, 2 zero channels per tap, 128 x 128 tiles
+    (16, 48, 41, 39, 40, 3, 5, 2, 1),   # packed, 64 x 64 tiles, KH != KW, P no multiple of 4
+    (9, 160, 31, 29, 96, 3, 3, 1, 2),   # packed and strided, R split over work-groups
+    (2, 37, 13, 14, 33, 3, 3, 1, 2),    # stored order, R = 333 split in chunks, the last ragged
+    (1, 256, 1, 1, 5, 1, 1, 0, 1),      # one position; two chunks of 8 slices
+])
+def test_conv2d_packed_and_split_against_oracle(shape):
+    # The packed tap order and the split contraction, forward and (stride 1) data gradient:
+    # the same bound as the plain forms above, rounding of a sum of Cin KH KW fp32 products.
+    N, Cin, H, W, Cout, KH, KW, pad, stride = shape
+    OH, OW = O.conv_out(H, W, KH, KW, pad, stride)
+    rng = np.random.default_rng(sum(shape) + 3)
+    X = rng.standard_normal((N, Cin * H * W)).astype(np.float32)
+    Kn = rng.standard_normal((Cout, Cin * KH * KW)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    G = rng.standard_normal((N, Cout * OH * OW)).astype(np.float32)
+    dX, dK, db, dG = (DB.from_numpy(a) for a in (X, Kn, b, G))
+    dY, gX = DB.empty((N, Cout * OH * OW), np.float32), DB.empty((N, Cin * H * W), np.float32)
+    X, Kn, b, G = (a.astype(np.float64) for a in (X, Kn, b, G))
+    try:
+        hip.conv2d_fwd(dX, dK, db, dY, N, Cin, H, W, Cout, KH, KW, pad, stride)
+        ref = O.conv2d(X, Kn, b, N, Cin, H, W, Cout, KH, KW, pad, stride)
+        assert maxrel(dY.numpy(), ref) <= 1e-5 * np.sqrt(Cin * KH * KW)
+        if stride == 1 and pad < min(KH, KW):
+            hip.conv2d_bwd_data(dG, dK, gX, N, Cin, H, W, Cout, KH, KW, pad, 1)
+            rX, _ = O.conv2d_bwd(X, Kn, G, N, Cin, H, W, Cout, KH, KW, pad, 1)
+            assert maxrel(gX.numpy(), rX) <= 1e-5 * np.sqrt(Cout * KH * KW)
+    finally:
+        for t in (dX, dK, db, dG, dY, gX):
+            t.free()
+
+
 def test_conv2d_fwd_rejects_bad_shapes():
     d = DB.empty((64,), np.float32)
     try:
