@@ -573,9 +573,9 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
     float* lb = la + SZ;
     WaveSlice<!TA> sa[2];
     WaveSlice<TB> sb[2];
-    f32x16 acc;
+    f32x16 acc[2];   // of even and odd slices: chains of half the length round less
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
     const int nk = (K + WV_BK - 1) / WV_BK;
     auto fetch = [&](auto set_c, int i) {   // the wave's slice i (past K: zeros)
         constexpr int set = decltype(set_c)::value;
@@ -596,7 +596,7 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
         for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], acc, 0, 0, 0);
+                acc[set] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], acc[set], 0, 0, 0);
     };
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
@@ -611,7 +611,7 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
     }
     // partial tiles, lane-major, in the waves' own LDS
 #pragma unroll
-    for (int r = 0; r < 16; ++r) la[r * 64 + lane] = acc[r];
+    for (int r = 0; r < 16; ++r) la[r * 64 + lane] = acc[0][r] + acc[1][r];
     __syncthreads();
     const bool row_bias = bias && (epi & DH_EPI_ROW_BIAS), relu = epi & DH_EPI_RELU;
 #pragma unroll
