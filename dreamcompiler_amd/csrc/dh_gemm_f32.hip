@@ -583,14 +583,23 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
         sa[set].fetch(A, lda, m0, k0, M, K, lane);
         sb[set].fetch(B, ldb, n0, k0, N, K, lane);
     };
+    // A wave's LDS accesses run in program order, and the lanes read what other lanes stored:
+    // the compiler must keep that order too (no instruction comes of this).
+    auto wave_fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     auto step = [&](auto set_c, int i) {
         constexpr int set = decltype(set_c)::value;
-        sa[set].store(la, lane);   // behind the last slice's reads: a wave's LDS accesses are in order
+        sa[set].store(la, lane);
         sb[set].store(lb, lane);
+        wave_fence();
         fetch(set_c, i + 2);
         float a[4][4], b[4][4];
         WaveSlice<!TA>::read(la, l32, h, a);
         WaveSlice<TB>::read(lb, l32, h, b);
+        wave_fence();   // the next stores into this LDS come after these reads
         __builtin_amdgcn_sched_barrier(0);   // all reads first: one LDS latency per slice
 #pragma unroll
         for (int s = 0; s < 4; ++s)
