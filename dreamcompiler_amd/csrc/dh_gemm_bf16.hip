@@ -1407,10 +1407,13 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     const bool mid = tiles <= (mid_max >= 0 ? mid_max : num_cus() / 2);
     const int K32 = K - K % 32;
     if (K < 1) return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
-    const long long a_bytes = 2LL * ((TA ? K : M) + 255) * lda,
-                    b_bytes = 2LL * ((TB ? N : K) + 255) * ldb;
+    // The direct-to-LDS kernels' byte offsets and buffer ranges have 32 bits.
+    auto fits = [&](int la, int lb) {
+        return 2LL * ((TA ? K : M) + 255) * la < (1LL << 32) &&
+               2LL * ((TB ? N : K) + 255) * lb < (1LL << 32);
+    };
     const bool stage64 = mid && mid_on && stage64_tiles(M, N, K, bt.count);
-    if ((K32 == 0 && !stage64) || (mid && !mid_on) || a_bytes >= (1LL << 32) || b_bytes >= (1LL << 32))
+    if ((K32 == 0 && !stage64) || (mid && !mid_on) || !fits(lda, ldb))
         return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
     const bool kmul = !stage64 || K % 8 == 0;
     const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0) && (TA || kmul);
@@ -1429,8 +1432,9 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
             st = launch_copies(c, n);
             const uint16_t *a = va ? A : c[0].dst, *b = vb ? B : c[n - 1].dst;
             const int la = va ? lda : c[0].ldo, lb = vb ? ldb : c[n - 1].ldo;
-            if (st == DH_OK)
-                st = stage64 ? launch_stage64<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
+            if (st == DH_OK)   // the padding may take an operand past 32-bit offsets
+                st = !fits(la, lb) ? launch_general<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
+                   : stage64 ? launch_stage64<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
                    : mid     ? launch_mid<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt)
                              : launch_fast<TA, TB>(M, N, K, a, la, b, lb, beta, C, ldc, bt);
         }

@@ -689,6 +689,29 @@ def test_bf16_64_wide_tiles(M, N, K, ta, tb, ldpad):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)      # exact bf16 products, fp32 sums
 
 
+def test_bf16_copied_rows_past_32_bit_offsets():
+    # 2,140,000 rows of 1001 values are below 2^32 bytes, their copy in rows of 1008 is not: that
+    # one needs 64-bit offsets.  One block of 1000 rows, stored 2140 times.
+    R, reps, K, N = 1000, 2140, 1001, 8
+    rng = np.random.default_rng(32)
+    A, B = (bf16_bits(rng.standard_normal(s, dtype=np.float32)) for s in ((R, K), (K, N)))
+    lib = hip.load()
+    dA, dB = hip.DeviceBuffer(reps * A.nbytes), hip.DeviceBuffer.from_numpy(B)
+    dC = hip.DeviceBuffer.empty((reps * R, N), np.float32)
+    try:
+        hip.check(lib.dh_memcpy_h2d(dA.ptr, A.ctypes.data, A.nbytes))
+        for i in range(1, reps):
+            hip.check(lib.dh_memcpy_d2d(dA.ptr + i * A.nbytes, dA.ptr, A.nbytes))
+        hip.gemm_bf16(0, 0, reps * R, N, K, dA, K, dB, N, 0.0, dC, N)
+        got = dC.numpy().reshape(reps, R, N)
+    finally:
+        for b in (dA, dB, dC):
+            b.free()
+        lib.dh_pool_release()   # 4 GB buffers
+    ref = bits_to_f32(A).astype(np.float64) @ bits_to_f32(B).astype(np.float64)
+    assert np.abs(got - ref).max() <= 1e-5 * np.sqrt(K) * np.abs(ref).max()
+
+
 # Between half a round and a round of 256 x 256 tiles the fast kernel runs a partial round
 # (144, 224 and 225 tiles here), at the boundary (128 tiles) the 128 x 128 path.
 @pytest.mark.parametrize("M,N,K", [(3000, 3000, 300), (3500, 4000, 96), (3840, 3840, 33),
