@@ -212,10 +212,13 @@ void* dh_malloc(size_t bytes) {
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
-        // One retry after returning the cached buffers to the driver.
+        // One retry after returning the cached buffers to the driver.  The runtime's copy of each
+        // failure is taken out: callers run a form without scratch, whose launch check reads it.
+        (void)hipGetLastError();
         dh_pool_release();
         e = hipMalloc(&p, bytes);
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             set_error(DH_ERR_OOM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
             return nullptr;
         }
@@ -404,6 +407,7 @@ void* dh_host_alloc(size_t bytes) {
     }
     void* p = nullptr;
     if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         set_error(DH_ERR_OOM, "hipHostMalloc(%zu) failed", bytes);
         return nullptr;
     }

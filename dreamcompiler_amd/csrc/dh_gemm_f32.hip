@@ -1650,10 +1650,7 @@ int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, Conv
     if (taps || flip) {
         Kt = static_cast<float*>(dh_malloc((size_t)Cout * (taps ? (long long)win * cp : R) * sizeof(float)));
         if (!Kt && flip) return set_error(DH_ERR_OOM, "dh_conv2d_bwd_data: flipped kernel");
-        if (!Kt) {   // the forward runs without scratch too
-            taps = false;
-            (void)hipGetLastError();
-        }
+        if (!Kt) taps = false;   // the forward runs without scratch too
     }
     if (taps) {
         R = (long long)win * cp;
@@ -1663,6 +1660,7 @@ int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, Conv
     } else if (flip) {
         conv_flip_kernel<<<stride_blocks((size_t)Cout * R), 256, 0, stream()>>>(Kn, Kt, g.Cin, Cout, g.KH, g.KW);
     }
+    int st = Kt ? check_launch("dh_conv2d(kernel)") : DH_OK;
     const long long t128 = (long long)((Cout + 127) / 128) * ((P + 127) / 128) * N;
     const long long t64 = (long long)((Cout + 63) / 64) * ((P + 63) / 64) * N;
     int S = 1;
@@ -1673,12 +1671,8 @@ int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, Conv
         const int nk = (int)((R + BK - 1) / BK), kz = (nk + S - 1) / S;
         S = (nk + kz - 1) / kz;   // no empty chunks
         if (S > 1) part = static_cast<float*>(dh_malloc(S * n * sizeof(float)));   // < 9 MB
-        if (!part) {
-            S = 1;
-            (void)hipGetLastError();
-        }
+        if (!part) S = 1;
     }
-    int st = Kt ? check_launch("dh_conv2d(kernel)") : DH_OK;
     if (st == DH_OK)
         st = (Cout <= 64 || t128 < cus ? launch_conv<64, 64> : launch_conv<128, 128>)(
             N, Cout, (int)P, (int)R, Kt ? Kt : Kn, X, g, part ? part : Y, part ? nullptr : bias,

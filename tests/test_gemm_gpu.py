@@ -689,6 +689,17 @@ def test_bf16_64_wide_tiles(M, N, K, ta, tb, ldpad):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)      # exact bf16 products, fp32 sums
 
 
+def test_failed_allocation_is_not_the_next_calls_error():
+    # Calls whose scratch cannot be had run a form without it: the runtime's record of the
+    # failed allocation must not reach their launch check.
+    lib = hip.load()
+    assert lib.dh_malloc(1 << 60) is None and b"hipMalloc" in lib.dh_last_error()
+    A = np.eye(40, dtype=np.float32)
+    for dtype in ("f32", "bf16"):
+        X = bf16_bits(A) if dtype == "bf16" else A
+        assert np.array_equal(gemm(X, X, dtype=dtype), A)
+
+
 def test_bf16_copied_rows_past_32_bit_offsets():
     # 2,140,000 rows of 1001 values are below 2^32 bytes, their copy in rows of 1008 is not: that
     # one needs 64-bit offsets.  One block of 1000 rows, stored 2140 times.
