@@ -1090,7 +1090,7 @@ struct StageOperand {
 // A k-contiguous operand has K a multiple of 8 (the host pads copies with zeros): past it whole
 // chunks of the last stage take an offset outside the buffer and land as zeros, as do k rows past
 // the end of the other kind, so no tail steps follow.
-template <bool TA, bool TB, int NS>
+template <bool TA, bool TB, int NS, bool CHAINS>
 __global__ void __launch_bounds__(256)
 gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
                          const uint16_t* __restrict__ B, int ldb, float beta,
@@ -1116,13 +1116,11 @@ gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, in
     const int nk = (K + 63) / 64;   // >= 1
     oa.init(lda, TA ? K : M, TA ? M : K, m0, K - 64 * (nk - 1), wave, lane);
     ob.init(ldb, TB ? N : K, TB ? K : N, n0, K - 64 * (nk - 1), wave, lane);
-    f32x16 acc[FM][FN];
+    // CHAINS: chains of 256 k in acc[0] and acc[1] in turn, each added to tot after the first
+    // products of the next.
+    f32x16 acc[2][FM][FN], tot[FM][FN];
 #pragma unroll
-    for (int a = 0; a < FM; ++a)
-#pragma unroll
-        for (int b = 0; b < FN; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+    for (int r = 0; r < 16; ++r) acc[0][0][0][r] = acc[1][0][0][r] = tot[0][0][r] = 0.f;
 
     auto stage_ptr = [&](int kt) { return ring + (kt % NS) * 2 * OA::ELEMS; };
     auto issue = [&](int kt) {
@@ -1140,15 +1138,21 @@ gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, in
         load_frags<OA, OB, FM, FN, OA::ELEMS>(stage_ptr(kt), kk, wm, wn, lane, fa, fb);
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto mma = [&](bf16x8 (&fa)[FM], bf16x8 (&fb)[FN]) {
-        mfma_block<FM, FN>(fa, fb, acc);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    read(0, 0, f0a, f0b);
-    for (int kt = 0; kt < nk; ++kt) {
+    auto stage = [&](auto cur_c, auto first_c, int kt) {   // into acc[cur]; first: of its chain
+        constexpr int cur = decltype(cur_c)::value;
+        auto mma = [&](bf16x8 (&fa)[FM], bf16x8 (&fb)[FN]) {
+            mfma_block<FM, FN>(fa, fb, acc[cur]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
         if (kt + NS - 1 < nk) issue(kt + NS - 1);
         read(kt, 1, f1a, f1b);
-        mma(f0a, f0b);
+        if (decltype(first_c)::value) {
+            acc[cur][0][0] = f32x16{};
+            mma(f0a, f0b);
+            tot[0][0] += acc[cur ^ 1][0][0];
+        } else {
+            mma(f0a, f0b);
+        }
         read(kt, 2, f0a, f0b);
         mma(f1a, f1b);
         read(kt, 3, f1a, f1b);
@@ -1161,8 +1165,27 @@ gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, in
             read(kt + 1, 0, f0a, f0b);
         }
         mma(f1a, f1b);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    read(0, 0, f0a, f0b);
+    if constexpr (CHAINS) {
+        constexpr int LEN = 4;   // stages
+        auto chain = [&](auto cur_c, int k0) {
+            stage(cur_c, std::true_type{}, k0);
+            const int k1 = min(nk, k0 + LEN);
+            for (int kt = k0 + 1; kt < k1; ++kt) stage(cur_c, std::false_type{}, kt);
+        };
+        for (int k0 = 0; k0 < nk; k0 += 2 * LEN) {
+            chain(even, k0);
+            if (k0 + LEN < nk) chain(odd, k0 + LEN);
+            else acc[1][0][0] = acc[0][0][0];   // the last chain, added below
+        }
+        acc[0][0][0] = tot[0][0] + acc[1][0][0];
+    } else {
+        for (int kt = 0; kt < nk; ++kt) stage(even, std::false_type{}, kt);
     }
-    store_tile<FM, FN, T>(M, N, beta, C, ldc, bias, epi, m0, n0, wm, wn, lane, acc);
+    store_tile<FM, FN, T>(M, N, beta, C, ldc, bias, epi, m0, n0, wm, wn, lane, acc[0]);
 }
 
 template <bool TA, bool TB>
@@ -1288,7 +1311,14 @@ int launch_stage64(int M, int N, int K, const uint16_t* A, int lda, const uint16
         return !e || std::atoi(e) != 0;
     }();
     const bool three = (long long)tiles * bt.count > 2LL * cus;   // see stage64_tiles
-    auto kern = three ? gemm_bf16_stage64_kernel<TA, TB, 3> : gemm_bf16_stage64_kernel<TA, TB, 4>;
+    // Long K: one chain of products over all of it rounds two to three times as much as K in up
+    // to 16 chunks does, chains of 256 k no more than that.  Error against 64 bits, one chain / 128 x
+    // 128 tiles split over K / chains: 768 x 768 x 4096 4.0e-7 / 1.17e-7 / 1.15e-7, 1023 x 1537 x 2050
+    // 2.7e-7 / 1.3e-7 / 1.0e-7; us: 19.9 / 33.0 / 21.0, 30.5 / 61 / 30.1; 1024 x 1536 x 2048 14.6 / 30.3 /
+    // 15.7.  (Rings of three: K <= 2048, and too many tiles for a split.)
+    auto kern = three     ? gemm_bf16_stage64_kernel<TA, TB, 3, false>
+              : K >= 2048 ? gemm_bf16_stage64_kernel<TA, TB, 4, true>
+                          : gemm_bf16_stage64_kernel<TA, TB, 4, false>;
     if (split_on && bt.count == 1 && 2 * tiles <= cus && K >= 2048) {
         int S = 2 * cus / tiles;
         S = S > 16 ? 16 : S;

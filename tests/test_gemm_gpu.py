@@ -689,6 +689,19 @@ def test_bf16_64_wide_tiles(M, N, K, ta, tb, ldpad):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)      # exact bf16 products, fp32 sums
 
 
+@pytest.mark.parametrize("M,N,K", [(768, 768, 4096), (1023, 1537, 2050), (483, 1760, 4630), (512, 512, 8192)])
+def test_bf16_64_wide_tiles_sum_long_k_in_chains(M, N, K):
+    # Products are exact in fp32, a rounding is uniform within 2^-24 of a partial sum (standard
+    # deviation u = 2^-24 / sqrt 3) and partial sums of k terms grow as sqrt k.  b steps of 16 k in each of
+    # n chains, whose n sums are then added: error / result = u sqrt((b + n) / 2).  Chains of 256 k:
+    # b = 16, n = K / 256; one chain of all of K (b = K / 16, n = 1) is two to three times that.
+    rng = np.random.default_rng(K)
+    A, B = (bf16_bits(rng.standard_normal(s, dtype=np.float32)) for s in ((M, K), (K, N)))
+    ref = bits_to_f32(A).astype(np.float64) @ bits_to_f32(B).astype(np.float64)
+    err = np.linalg.norm(gemm(A, B, dtype="bf16") - ref) / np.linalg.norm(ref)
+    assert err <= 1.1 * 2.0 ** -24 / np.sqrt(3) * np.sqrt((16 + K / 256) / 2)
+
+
 def test_failed_allocation_is_not_the_next_calls_error():
     # Calls whose scratch cannot be had run a form without it: the runtime's record of the
     # failed allocation must not reach their launch check.
