@@ -1053,8 +1053,16 @@ struct StageOperand {
             }
         }
         step = KCONTIG ? 128u : 128u * (uint32_t)ld;
-        // (a k-contiguous row ends with its last chunk: K is a multiple of 8, or the row is padded)
-        bytes = 2u * ((uint32_t)(rows - 1) * (uint32_t)ld + (KCONTIG ? (cols + 7) & ~7 : (cols + 1) & ~1));
+        bytes = 2u * ((uint32_t)(rows - 1) * (uint32_t)ld + ((cols + 1) & ~1));
+    }
+    // Zeros past k = klast in the last stage's chunk that holds the end of K, row by row: what
+    // follows a k-contiguous row may be the next one's values, possibly non-finite.
+    __device__ static void end_row(uint16_t* lds, int row, int klast) {
+        s16x8* p = reinterpret_cast<s16x8*>(lds + row * 64 + 8 * ((klast >> 3) ^ ((row >> 1) & 7)));
+        s16x8 v = *p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = e < (klast & 7) ? v[e] : (short)0;
+        *p = v;
     }
     __device__ void issue(const uint16_t* __restrict__ g, int kt, bool at_end, uint16_t* lds,
                           int wave) const {
@@ -1087,9 +1095,9 @@ struct StageOperand {
     }
 };
 
-// A k-contiguous operand has K a multiple of 8 (the host pads copies with zeros): past it whole
-// chunks of the last stage take an offset outside the buffer and land as zeros, as do k rows past
-// the end of the other kind, so no tail steps follow.
+// No tail steps follow the last stage: past K whole chunks of a k-contiguous operand take an offset
+// outside the buffer and land as zeros, as do k rows past the end of the other kind, and a K that
+// ends inside a chunk is cut off in LDS (StageOperand::end_row).
 template <bool TA, bool TB, int NS, bool CHAINS>
 __global__ void __launch_bounds__(256)
 gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
@@ -1132,6 +1140,15 @@ gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, in
     for (int s = 0; s < pre; ++s) issue(s);
     wait_dma_stages<2 * OA::PER>(pre - 1);
     __syncthreads();
+    auto end_rows = [&] {   // the last stage, once it has landed
+        const int klast = K - 64 * (nk - 1);
+        uint16_t* st = stage_ptr(nk - 1);
+        if (!TA && wave == 0) OA::end_row(st, lane, klast);
+        if (TB && wave == 1) OB::end_row(st + OA::ELEMS, lane, klast);
+        __syncthreads();
+    };
+    const bool cut = (!TA || TB) && K % 8 != 0;
+    if (cut && nk == 1) end_rows();
     asm volatile("" ::"s"(C), "s"(ldc), "s"(beta), "s"(bias), "s"(epi));
     bf16x8 f0a[FM], f0b[FN], f1a[FM], f1b[FN];
     auto read = [&](int kt, int kk, bf16x8 (&fa)[FM], bf16x8 (&fb)[FN]) {
@@ -1162,6 +1179,7 @@ gemm_bf16_stage64_kernel(int M, int N, int K, const uint16_t* __restrict__ A, in
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             wait_dma_stages<2 * OA::PER>(min(nk - 1, kt + NS - 1) - (kt + 1));
             __syncthreads();
+            if (cut && kt + 2 == nk) end_rows();
             read(kt + 1, 0, f0a, f0b);
         }
         mma(f1a, f1b);
@@ -1420,9 +1438,8 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     // way).
     // Ragged M and N are edge tiles, a K that is not a multiple of 32 ends with the larger tiles'
     // masked tail steps (a DMA'd k-contiguous tile would read the next row's values, possibly
-    // non-finite, past K; the 64 x 64 kernel leaves out whole 16-byte chunks, so it takes K in
-    // eights of such an operand).  One product's rows that do not fit this are copied to aligned,
-    // zero-padded ones first, both operands in one launch, unless
+    // non-finite, past K; the 64 x 64 kernel zeroes those in LDS).  One product's rows that are not
+    // 16-byte aligned are copied to aligned ones first, both operands in one launch, unless
     // K <= 16, one step of the general kernel.  Row-major with odd rows, us, general / copied:
     // 5 x 7 x 9 5.7 / 8.0, 33 x 65 x 17 10.2 / 8.1, 255^3 22.4 / 7.5, 1 x 1000 x 1001 24.7 / 9.0.
     static const bool mid_on = [] {
@@ -1445,9 +1462,8 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     const bool stage64 = mid && mid_on && stage64_tiles(M, N, K, bt.count);
     if ((K32 == 0 && !stage64) || (mid && !mid_on) || !fits(lda, ldb))
         return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
-    const bool kmul = !stage64 || K % 8 == 0;
-    const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0) && (TA || kmul);
-    const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0) && (!TB || kmul);
+    const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0);
+    const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0);
     if (!va || !vb) {
         if (bt.count > 1 || K <= 16)
             return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);

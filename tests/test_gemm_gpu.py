@@ -689,6 +689,32 @@ def test_bf16_64_wide_tiles(M, N, K, ta, tb, ldpad):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)      # exact bf16 products, fp32 sums
 
 
+@pytest.mark.parametrize("Bt", [1, 3])
+@pytest.mark.parametrize("M,N,K", [(70, 64, 50), (128, 130, 100), (64, 65, 33), (130, 72, 257), (96, 200, 2051),
+                                   (1100, 1100, 132)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+def test_bf16_aligned_rows_with_k_inside_a_chunk(Bt, M, N, K, ta, tb):
+    # Rows padded to eights whose K ends inside a 16-byte chunk, one product and batches: 64 x 64
+    # tiles (one stage, several, split K) and, for 3 of 1100 x 1100, 128 x 128.  The padding is
+    # infinite, so a value taken from past a row's end would show.  Bound as above.
+    rng = np.random.default_rng(M + N + K + Bt)
+    A = rng.standard_normal((Bt,) + ((K, M) if ta else (M, K)), dtype=np.float32)
+    B = rng.standard_normal((Bt,) + ((N, K) if tb else (K, N)), dtype=np.float32)
+
+    def padded(X):
+        P = np.full(X.shape[:2] + ((X.shape[2] + 7) // 8 * 8,), np.inf, np.float32)
+        P[:, :, :X.shape[2]] = X
+        return hip.DeviceBuffer.from_numpy(bf16_bits(P)), P.shape[2]
+
+    (dA, lda), (dB, ldb) = padded(A), padded(B)
+    dC = hip.DeviceBuffer.empty((Bt, M, N), np.float32)
+    hip.gemm_ex("bf16", ta, tb, M, N, K, dA, lda, A.shape[1] * lda, dB, ldb, B.shape[1] * ldb, 0.0, dC,
+                N, M * N, Bt)
+    A, B = (bits_to_f32(bf16_bits(X)).astype(np.float64) for X in (A, B))
+    ref = np.matmul(np.swapaxes(A, 1, 2) if ta else A, np.swapaxes(B, 1, 2) if tb else B)
+    assert maxrel(dC.numpy(), ref) <= 1e-5 * np.sqrt(K)
+
+
 @pytest.mark.parametrize("M,N,K", [(768, 768, 4096), (1023, 1537, 2050), (483, 1760, 4630), (512, 512, 8192)])
 def test_bf16_64_wide_tiles_sum_long_k_in_chains(M, N, K):
     # Products are exact in fp32, a rounding is uniform within 2^-24 of a partial sum (standard
