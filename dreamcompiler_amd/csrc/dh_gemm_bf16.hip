@@ -1426,6 +1426,23 @@ int launch_copies(const RowCopy* c, int n) {
     return check_launch("dh_gemm_bf16(aligned copy)");
 }
 
+// One product with unaligned rows: us that the general kernel takes on them, fitted over M, N of 1 to
+// 8001 and K of 17 to 129, and what the copy and a 64 x 64 grid take while both are bound by
+// their launches (6.8 to 7.9 by box).  General / copied, NN with odd rows: 1 x 1 x 17 5.0 / 7.7,
+// 5 x 7 x 33 5.8 / 8.6, 16 x 8 x 65 6.7 / 7.9, 33 x 16 x 33 6.7 / 7.7, 1 x 1001 x 33 6.9 / 7.6, 33 x 65 x 17
+// 10.2 / 8.1, 129 x 131 x 63 16.6 / 8.7, 1 x 1001 x 401 27 / 8.8; B's rows aligned: 4 x 64 x 65 7.0 / 8.1, 33 x
+// 64 x 17 9.2 / 6.8; 1 x 1 x 129 NT 6.8 / 7.7, TN 8.4 / 8.0.
+constexpr double COPIED_US = 7.4;
+
+template <bool TA, bool TB>
+double small_general_us(int M, int N, int K, bool aligned_b) {
+    const double m = M < 64 ? M : 64;
+    double n = N < 16 ? 0 : N < 40 ? N - 16 : 24;
+    if (aligned_b && M < 32) n *= m / 32;
+    const double ta = TA ? (M < 10 ? M : 10) : 0;   // A's k rows: more loads, each of few values
+    return 4.9 + 0.055 * m + 0.07 * n + 0.1 * ta + (TB && !TA ? 0.017 : 0.021 + 0.002 * ta) * K;
+}
+
 template <bool TA, bool TB>
 int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb,
            float beta, float* C, int ldc, const Batch& bt) {
@@ -1439,9 +1456,8 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     // Ragged M and N are edge tiles, a K that is not a multiple of 32 ends with the larger tiles'
     // masked tail steps (a DMA'd k-contiguous tile would read the next row's values, possibly
     // non-finite, past K; the 64 x 64 kernel zeroes those in LDS).  One product's rows that are not
-    // 16-byte aligned are copied to aligned ones first, both operands in one launch, unless
-    // K <= 16, one step of the general kernel.  Row-major with odd rows, us, general / copied:
-    // 5 x 7 x 9 5.7 / 8.0, 33 x 65 x 17 10.2 / 8.1, 255^3 22.4 / 7.5, 1 x 1000 x 1001 24.7 / 9.0.
+    // 16-byte aligned are copied to aligned ones first, both operands in one launch, unless K <= 16
+    // or the general kernel is the faster one (small_general_us).
     static const bool mid_on = [] {
         const char* e = std::getenv("DH_GEMM_BF16_MID");   // tuning knob: 0 or 1
         return !e || std::atoi(e) != 0;
@@ -1465,7 +1481,7 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0);
     const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0);
     if (!va || !vb) {
-        if (bt.count > 1 || K <= 16)
+        if (bt.count > 1 || K <= 16 || small_general_us<TA, TB>(M, N, K, vb) < COPIED_US)
             return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
         RowCopy c[2];
         int n = 0;
