@@ -92,6 +92,12 @@ hipStream_t stream() {
 
 int num_cus() { return st().cus; }
 
+bool capturing() {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream(), &c) != hipSuccess) (void)hipGetLastError();
+    return c != hipStreamCaptureStatusNone;
+}
+
 int check_launch(const char* what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(DH_ERR_HIP, "%s launch failed: %s", what,

@@ -1433,6 +1433,9 @@ int launch_copies(const RowCopy* c, int n) {
 // 10.2 / 8.1, 129 x 131 x 63 16.6 / 8.7, 1 x 1001 x 401 27 / 8.8; B's rows aligned: 4 x 64 x 65 7.0 / 8.1, 33 x
 // 64 x 17 9.2 / 6.8; 1 x 1 x 129 NT 6.8 / 7.7, TN 8.4 / 8.0.
 constexpr double COPIED_US = 7.4;
+// Under stream capture, products of fewer multiply-adds go without the copies' scratch (33 x 65 x 401
+// 28.0 us instead of 8.5); from here on the general kernel takes 5 to 10 times as long.
+constexpr long long CAPTURE_MAC = 1LL << 22;
 
 template <bool TA, bool TB>
 double small_general_us(int M, int N, int K, bool aligned_b) {
@@ -1481,7 +1484,8 @@ int launch(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, i
     const bool va = ((uintptr_t)A % 16 == 0) && (lda % 8 == 0) && (bt.sA % 8 == 0);
     const bool vb = ((uintptr_t)B % 16 == 0) && (ldb % 8 == 0) && (bt.sB % 8 == 0);
     if (!va || !vb) {
-        if (bt.count > 1 || K <= 16 || small_general_us<TA, TB>(M, N, K, vb) < COPIED_US)
+        if (bt.count > 1 || K <= 16 || small_general_us<TA, TB>(M, N, K, vb) < COPIED_US ||
+            (mid && (long long)M * N * K < CAPTURE_MAC && capturing()))
             return launch_general<TA, TB>(M, N, K, A, lda, B, ldb, beta, C, ldc, bt);
         RowCopy c[2];
         int n = 0;

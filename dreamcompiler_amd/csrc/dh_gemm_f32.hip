@@ -1641,11 +1641,12 @@ constexpr double CONV_PACK_FLOPS = 1e9;
 int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, ConvGeom g, float* Y,
              const float* bias, int accumulate, bool flip) {
     const int cus = num_cus(), win = g.KH * g.KW;
+    const bool scratch = !capturing();
     long long R = (long long)g.Cin * win;
     const int cp = (g.Cin + BK - 1) / BK * BK;
     bool taps = 8ll * (cp - g.Cin) <= g.Cin && (long long)win * cp <= LD_BUF_MAX &&
                 (long long)Cout * win * cp <= 1ll << 30 &&
-                (flip || 2.0 * N * Cout * P * R >= CONV_PACK_FLOPS);
+                (flip || (scratch && 2.0 * N * Cout * P * R >= CONV_PACK_FLOPS));
     float* Kt = nullptr;
     if (taps || flip) {
         Kt = static_cast<float*>(dh_malloc((size_t)Cout * (taps ? (long long)win * cp : R) * sizeof(float)));
@@ -1666,7 +1667,7 @@ int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, Conv
     int S = 1;
     float* part = nullptr;
     const size_t n = (size_t)N * Cout * P;
-    if (2 * t64 <= cus && R >= 16 * BK) {
+    if (scratch && 2 * t64 <= cus && R >= 16 * BK) {
         S = (int)std::min<long long>(2 * cus / t64, R / (8 * BK));
         const int nk = (int)((R + BK - 1) / BK), kz = (nk + S - 1) / S;
         S = (nk + kz - 1) / kz;   // no empty chunks

@@ -157,6 +157,60 @@ def _hip_runtime():
     return rt
 
 
+@pytest.mark.parametrize("case", ["conv_packed", "conv_split", "bf16_copy"])
+def test_calls_with_optional_scratch_under_stream_capture(case):
+    """conv2d's packed kernel and split contraction and the bf16 products' aligned copies are scratch for
+    speed: recorded with an empty pool, where a hipMalloc would end the capture, these calls
+    run without.  Replayed three times with eager work on the outputs between; the eager call
+    adds in another order, hence 1e-5 sqrt(terms) as for the kernels themselves."""
+    rng = np.random.default_rng(3)
+    if case == "bf16_copy":
+        M, N, K = 33, 65, 401
+        bufs = [DB.from_numpy((rng.standard_normal(s).astype(np.float32).view(np.uint32) >> 16)
+                              .astype(np.uint16)) for s in ((M, K), (K, N))]
+        out, terms = DB.empty((M, N), np.float32), K
+        call = lambda: hip.load().dh_gemm_bf16(0, 0, M, N, K, bufs[0].ptr, K, bufs[1].ptr, N, 0.0,  # noqa: E731
+                                               out.ptr, N)
+    else:
+        N, C, H = (20, 64, 28) if case == "conv_packed" else (2, 64, 14)
+        bufs = [DB.from_numpy(rng.standard_normal(s).astype(np.float32))
+                for s in ((N, C * H * H), (C, 9 * C))]
+        out, terms = DB.empty((N, C * H * H), np.float32), 9 * C
+        call = lambda: hip.load().dh_conv2d_fwd(bufs[0].ptr, bufs[1].ptr, None, out.ptr, N, C, H, H,  # noqa: E731
+                                                C, 3, 3, 1, 1)
+    R, lib = _hip_runtime(), hip.load()
+    garbage = np.full(out.shape, 7.0, np.float32)
+    s, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert R.hipStreamCreate(ctypes.byref(s)) == 0
+    try:
+        hip.check(lib.dh_set_stream(s), "dh_set_stream")
+        hip.check(call(), "eager call")
+        want = out.numpy()
+        hip.check(lib.dh_pool_release(), "dh_pool_release")
+        assert R.hipStreamBeginCapture(s, 0) == 0            # hipStreamCaptureModeGlobal
+        st = call()
+        end = R.hipStreamEndCapture(s, ctypes.byref(graph))
+        hip.check(st, case + " under capture")
+        assert end == 0
+        assert R.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for _ in range(3):
+            hip.check(lib.dh_memcpy_h2d(out.ptr, garbage.ctypes.data, garbage.nbytes), "dh_memcpy_h2d")
+            hip.sync()
+            assert R.hipGraphLaunch(exe, s) == 0
+            assert R.hipStreamSynchronize(s) == 0
+            assert np.abs(out.numpy() - want).max() <= 1e-5 * np.sqrt(terms) * np.abs(want).max()
+    finally:
+        lib.dh_set_stream(None)
+        if exe.value:
+            R.hipGraphExecDestroy(exe)
+        if graph.value:
+            R.hipGraphDestroy(graph)
+        R.hipStreamSynchronize(s)
+        R.hipStreamDestroy(s)
+        for b in bufs + [out]:
+            b.free()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_noalloc_under_stream_capture_replays(dtype):
     """A warm call (first-use set-up: scratch address, kernel attributes), then the same call
