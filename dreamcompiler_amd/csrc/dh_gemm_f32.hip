@@ -1162,6 +1162,8 @@ auto pick_kernel(int M, int N, int K, const float* A, int lda, long long sA, con
     return buf && k4  ? gemm_f32_kernel<TA, TB, LD_BUF4, LD_BUF4, TBM, TBN>
          : buf        ? gemm_f32_kernel<TA, TB, LD_BUF, LD_BUF, TBM, TBN>
          : va && vb   ? gemm_f32_kernel<TA, TB, LD_VEC, LD_VEC, TBM, TBN>
+         : va         ? gemm_f32_kernel<TA, TB, LD_VEC, LD_SCALAR, TBM, TBN>
+         : vb         ? gemm_f32_kernel<TA, TB, LD_SCALAR, LD_VEC, TBM, TBN>
                       : gemm_f32_kernel<TA, TB, LD_SCALAR, LD_SCALAR, TBM, TBN>;
 }
 
@@ -1483,7 +1485,12 @@ int launch_ks(int M, int N, int K, const float* A, int lda, const float* B, int 
                                   : gemm_f32_ks_kernel<TA, TB, LD_BUF, LD_BUF, 2>)
               : va && vb  ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_VEC, 4>
                                   : gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_VEC, 2>)
-                          : gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_SCALAR, 2>;
+              : va        ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_SCALAR, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_VEC, LD_SCALAR, 2>)
+              : vb        ? (deep ? gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_VEC, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_VEC, 2>)
+                          : (deep ? gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_SCALAR, 4>
+                                  : gemm_f32_ks_kernel<TA, TB, LD_SCALAR, LD_SCALAR, 2>);
     const int tiles = ((M + 63) / 64) * ((N + 63) / 64);
     for (int b0 = 0; b0 < bt.count; b0 += 65535) {
         const int nb = bt.count - b0 < 65535 ? bt.count - b0 : 65535;

@@ -889,6 +889,36 @@ def test_fp32_32x32_tiles_batched_epilogue(Bt, M, N, K, relu, row_bias):
         assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)
 
 
+@pytest.mark.parametrize("M,N,K", [(20, 24, 36), (100, 99, 300), (130, 72, 516), (70, 300, 2052)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("which", ["A", "B"])
+def test_fp32_one_operand_aligned_past_32_bit_offsets(M, N, K, ta, tb, which):
+    # one operand in rows of 2^20 + 8 on 16-byte boundaries, the other 4 bytes past one
+    rng = np.random.default_rng(M + N + K)
+    X = [f32(rng.standard_normal((M, K))), f32(rng.standard_normal((K, N)))]
+    dev, ld = [], []
+    for x, t, wide in ((X[0], ta, which == "A"), (X[1], tb, which == "B")):
+        x = np.ascontiguousarray(x.T if t else x)
+        ld.append((1 << 20) + 8 if wide else x.shape[1])
+        if wide:
+            d = hip.DeviceBuffer(4 * ((x.shape[0] - 1) * ld[-1] + x.shape[1]))
+            for i in range(x.shape[0]):
+                hip.check(hip.load().dh_memcpy_h2d(d.ptr + 4 * i * ld[-1], x[i].ctypes.data, x[i].nbytes))
+            hip.sync()
+        else:
+            d = hip.DeviceBuffer.from_numpy(np.concatenate([[np.float32(np.nan)], x.ravel()]))
+        dev.append((d, d.ptr + (0 if wide else 4)))
+    dC = hip.DeviceBuffer.empty((M, N), np.float32)
+    try:
+        hip.gemm_f32(ta, tb, M, N, K, dev[0][1], ld[0], dev[1][1], ld[1], 0.0, dC, N)
+        got = dC.numpy()
+    finally:
+        for d, _ in dev:
+            d.free()
+        hip.load().dh_pool_release()   # up to 9 GB
+    assert maxrel(got, X[0].astype(np.float64) @ X[1].astype(np.float64)) <= 1e-5 * np.sqrt(K)
+
+
 def test_fp32_leading_dimensions_past_32_bit_offsets():
     # above 2^20: element by element, or (aligned) with 64-bit addresses
     for ld in ((1 << 20) + 1, (1 << 20) + 4):
