@@ -854,12 +854,14 @@ __global__ void __launch_bounds__(256) conv_split_reduce(const float* __restrict
 template <int TBM, int TBN>
 int launch_conv(int N, int Cout, int P, int R, const float* Kn, const float* X,
                 const ConvGeom& g, float* Y, const float* bias, int accumulate, bool taps, int S) {
-    // kernel rows of any alignment by 16-byte buffer loads; longer than 32-bit offsets reach:
-    // element by element
+    // kernel rows of any alignment by 16-byte buffer loads; longer than 32-bit offsets reach: with
+    // 64-bit addresses, 16 bytes at a time where aligned
+    const bool vec = R % 4 == 0 && (uintptr_t)Kn % 16 == 0;
     auto kern = taps             ? conv_fwd_kernel<TBM, TBN, LD_BUF4, true>
-              : R > LD_BUF_MAX   ? conv_fwd_kernel<TBM, TBN, LD_SCALAR, false>
-              : R % 4 == 0       ? conv_fwd_kernel<TBM, TBN, LD_BUF4, false>
-                                 : conv_fwd_kernel<TBM, TBN, LD_BUF, false>;
+              : R <= LD_BUF_MAX  ? (R % 4 == 0 ? conv_fwd_kernel<TBM, TBN, LD_BUF4, false>
+                                               : conv_fwd_kernel<TBM, TBN, LD_BUF, false>)
+              : vec              ? conv_fwd_kernel<TBM, TBN, LD_VEC, false>
+                                 : conv_fwd_kernel<TBM, TBN, LD_SCALAR, false>;
     const int tiles = ((Cout + TBM - 1) / TBM) * ((P + TBN - 1) / TBN);
     const int nk = (R + BK - 1) / BK, kz = (nk + S - 1) / S;
     for (int z0 = 0; z0 < N; z0 += 65535) {
@@ -1120,9 +1122,11 @@ int launch_wgrad(int N, int Cout, int P, int R, const float* dY, const float* X,
     S = (total + chunk - 1) / chunk;
     float* part = static_cast<float*>(dh_malloc((size_t)S * Cout * R * sizeof(float)));
     if (!part) return set_error(DH_ERR_OOM, "dh_conv2d_bwd_filter: partials");
-    auto kern = P > LD_BUF_MAX ? conv_wgrad_kernel<TBM, TBN, LD_SCALAR>
-              : P % 4 == 0     ? conv_wgrad_kernel<TBM, TBN, LD_BUF4>
-                               : conv_wgrad_kernel<TBM, TBN, LD_BUF>;
+    const bool vec = P % 4 == 0 && (uintptr_t)dY % 16 == 0;
+    auto kern = P <= LD_BUF_MAX ? (P % 4 == 0 ? conv_wgrad_kernel<TBM, TBN, LD_BUF4>
+                                              : conv_wgrad_kernel<TBM, TBN, LD_BUF>)
+              : vec             ? conv_wgrad_kernel<TBM, TBN, LD_VEC>
+                                : conv_wgrad_kernel<TBM, TBN, LD_SCALAR>;
     const dim3 grid(tiles, (unsigned)S);
     hipStream_t s = stream();
     kern<<<grid, NTHREADS, 0, s>>>(Cout, P, R, dY, X, g, nkp, (int)total, (int)chunk, part);

@@ -139,6 +139,24 @@ def test_conv2d_packed_and_split_against_oracle(shape):
             t.free()
 
 
+def test_conv2d_bwd_filter_planes_past_32_bit_offsets():
+    # planes of more than 2^20 positions: rows of dY by 64-bit addresses, 16 bytes at a time (a
+    # multiple of 4 positions on 16-byte boundaries) or value by value
+    for H, W, off in ((1030, 1028, 0), (1030, 1028, 1), (1031, 1029, 0)):
+        N, Cin, Cout, k = 1, 2, 3, 3
+        rng = np.random.default_rng(H + off)
+        X = rng.standard_normal((N, Cin * H * W)).astype(np.float32)
+        G = rng.standard_normal((N, Cout * H * W)).astype(np.float32)
+        dX, dG = DB.from_numpy(X), DB.from_numpy(np.concatenate([np.zeros(off, np.float32), G.ravel()]))
+        dK = DB.empty((Cout, Cin * k * k), np.float32)
+        hip.conv2d_bwd_filter(dG.ptr + 4 * off, dX, dK, N, Cin, H, W, Cout, k, k, 1, 1)
+        ref = O.conv2d_bwd(X.astype(np.float64), np.zeros((Cout, Cin * k * k)), G.astype(np.float64), N,
+                           Cin, H, W, Cout, k, k, 1, 1)[1]
+        assert maxrel(dK.numpy(), ref) <= 1e-5 * np.sqrt(N * H * W)
+        for t in (dX, dG, dK):
+            t.free()
+
+
 def test_conv2d_fwd_rejects_bad_shapes():
     d = DB.empty((64,), np.float32)
     try:
