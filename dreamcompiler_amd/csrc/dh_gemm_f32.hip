@@ -573,9 +573,11 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
     float* lb = la + SZ;
     WaveSlice<!TA> sa[2];
     WaveSlice<TB> sb[2];
-    f32x16 acc[2];   // of even and odd slices: chains of half the length round less
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+    // acc: the chain of products of two slices, added to tot under the next one's LDS reads.  Error
+    // against 64 bits, chains of every other slice of a wave / 64 x 64 tiles split over K / these:
+    // 512 x 512 x 4096 2.9e-7 / 2.3e-7 / 1.65e-7, 1292 x 128 x 3680 2.8e-7 / 2.35e-7 / 1.6e-7; us: 25.1 / 41.5 /
+    // 25.8, 22.8 / 43.6 / 23.1.
+    f32x16 acc = {}, tot = {};
     const int nk = (K + WV_BK - 1) / WV_BK;
     auto fetch = [&](auto set_c, int i) {   // the wave's slice i (past K: zeros)
         constexpr int set = decltype(set_c)::value;
@@ -601,11 +603,15 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
         WaveSlice<TB>::read(lb, l32, h, b);
         wave_fence();   // the next stores into this LDS come after these reads
         __builtin_amdgcn_sched_barrier(0);   // all reads first: one LDS latency per slice
+        if (set == 0) {
+            tot += acc;
+            acc = f32x16{};
+        }
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc[set] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], acc[set], 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][j], b[s][j], acc, 0, 0, 0);
     };
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
@@ -620,7 +626,7 @@ gemm_f32_wave_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
     }
     // partial tiles, lane-major, in the waves' own LDS
 #pragma unroll
-    for (int r = 0; r < 16; ++r) la[r * 64 + lane] = acc[0][r] + acc[1][r];
+    for (int r = 0; r < 16; ++r) la[r * 64 + lane] = tot[r] + acc[r];
     __syncthreads();
     const bool row_bias = bias && (epi & DH_EPI_ROW_BIAS), relu = epi & DH_EPI_RELU;
 #pragma unroll

@@ -889,6 +889,21 @@ def test_fp32_32x32_tiles_batched_epilogue(Bt, M, N, K, relu, row_bias):
         assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1292, 128, 3680), (512, 512, 4096)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+def test_fp32_32x32_tiles_sum_long_k_in_chains(M, N, K, ta, tb):
+    # As for the bf16 chains: roundings of standard deviation u = 2^-24 / sqrt 3 of partial sums that
+    # grow as sqrt k.  Chains of 64 k in steps of 2, those of each of 8 waves added up, then the
+    # waves: error / result = u sqrt(16 + K / 1024 + 4); chains over a wave's whole K / 8, u sqrt(K / 16 + 4).
+    rng = np.random.default_rng(K)
+    A, B = f32(rng.standard_normal((M, K))), f32(rng.standard_normal((K, N)))
+    got = gemm(np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, bool(ta),
+               bool(tb))
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= 1.1 * 2.0 ** -24 / np.sqrt(3) * np.sqrt(20 + K / 1024)
+
+
 @pytest.mark.parametrize("M,N,K", [(20, 24, 36), (100, 99, 300), (130, 72, 516), (70, 300, 2052)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("which", ["A", "B"])
