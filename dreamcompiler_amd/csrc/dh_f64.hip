@@ -57,6 +57,8 @@ constexpr int F64_PAD = 80;       // 64-wide tile + 16-deep stage (or 32 + 32)
 
 // Explicitly global pointers: through the argument struct they would become flat loads.
 typedef const double __attribute__((address_space(1)))* GlobalF64;
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef const f64x2u __attribute__((address_space(1)))* GlobalF64x2;
 typedef const char __attribute__((address_space(1)))* GlobalBytes;
 __device__ double g_zero64;   // zero-initialised, never written
 
@@ -227,7 +229,13 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
         const int k0 = k_of(q), valid = valid_of(q);
         const GlobalBytes pa = abase + 8LL * (TA == 0 ? k0 : (long long)k0 * ar.lda);
         const GlobalBytes pb = bbase + 8LL * (TB == 1 ? k0 : (long long)k0 * ar.ldb);
-        if constexpr (WIDE) {   // 64-bit offsets, value by value
+        if (WIDE && valid == KT && ma == TILE && nb == TILE) {   // 64-bit offsets
+#pragma unroll
+            for (int r = 0; r < NLD; ++r) {
+                ra[set][r] = *(GlobalF64x2)(pa + ao[r]);
+                rb[set][r] = *(GlobalF64x2)(pb + bo[r]);
+            }
+        } else if constexpr (WIDE) {   // the same at an edge, value by value
             const GlobalBytes zero = (GlobalBytes)&g_zero64;
 #pragma unroll
             for (int r = 0; r < NLD; ++r)
@@ -538,11 +546,13 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
     // 1024 22.6 / 17.9, 256 x 1023 x 4096 81.9 / 58.4), or, where the tiles leave half the CUs
     // idle, one work-group per block, whose chain sums gemm_f64_reduce adds in k order (64^2 x
     // 4096 77.7 / 15.3, 300^2 x 1000 21.8 / 15.6; with groups 56.7 and 17.5).  Every form leaves
-    // the results bit-identical.  Leading dimensions past 2^22 need 64-bit offsets within a
-    // tile: one form has them.
+    // the results bit-identical.  Leading dimensions that take a tile past 32-bit
+    // offsets (2^22 to 2^24, see `wide`) have forms with 64-bit ones.
     const long long cus = num_cus();
-    const bool wide = lda > (1 << 22) || ldb > (1 << 22);
-    const int wb = !wide && ((M + 63) / 64) * (long long)((N + 63) / 64) * batch >= 2 * cus ? 2 : 1;
+    const int wb = ((M + 63) / 64) * (long long)((N + 63) / 64) * batch >= 2 * cus ? 2 : 1;
+    // rows of a tile and stage: the tile's, or its k
+    const int rows_a = transA ? (wb == 2 ? 16 : 32) : 32 * wb, rows_b = transB ? 32 * wb : wb == 2 ? 16 : 32;
+    const bool wide = 8LL * rows_a * lda > 0x7fffffffLL || 8LL * rows_b * ldb > 0x7fffffffLL;
     const long long tilesM = (M + 32 * wb - 1) / (32 * wb), tilesN = (N + 32 * wb - 1) / (32 * wb);
     const long long tiles = tilesM * tilesN * batch;
     const long long nkb = ((long long)K + F64_KC - 1) / F64_KC;
@@ -560,7 +570,8 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
                     part ? (unsigned)nkb : 1u);
     const F64Args ar{M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, (int)tilesN, part,
                      causal, row0, (int)cus};
-    if (wide) launch_f64<1, 32, 1, true>(transA, transB, grid, ar);
+    if (wide && wb == 2) launch_f64<2, 16, 1, true>(transA, transB, grid, ar);
+    else if (wide) launch_f64<1, 32, 1, true>(transA, transB, grid, ar);
     else if (wb == 2) launch_f64<2, 16, 1>(transA, transB, grid, ar);
     else if (G == 1) launch_f64<1, 32, 1>(transA, transB, grid, ar);
     else if (G == 2) launch_f64<1, 32, 2>(transA, transB, grid, ar);

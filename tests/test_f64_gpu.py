@@ -266,17 +266,29 @@ def test_gemm_f64_forms_are_bit_identical(M, N, K):
             assert np.array_equal(dC.numpy(), ref), (ta, tb)
 
 
-def test_gemm_f64_huge_leading_dimension():
-    # a leading dimension past 2^22: the form with 64-bit offsets
-    ld, M, N, K = (1 << 22) + 3, 5, 7, 300
+@pytest.mark.parametrize("which,M,N,K,ld", [("A", 5, 7, 300, (1 << 22) + 3), ("A", 40, 70, 40, (1 << 23) + 3),
+                                            ("A", 64, 33000, 40, (1 << 22) + 3), ("B", 40, 70, 300, (1 << 23) + 5),
+                                            ("B", 65, 33000, 20, (1 << 24) + 9)])
+def test_gemm_f64_huge_leading_dimension(which, M, N, K, ld):
+    # leading dimensions that take a tile past 32-bit offsets (but the first), 32- and 64-wide
+    # tiles, whole and ragged ones and stages: the forms with 64-bit offsets
     rng = np.random.default_rng(22)
     A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
-    wide = np.zeros((M - 1) * ld + K)
-    for i in range(M):
-        wide[i * ld:i * ld + K] = A[i]
-    dA, dB, dC = DB.from_numpy(wide), DB.from_numpy(B), DB.empty((M, N), np.float64)
-    hip.gemm_f64(0, 0, M, N, K, dA, ld, dB, N, 0.0, dC, N)
-    assert np.array_equal(dC.numpy(), O.gemm_d(A, B))
+    X = A if which == "A" else B
+    wide = DB(8 * ((X.shape[0] - 1) * ld + X.shape[1]))
+    other, dC = DB.from_numpy(B if which == "A" else A), DB.empty((M, N), np.float64)
+    try:
+        for i in range(X.shape[0]):
+            hip.check(hip.load().dh_memcpy_h2d(wide.ptr + 8 * i * ld, X[i].ctypes.data, X[i].nbytes))
+        if which == "A":
+            hip.gemm_f64(0, 0, M, N, K, wide, ld, other, N, 0.0, dC, N)
+        else:
+            hip.gemm_f64(0, 0, M, N, K, other, K, wide, ld, 0.0, dC, N)
+        assert np.array_equal(dC.numpy(), O.gemm_d(A, B))
+    finally:
+        for t in (wide, other, dC):
+            t.free()
+        hip.load().dh_pool_release()   # up to 20 GB
 
 
 @pytest.mark.parametrize("B,S,D,rows", [(2, 63, 40, 0), (1, 64, 8, 0), (3, 65, 130, 0),
