@@ -124,16 +124,18 @@ struct F64Cfg {
 // g, g + G, ... and the chain sums meet in LDS, where group 0 adds them in k order.  A
 // small grid is bound by the chain of memory latencies of a work-group's k-stages; G groups
 // run G such chains at a time without a second launch and its partials.  Each group stages its
-// own operands: KT k per stage, double-buffered in LDS, two stages in flight in registers (a
-// load has two stages' products to land).  With `part`, blockIdx.z takes G blocks and every
+// own operands: KT k per stage, double-buffered in LDS.  DEEP: stages in pairs, two in flight in
+// registers (a load has two stages' products to land); else stage by stage, one in flight, in
+// the compiler's schedule.  With `part`, blockIdx.z takes G blocks and every
 // group writes its chain sum there instead.
-template <int TA, int TB, int WB, int KT, int G, bool WIDE>
+template <int TA, int TB, int WB, int KT, int G, bool WIDE, bool DEEP>
 __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_kernel(F64Args ar) {
     using Cf = F64Cfg<WB, KT>;
     constexpr int TILE = Cf::TILE, NLD = Cf::NLD;
     constexpr int SZA = TA == 0 ? Cf::SZ_K : Cf::SZ_R, SZB = TB == 1 ? Cf::SZ_K : Cf::SZ_R;
     constexpr int SPB = F64_KC / KT;             // stages per block
     static_assert(SPB % 2 == 0, "stages run in pairs");
+    static_assert(DEEP || G == 1, "stage by stage: no groups");
     static_assert(G == 1 || SZA + SZB >= TILE * TILE, "a stage buffer holds a group's chain sums");
     __shared__ __attribute__((aligned(16))) double lds[G][2][SZA + SZB];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -260,7 +262,7 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
     };
     auto stash = [&](auto set_c, int q) {
         constexpr int set = decltype(set_c)::value;
-        double* d = lds[g][set];
+        double* d = lds[g][DEEP ? set : q & 1];
         const int valid = valid_of(q);
 #pragma unroll
         for (int r = 0; r < NLD; ++r) {
@@ -283,9 +285,9 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
     const int kr0 = lane >> 4, c0 = lane & 15;
     auto step = [&](auto set_c, int q) {   // stage q from LDS buffer q % 2 = set
         constexpr int set = decltype(set_c)::value;
-        fetch(set_c, q + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        const double* as = lds[g][set];
+        fetch(set_c, q + (DEEP ? 2 : 1));
+        if (DEEP) __builtin_amdgcn_sched_barrier(0);
+        const double* as = lds[g][DEEP ? set : q & 1];
         const double* bs = as + SZA;
         double a[KT / 4][WB], bb[KT / 4][WB];
 #pragma unroll
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
         // One block per wave: a dependent chain of products; with the reads between them each
         // pair waited for its own LDS latency (200 cycles a product instead of 64), so a
         // stage's reads all go first.
-        if (WB == 1) __builtin_amdgcn_sched_barrier(0);
+        if (DEEP && WB == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k4 = 0; k4 < KT / 4; ++k4)
 #pragma unroll
@@ -311,26 +313,29 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
                     acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k4][i], bb[k4][j], acc[i][j], 0, 0, 0);
         // stage q + 1, fetched a step ago; kept behind the products (the scheduler would move its
         // wait to the front, and the loads would have one stage to land instead of two)
-        __builtin_amdgcn_sched_barrier(0);
-        stash(std::integral_constant<int, set ^ 1>{}, q + 1);
+        if (DEEP) __builtin_amdgcn_sched_barrier(0);
+        stash(std::integral_constant<int, DEEP ? set ^ 1 : 0>{}, q + 1);
         __syncthreads();
     };
-    // Stages run in pairs (a pair's second stage past the end multiplies zeros), so the loop
-    // has no branch around the accumulators; the blocks of 256 k are an outer loop, which adds
-    // their chain sums in k order.
+    // A pair's second stage past the end multiplies zeros, so the loop has no branch around the
+    // accumulators; the blocks of 256 k are an outer loop, which adds their chain sums in k order.
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
     if (q0 < nq) {
         fetch(even, q0);
-        fetch(odd, q0 + 1);
+        if (DEEP) fetch(odd, q0 + 1);
         stash(even, q0);
         __syncthreads();
     }
     for (int q = q0; q < nq;) {
         const int qe = min(nq, (q / SPB + 1) * SPB);
-        for (; q < qe; q += 2) {
-            step(even, q);
-            step(odd, q + 1);
+        if constexpr (DEEP) {
+            for (; q < qe; q += 2) {
+                step(even, q);
+                step(odd, q + 1);
+            }
+        } else {
+            for (; q < qe; ++q) step(even, q);
         }
         if (G > 1 && !ar.part) {
             // lds[.][1] was read in the last step and is not written before the next round
@@ -524,10 +529,10 @@ __global__ __launch_bounds__(256) void attn_softmax_bwd_f64(const double* __rest
     }
 }
 
-template <int WB, int KT, int G, bool WIDE = false>
+template <int WB, int KT, int G, bool WIDE = false, bool DEEP = true>
 void launch_f64(int transA, int transB, dim3 grid, const F64Args& ar) {
 #define DH_F64_LAUNCH(TA, TB) \
-    gemm_f64_kernel<TA, TB, WB, KT, G, WIDE><<<grid, F64_THREADS * G, 0, stream()>>>(ar)
+    gemm_f64_kernel<TA, TB, WB, KT, G, WIDE, DEEP><<<grid, F64_THREADS * G, 0, stream()>>>(ar)
     if (!transA && !transB) DH_F64_LAUNCH(0, 0);
     else if (!transA) DH_F64_LAUNCH(0, 1);
     else if (!transB) DH_F64_LAUNCH(1, 0);
@@ -539,30 +544,44 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
                     int lda, long long sA, const double* B, int ldb, long long sB, double beta,
                     double* C, int ldc, long long sC, int batch, int causal = F64_ALL,
                     int row0 = 0) {
-    // 64 x 64 tiles (2 x 2 blocks per wave) when they fill the chip twice over, else 32 x 32.
+    // 64 x 64 tiles (2 x 2 blocks per wave) when they fill the chip twice over (from 1.6 times on for K
+    // of one block), else 32 x 32.  K of few stages, and 32 x 32 tiles without groups, run stage by
+    // stage: a pair of stages multiplies up to a whole stage of zeros, and with several
+    // work-groups on a CU they cover each other's loads (us, pairs / stage by stage: 2048^2 x 11 14.4 /
+    // 11.0, x 130 30.5 / 28.8, x 257 48.4 / 47.6; 1292 x 1395 x 34 13.2 / 10.3, 490 x 1561 x 11 8.2 / 6.4, 1000 x 700 x
+    // 513 26.5 / 23.3, 1000 x 700 x 1030 49.5 / 45.9; but one block per work-group and CU, 1024 x 128 x 511, 11.9 /
+    // 13.1).
     // A small grid is bound by the latencies of its work-groups' k-stages, so it runs the
-    // 256-deep blocks of k side by side: up to four groups of waves in a work-group, as many as
-    // bring a CU about 16 waves (same box, us, one group / chosen: 511^3 13.6 / 12.5, 512^2 x
-    // 1024 22.6 / 17.9, 256 x 1023 x 4096 81.9 / 58.4), or, where the tiles leave half the CUs
-    // idle, one work-group per block, whose chain sums gemm_f64_reduce adds in k order (64^2 x
-    // 4096 77.7 / 15.3, 300^2 x 1000 21.8 / 15.6; with groups 56.7 and 17.5).  Every form leaves
-    // the results bit-identical.  Leading dimensions that take a tile past 32-bit
-    // offsets (2^22 to 2^24, see `wide`) have forms with 64-bit ones.
+    // 256-deep blocks of k side by side: one work-group per block, whose chain sums gemm_f64_reduce
+    // adds in k order, where the tiles leave half the CUs idle (64^2 x 4096 77.7 -> 15.3, 300^2 x 1000
+    // 21.8 -> 15.6), or up to four groups of waves in a work-group, as many as fit the CUs at once
+    // (four take 135 KB of LDS, two 68 KB), whichever takes less by the two estimates below (in
+    // us, fitted to tiles of 137 to 512 and 2 to 16 blocks; one group / groups / blocks: 511^3
+    // 13.6 / 12.4 / 17.9, 500 x 300 x 1500 - / 31.7 / 22.8, 1756 x 149 x 2000 - / 51.0 / 37.4, 700^2 x 2000 - / 51.9 / 58.2).
+    // Every form leaves the results bit-identical.  Leading dimensions that take a tile past
+    // 32-bit offsets (2^22 to 2^24, see `wide`) have forms with 64-bit ones.
     const long long cus = num_cus();
-    const int wb = ((M + 63) / 64) * (long long)((N + 63) / 64) * batch >= 2 * cus ? 2 : 1;
+    const long long tiles64 = ((M + 63) / 64) * (long long)((N + 63) / 64) * batch;
+    const bool short2 = causal == F64_ALL && (tiles64 >= 2 * cus ? K <= 160 : K <= 256 && 5 * tiles64 >= 8 * cus);
+    const int wb = tiles64 >= 2 * cus || short2 ? 2 : 1;
     // rows of a tile and stage: the tile's, or its k
     const int rows_a = transA ? (wb == 2 ? 16 : 32) : 32 * wb, rows_b = transB ? 32 * wb : wb == 2 ? 16 : 32;
     const bool wide = 8LL * rows_a * lda > 0x7fffffffLL || 8LL * rows_b * ldb > 0x7fffffffLL;
     const long long tilesM = (M + 32 * wb - 1) / (32 * wb), tilesN = (N + 32 * wb - 1) / (32 * wb);
     const long long tiles = tilesM * tilesN * batch;
     const long long nkb = ((long long)K + F64_KC - 1) / F64_KC;
+    int G = 1;
+    if (wb == 1 && !wide)
+        while (G < 4 && G < nkb && tiles * G <= 2 * cus) G *= 2;
+    const double blocks_us = 7.7 + 3.7 * (double)((tiles * nkb + cus - 1) / cus);
+    const double groups_us = G == 4 ? 5.5 + 13.2 * (double)(nkb / 4) + (nkb % 4 > 1 ? 13.2 : 3.7 * (nkb % 4))
+                           : tiles <= cus ? 12.0 : 6.2 + 11.3 * (double)(nkb / 2) + (nkb % 2 ? 3.5 + 0.028 * ((K - 1) % F64_KC) : 0.0);
     const size_t pbytes = (size_t)nkb * batch * M * N * sizeof(double);
     double* part = nullptr;
-    if (nkb > 1 && nkb <= 65535 && 2 * tiles <= cus && pbytes <= ((size_t)512 << 20))
+    if (nkb > 1 && nkb <= 65535 && pbytes <= ((size_t)512 << 20) &&
+        (2 * tiles <= cus || (G > 1 && blocks_us < groups_us)))
         part = static_cast<double*>(dh_malloc(pbytes));   // none: the unsplit grid
-    int G = 1;
-    if (wb == 1 && !wide && !part)
-        while (G < 4 && G < nkb && tiles * G < 4 * cus) G *= 2;
+    if (part) G = 1;
     const long long o = (row0 + 32 * wb - 1) / (32 * wb);   // F64_SCORES: visible tiles only
     const dim3 grid((unsigned)(causal == F64_SCORES ? tilesM * (tilesM + 1) / 2 + tilesM * o
                                                     : tilesM * tilesN),
@@ -570,10 +589,14 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
                     part ? (unsigned)nkb : 1u);
     const F64Args ar{M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, (int)tilesN, part,
                      causal, row0, (int)cus};
-    if (wide && wb == 2) launch_f64<2, 16, 1, true>(transA, transB, grid, ar);
-    else if (wide) launch_f64<1, 32, 1, true>(transA, transB, grid, ar);
+    if (wide && wb == 2) launch_f64<2, 16, 1, true, false>(transA, transB, grid, ar);
+    else if (wide) launch_f64<1, 32, 1, true, false>(transA, transB, grid, ar);
+    else if (short2) launch_f64<2, 16, 1, false, false>(transA, transB, grid, ar);
     else if (wb == 2) launch_f64<2, 16, 1>(transA, transB, grid, ar);
-    else if (G == 1) launch_f64<1, 32, 1>(transA, transB, grid, ar);
+    else if (G == 1 && !part && causal == F64_ALL && (K <= 16 || (K > 32 && K <= 48)))
+        launch_f64<1, 16, 1, false, false>(transA, transB, grid, ar);
+    else if (part && tiles * nkb <= cus) launch_f64<1, 32, 1>(transA, transB, grid, ar);
+    else if (G == 1) launch_f64<1, 32, 1, false, false>(transA, transB, grid, ar);
     else if (G == 2) launch_f64<1, 32, 2>(transA, transB, grid, ar);
     else launch_f64<1, 32, 4>(transA, transB, grid, ar);
     if (part) {

@@ -247,10 +247,12 @@ def test_attention_f64_query_row_blocks(causal, monkeypatch):
 
 @pytest.mark.parametrize("M,N,K", [(511, 511, 511), (500, 330, 1030), (256, 257, 2051),
                                    (65, 31, 1300), (1, 1, 513), (33, 64, 33), (32, 96, 32),
-                                   (1450, 1500, 47), (1500, 1450, 271)])
+                                   (1450, 1500, 47), (1500, 1450, 271), (490, 1561, 11), (700, 690, 35),
+                                   (1292, 1395, 29), (2048, 1030, 100), (900, 300, 700), (350, 600, 1500),
+                                   (640, 500, 1030)])
 def test_gemm_f64_forms_are_bit_identical(M, N, K):
-    # One, two and four groups of waves per tile, blocks of k over work-groups, 64-wide tiles;
-    # ragged stages, odd leading dimensions (pairs across a row's end), rows past the edge.
+    # One, two and four groups of waves per tile, blocks of k over work-groups (also with more
+    # tiles than CUs), 64-wide tiles, each in pairs of stages or stage by stage, of 16 and 32 k; ragged stages, odd leading dimensions (pairs across a row's end), rows past the edge.
     # Every layout runs the reference's chains, so all four equal the oracle bit for bit.
     rng = np.random.default_rng(M * N + K)
     A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
