@@ -49,8 +49,11 @@ typedef double f64x2 __attribute__((ext_vector_type(2)));
 //   F64_SCORES     C[m][n]: tiles whose keys n all lie past their queries row0 + m are left out;
 //   F64_TO_DIAG    A[m][k] masked past k = row0 + m: k stops at the end of the tile's queries;
 //   F64_FROM_DIAG  A^T[m][k] (m a key, k a query row0 + k): k starts at the tile's first key.
-// A masked product is an exact zero, and adding it changes no chain, so the results are those
-// of the full product.  The row kernels write zeros up to F64_PAD keys past the diagonal, as
+// A masked product of finite values is an exact zero, and adding it changes no chain.  Within a
+// tile and a stage of the diagonal it is formed all the same: a masked zero times an infinity or
+// NaN makes a NaN there, and outputs that are NaN are formed again from their visible k
+// (f64_visible).  So every output depends on what its queries and keys see, as in the
+// reference's loops, whatever the tile.  The row kernels write zeros up to F64_PAD keys past the diagonal, as
 // far as a tile's edge and a stage's start reach.
 enum { F64_ALL = 0, F64_SCORES, F64_TO_DIAG, F64_FROM_DIAG };
 constexpr int F64_PAD = 80;       // 64-wide tile + 16-deep stage (or 32 + 32)
@@ -93,6 +96,22 @@ struct F64Args {
     double* part;                 // split mode: the chain sums' buffer
     int causal, row0, snake;
 };
+
+// One output of a causal product from its visible k alone, k0 .. k1 - 1: the chains and block sums
+// of the kernel below.
+template <int TA>
+__device__ inline double f64_visible(const F64Args& ar, long long b, int m, int n, int k0, int k1) {
+    GlobalF64 A = (GlobalF64)(ar.A + b * ar.sA), B = (GlobalF64)(ar.B + b * ar.sB);
+    double sum = 0.0;
+    for (int kb = k0 / F64_KC * F64_KC; kb < k1; kb += F64_KC) {
+        double c = 0.0;
+        for (int k = max(k0, kb); k < min(k1, kb + F64_KC); ++k)
+            c = __builtin_fma(A[TA == 0 ? (long long)m * ar.lda + k : (long long)k * ar.lda + m],
+                              B[(long long)k * ar.ldb + n], c);
+        sum = sum + c;
+    }
+    return sum;
+}
 
 template <int WB, int KT>
 struct F64Cfg {
@@ -382,6 +401,24 @@ __global__ __launch_bounds__(F64_THREADS * G, WB == 2 ? 4 : 1) void gemm_f64_ker
     const int block = blockIdx.z * G + g;   // split mode: this group's block
     if (ar.part ? block * F64_KC >= K : g > 0) return;
     // lane l, register r of block (i, j): row wr + 16 i + l / 16 + 4 r, column wc + 16 j + l % 16
+    if (TB == 0 && ar.causal >= F64_TO_DIAG) {
+#pragma unroll
+        for (int i = 0; i < WB; ++i)
+#pragma unroll
+            for (int j = 0; j < WB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int gm = m0 + wr + 16 * i + kr0 + 4 * r, gn = n0 + wc + 16 * j + c0;
+                    if (tot[i][j][r] == tot[i][j][r] || gm >= M || gn >= N) continue;
+                    int k0 = ar.causal == F64_TO_DIAG ? 0 : max(0, gm - ar.row0);
+                    int k1 = ar.causal == F64_TO_DIAG ? min(K, ar.row0 + gm + 1) : K;
+                    if (ar.part) {
+                        k0 = max(k0, block * F64_KC);
+                        k1 = min(k1, (block + 1) * F64_KC);
+                    }
+                    tot[i][j][r] = f64_visible<TA>(ar, b, gm, gn, k0, k1);
+                }
+    }
     double* out = ar.part ? ar.part + ((long long)block * gridDim.y + b) * ((long long)M * N)
                           : ar.C + b * ar.sC;
     const long long ld = ar.part ? N : ar.ldc;

@@ -314,3 +314,30 @@ def test_attention_f64_causal_leaves_masked_scores_alone(B, S, D, rows, monkeypa
     ref = O.attention_bwd(Q, K, V, G, B, S, D, True)
     for g, r in zip(attn64_bwd(Q, K, V, G, B, S, D, True), ref):
         assert maxrel(g, r) <= 1e-11
+
+
+@pytest.mark.parametrize("B,S,D,rows", [(2, 70, 24, 0), (1, 600, 16, 0), (8, 600, 40, 0), (40, 300, 64, 0),
+                                        (2, 330, 24, 77)])
+@pytest.mark.parametrize("which", ["Q", "K", "V", "dO"])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_attention_f64_causal_nonfinite_values_reach_visible_rows_only(B, S, D, rows, which, bad, monkeypatch):
+    """An infinity or NaN of one row reaches the outputs that see the row, whatever tile they lie in,
+    and no others: non-finite in the same places as the oracle's loops over visible keys, the
+    rest within the bounds of the tests above.  One value of a row in slice 0, near a tile's start and
+    inside one; 32- and 64-wide tiles, groups, blocks over work-groups, query-row passes."""
+    if rows:
+        monkeypatch.setenv("DH_ATTN_F64_SCORE_BYTES", str(rows * S * 8))
+    rng = np.random.default_rng(S + D)
+    T = {n: rng.standard_normal((B, S * D)) for n in ("Q", "K", "V", "dO")}
+    for row in (S // 2 + 7, 3):
+        X = {n: x.copy() for n, x in T.items()}
+        X[which][0, row * D + 5] = bad
+        with np.errstate(all="ignore"):
+            want = [O.attention(X["Q"], X["K"], X["V"], B, S, D, True),
+                    *O.attention_bwd(X["Q"], X["K"], X["V"], X["dO"], B, S, D, True)]
+        got = [attn64(X["Q"], X["K"], X["V"], B, S, D, True),
+               *attn64_bwd(X["Q"], X["K"], X["V"], X["dO"], B, S, D, True)]
+        for g, w, tol in zip(got, want, (1e-12, 1e-11, 1e-11, 1e-11)):
+            ok = np.isfinite(w)
+            assert np.array_equal(np.isfinite(g), ok)
+            assert not ok.any() or maxrel(g[ok], w[ok]) <= tol
