@@ -660,7 +660,10 @@ struct ConvGeom {
 // B slice of the implicit GEMM: rows k0 .. k0 + BK of col_n, columns t0 .. t0 + TILE.  A wave's
 // lanes take consecutive columns of one row, so a row's decomposition into (ci, kh, kw) is
 // wave-uniform and runs on the scalar unit, and a thread keeps one column, whose window origin
-// is computed once per tile.  What is left per element for the vector unit, which shares the
+// is computed once per tile.  The scalar unit takes a slice's rows one step ahead, among the
+// products before it: at the head of a step its chain held the loads and products back (data
+// gradient of 16 images 82 x 48 x 48 -> 3, 3 x 3: 63.2 -> 59.5 us, 5 x 5 158 -> 147; forward of 64 images
+// 3 x 112 x 112 -> 64, 5 x 5, 128 -> 123).  What is left per element for the vector unit, which shares the
 // SIMD's issue with the MFMAs, are two sums, two compares and the offset.  Every element is one
 // 32-bit-offset buffer load of the image's planes: byte offset = 4 (tap term of its row + pixel
 // term of its column); a tap outside the input takes an offset past the buffer's range, which
@@ -686,18 +689,28 @@ struct ConvSlice {
         hb = p < P ? h0 : -(1 << 30);   // a column past P: h < 0
         row = __builtin_amdgcn_readfirstlane(tid / TILE);
     }
-    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int R, int k0) {
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(X), 0, (int)(4u * g.Cin * g.H * g.W), 0x00020000);
+    struct Rows {   // the decomposed rows of a slice
+        int kh[CH], kw[CH], tap[CH];
+    };
+    __device__ void rows(const ConvGeom& g, int R, int k0, Rows& d) const {
 #pragma unroll
         for (int r = 0; r < CH; ++r) {
             const int k = k0 + row + RSTEP * r;
             const int q = (int)fdiv((uint32_t)k, g.f_kw), kw = k - q * g.KW;
             const int ci = (int)fdiv((uint32_t)k, g.f_khkw);
-            const int kh = k < R ? q - ci * g.KH : -(1 << 30);   // a row past R: h < 0
-            const int tap = 4 * ((ci * g.H + q - ci * g.KH) * g.W + kw);
-            const bool in = (unsigned)(hb + kh) < (unsigned)g.H && (unsigned)(wb + kw) < (unsigned)g.W;
-            const uint32_t off = in ? (uint32_t)(tap + pix) : CONV_OOB;
+            d.kh[r] = k < R ? q - ci * g.KH : -(1 << 30);   // a row past R: h < 0
+            d.kw[r] = kw;
+            d.tap[r] = 4 * ((ci * g.H + q - ci * g.KH) * g.W + kw);
+        }
+    }
+    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int, int, const Rows& d) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(X), 0, (int)(4u * g.Cin * g.H * g.W), 0x00020000);
+#pragma unroll
+        for (int r = 0; r < CH; ++r) {
+            const bool in = (unsigned)(hb + d.kh[r]) < (unsigned)g.H &&
+                            (unsigned)(wb + d.kw[r]) < (unsigned)g.W;
+            const uint32_t off = in ? (uint32_t)(d.tap[r] + pix) : CONV_OOB;
             v[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
         }
     }
@@ -714,7 +727,9 @@ struct ConvSlice {
 template <int TILE>
 struct ConvTapSlice : ConvSlice<TILE> {
     using Base = ConvSlice<TILE>;
-    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int R, int k0) {
+    struct Rows {};
+    __device__ void rows(const ConvGeom&, int, int, Rows&) const {}
+    __device__ void fetch(const float* __restrict__ X, const ConvGeom& g, int R, int k0, const Rows&) {
         const int t = (int)fdiv((uint32_t)k0 / BK, g.f_nc);
         const int kq = (int)fdiv((uint32_t)t, g.f_kw), kw = t - kq * g.KW;
         const int c0 = k0 - t * ((int)g.f_nc.d * BK) + Base::row;
@@ -779,9 +794,13 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
 
     const int nk = (Re - kb + BK - 1) / BK;   // >= 1
     sa[0].fetch(Kn, R, m0, kb, Cout, Re, tid);
-    sb[0].fetch(X, g, Re, kb);
+    typename std::remove_reference_t<decltype(sb[0])>::Rows rows;
+    sb[0].rows(g, Re, kb, rows);
+    sb[0].fetch(X, g, Re, kb, rows);
     sa[1].fetch(Kn, R, m0, kb + BK, Cout, Re, tid);
-    sb[1].fetch(X, g, Re, kb + BK);
+    sb[1].rows(g, Re, kb + BK, rows);
+    sb[1].fetch(X, g, Re, kb + BK, rows);
+    sb[0].rows(g, Re, kb + 2 * BK, rows);
     sa[0].store(As[0], LDS_A, tid);
     sb[0].store(Bs[0], LDS_B, tid);
     __syncthreads();
@@ -804,7 +823,8 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     auto step = [&](auto cur_c, int kt) {
         constexpr int cur = decltype(cur_c)::value;
         sa[cur].fetch(Kn, R, m0, kb + (kt + 2) * BK, Cout, Re, tid);
-        sb[cur].fetch(X, g, Re, kb + (kt + 2) * BK);
+        sb[cur].fetch(X, g, Re, kb + (kt + 2) * BK, rows);
+        sb[cur].rows(g, Re, kb + (kt + 3) * BK, rows);   // under this slice's products
         mma(As[cur], Bs[cur]);
         sa[cur ^ 1].store(As[cur ^ 1], LDS_A, tid);
         sb[cur ^ 1].store(Bs[cur ^ 1], LDS_B, tid);
@@ -1658,12 +1678,11 @@ constexpr double CONV_PACK_FLOPS = 1e9;
 int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, ConvGeom g, float* Y,
              const float* bias, int accumulate, bool flip) {
     const int cus = num_cus(), win = g.KH * g.KW;
-    const bool scratch = !capturing();
     long long R = (long long)g.Cin * win;
     const int cp = (g.Cin + BK - 1) / BK * BK;
     bool taps = 8ll * (cp - g.Cin) <= g.Cin && (long long)win * cp <= LD_BUF_MAX &&
                 (long long)Cout * win * cp <= 1ll << 30 &&
-                (flip || (scratch && 2.0 * N * Cout * P * R >= CONV_PACK_FLOPS));
+                (flip || (2.0 * N * Cout * P * R >= CONV_PACK_FLOPS && !capturing()));
     float* Kt = nullptr;
     if (taps || flip) {
         Kt = static_cast<float*>(dh_malloc((size_t)Cout * (taps ? (long long)win * cp : R) * sizeof(float)));
@@ -1684,7 +1703,7 @@ int run_conv(int N, int Cout, long long P, const float* Kn, const float* X, Conv
     int S = 1;
     float* part = nullptr;
     const size_t n = (size_t)N * Cout * P;
-    if (scratch && 2 * t64 <= cus && R >= 16 * BK) {
+    if (2 * t64 <= cus && R >= 16 * BK && !capturing()) {
         S = (int)std::min<long long>(2 * cus / t64, R / (8 * BK));
         const int nk = (int)((R + BK - 1) / BK), kz = (nk + S - 1) / S;
         S = (nk + kz - 1) / kz;   // no empty chunks
