@@ -19,8 +19,10 @@
 //   B[k = l / 32][j = l % 32]; accumulator register r of lane l holds
 //   C[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32].
 // Edges: rows/cols beyond M, N and K are loaded as zeros and never stored, so any
-//   shape is exact.  When a matrix's leading dimension and base address allow it the
-//   contiguous dimension is fetched with 128-bit loads.
+//   shape is exact.  The contiguous dimension is fetched with 128-bit loads at any alignment
+//   (LD_BUF below), but for leading dimensions above 2^20 only where it is aligned.
+// Grids that such tiles leave idle: 64 x 64 tiles, or 32 x 32 with k split over a work-group's
+//   waves (gemm_f32_wave_kernel).
 #include <type_traits>
 
 #include "dh_common.hpp"
@@ -1229,8 +1231,8 @@ int launch_split(int M, int N, int K, int S, const float* A, int lda, const floa
     if (!part) return DH_ERR_UNSUPPORTED;
     // chunk j: A columns (or rows, TA) and B rows (or columns, TB) j Kc .. + Kc; the last
     // chunk K - (S - 1) Kc.  One grid, so the chunks run side by side.  The kernel choice sees
-    // the whole K: 16-byte loads along k only where K is a multiple of 4, so that a ragged last
-    // chunk has no 4-wide group crossing its end.
+    // the whole K: the forms without a mask along k (LD_BUF4, LD_VEC) only where it is a multiple
+    // of 4, as then the last chunk's is.
     const long long sA = TA ? (long long)Kc * lda : Kc, sB = TB ? Kc : (long long)Kc * ldb;
     auto kern = pick(sA, sB);
     kern<<<dim3(tiles, S), threads, 0, s>>>(M, N, Kc, A, lda, B, ldb, 0.f, part, N, sA, sB,

@@ -609,13 +609,14 @@ def test_bf16_ragged_k_tail_keeps_nonfinite_values_in_their_row():
     assert maxrel(got[rows], A64[rows] @ B64) <= 1e-5 * np.sqrt(K)
 
 
-# The 128 x 128 direct-to-LDS path: shapes whose 256 x 256 tiles do not make one round of
-# the CUs.  1..5 stages of 32 k (ring fill and drain), K tails, ragged edge tiles, a grid
-# of more than two tiles per CU (3000^2), one-tile and one-row products, and split K (at most
-# half the CUs' worth of tiles and K >= 2048: 784 x 257 x 4096, 512^2 x 8192, 300 x 200 x 2048,
-# 1000 x 700 x 2100, chunks whose last one takes the rest of K); every element against fp64
-# on the bf16-rounded inputs.
-MID = [(2048, 2048, 2048), (128, 128, 32), (256, 384, 64), (129, 255, 96), (300, 200, 128),
+# The direct-to-LDS paths of smaller tiles: shapes whose 256 x 256 tiles do not make half a round
+# of the CUs.  128 x 128 tiles (more than three 64-wide ones per CU): 2048^2, 2000 x 1900 (a K tail of
+# 8, edge tiles), 1200 x 3000 x 50 (one stage and a tail), 3000 x 2000 x 160 (a full ring); 64 x 64 tiles:
+# one to three stages, edge tiles, one-tile and one-row products, copied rows and, where the
+# tiles fill at most half the CUs with K >= 2048, split K (784 x 257 x 4096, 512^2 x 8192,
+# 300 x 200 x 2048; 1000 x 700 x 2100 has chains but no split).  3000^2 x 500 is on the 256 x 256 side of
+# the line.  Every element against fp64 on the bf16-rounded inputs.
+MID = [(1200, 3000, 50), (3000, 2000, 160), (2048, 2048, 2048), (128, 128, 32), (256, 384, 64), (129, 255, 96), (300, 200, 128),
        (1000, 1900, 160), (2000, 1900, 1000), (3000, 3000, 500), (1, 64, 64), (70, 1, 33),
        (4096, 10, 257), (784, 257, 4096), (512, 512, 8192), (300, 200, 2048), (1000, 700, 2100)]
 
@@ -634,7 +635,10 @@ def test_bf16_mid_path(M, N, K, ta, tb):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)
 
 
-@pytest.mark.parametrize("Bt,M,N,K", [(3, 500, 300, 200), (2, 1024, 1024, 97), (1, 256, 384, 4099)])
+# 64-wide tiles, the general kernel (batched odd rows), split K; 128-wide tiles: 972 and 972
+# 64-wide ones, K without and with a tail
+@pytest.mark.parametrize("Bt,M,N,K", [(3, 500, 300, 200), (2, 1024, 1024, 97), (1, 256, 384, 4099),
+                                      (3, 1104, 1096, 192), (3, 1104, 1096, 200)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
 @pytest.mark.parametrize("relu,row_bias", [(False, False), (True, False), (True, True)])
 def test_bf16_mid_path_batched_epilogue(Bt, M, N, K, ta, tb, relu, row_bias):
@@ -643,8 +647,10 @@ def test_bf16_mid_path_batched_epilogue(Bt, M, N, K, ta, tb, relu, row_bias):
     assert maxrel(got, ref) <= 1e-5 * np.sqrt(K)
 
 
-def test_bf16_mid_path_k_tail_keeps_nonfinite_values_in_their_row():
-    M, N, K = 1000, 900, 300
+# 64-wide tiles on copied rows; 128-wide tiles on aligned ones, whose masked K tail of 8 lies
+# before the next row's NaN or infinity
+@pytest.mark.parametrize("M,N,K", [(1000, 900, 300), (2000, 1904, 296)])
+def test_bf16_mid_path_k_tail_keeps_nonfinite_values_in_their_row(M, N, K):
     rng = np.random.default_rng(6)
     Af = rng.standard_normal((M, K), dtype=np.float32)
     Af[500, K - 1] = np.nan

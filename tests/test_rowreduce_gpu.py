@@ -4,8 +4,8 @@ Row ops: dh_row_softmax (softmax / log_softmax), dh_row_softmax_bwd, dh_layer_no
 dh_layer_norm_bwd.  Tolerance: max |got - ref| <= 1e-5 * sqrt(C) * max(1, max |ref|) against the
 fp64 oracle on the same fp32 inputs (C = row length, the reduction length); the reference's
 own golden vectors are checked at the same bound.  Shapes cover every kernel form: segments
-of 4, 16 and 64 lanes with 4-value and 1-value chunks (C % 4 == 0 or not) and the streaming
-long-row kernels (C > 1024), plus accumulate on and off.
+of 4, 16 and 64 lanes, one work-group per row in registers (1024 < C <= 32768) and the streaming
+kernels above, rows that start and end inside a 16-byte chunk, plus accumulate on and off.
 """
 import os
 
