@@ -1539,7 +1539,9 @@ int launch_ks(int M, int N, int K, const float* A, int lda, const float* B, int 
 // from 128 x 128 x 64 to 1500^3): a CU takes 0.16 us per tile and 32-deep slice, 0.185 with
 // several tiles on it, a work-group's slices rounded up to its waves; a 64 x 64 tile takes
 // 0.0185 us per k, and the grid as many as its fullest CU (past one 128 x 128 tile per CU the
-// larger tiles are always better).  Few tiles with a long K also split K over work-groups (6 us
+// larger tiles are always better).  A CU holds four work-groups, and past 4.5 tiles on each the rest
+// runs at low occupancy, which the estimate does not see: 64 x 64 tiles there (30 x 200 x 200 x 512
+// 34.4 / 23.9, 32 x 252 x 156 x 320 22.0 / 17.4, 1400 x 1500 x 128 16.0 / 13.0).  Few tiles with a long K also split K over work-groups (6 us
 // for the second launch), where the 64 x 64 form does the same at about 0.6 of the matrix rate.
 template <bool TA, bool TB>
 int launch_wave(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta,
@@ -1549,7 +1551,8 @@ int launch_wave(int M, int N, int K, const float* A, int lda, const float* B, in
     const long long t32 = tiles * bt.count;
     const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * bt.count;
     const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * bt.count;
-    if (K < 1 || lda > LD_BUF_MAX || ldb > LD_BUF_MAX || bt.count > 65535 || t128 >= cus)
+    if (K < 1 || lda > LD_BUF_MAX || ldb > LD_BUF_MAX || bt.count > 65535 || t128 >= cus ||
+        2 * t32 > 9 * cus)
         return DH_ERR_UNSUPPORTED;
     auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
     auto wave_us = [&](int S, int nw) {
