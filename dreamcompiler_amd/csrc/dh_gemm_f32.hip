@@ -108,6 +108,8 @@ struct Slice {
                 const int c = 4 * (KCONTIG ? f % (BKT / 4) : f % (TILE / 4));
                 int off = 4 * (row * ld + c);
                 if (LD == LD_BUF4 && KCONTIG) off = c < left ? off : -16;
+                // a chunk past the tile's columns: no traffic (64 x 100 x 100 x 800 TN 26.9 -> 24.3 us)
+                if (!KCONTIG) off = c < cols ? off : -16;
                 asm volatile("" : "+v"(off));   // one 128-bit load: constant distances from off
                 float x[4];
                 buf_load_floats<4>(rs, off, x);
@@ -1541,7 +1543,8 @@ int launch_ks(int M, int N, int K, const float* A, int lda, const float* B, int 
 // 0.0185 us per k, and the grid as many as its fullest CU (past one 128 x 128 tile per CU the
 // larger tiles are always better).  A CU holds four work-groups, and past 4.5 tiles on each the rest
 // runs at low occupancy, which the estimate does not see: 64 x 64 tiles there (30 x 200 x 200 x 512
-// 34.4 / 23.9, 32 x 252 x 156 x 320 22.0 / 17.4, 1400 x 1500 x 128 16.0 / 13.0).  Few tiles with a long K also split K over work-groups (6 us
+// 34.4 / 23.9, 32 x 252 x 156 x 320 22.0 / 17.4, 1400 x 1500 x 128 16.0 / 13.0).
+// Few tiles with a long K also split K over work-groups (6 us
 // for the second launch), where the 64 x 64 form does the same at about 0.6 of the matrix rate.
 template <bool TA, bool TB>
 int launch_wave(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float beta,
