@@ -664,8 +664,8 @@ struct ConvGeom {
 // B slice of the implicit GEMM: rows k0 .. k0 + BK of col_n, columns t0 .. t0 + TILE.  A wave's
 // lanes take consecutive columns of one row, so a row's decomposition into (ci, kh, kw) is
 // wave-uniform and runs on the scalar unit, and a thread keeps one column, whose window origin
-// is computed once per tile.  The scalar unit takes a slice's rows one step ahead, among the
-// products before it: at the head of a step its chain held the loads and products back (data
+// is computed once per tile.  On grids that share CUs (launch_conv) the scalar unit takes a
+// slice's rows one step ahead, among the products before it: at the head of a step its chain held the loads and products back (data
 // gradient of 16 images 82 x 48 x 48 -> 3, 3 x 3: 63.2 -> 59.5 us, 5 x 5 158 -> 147; forward of 64 images
 // 3 x 112 x 112 -> 64, 5 x 5, 128 -> 123).  What is left per element for the vector unit, which shares the
 // SIMD's issue with the MFMAs, are two sums, two compares and the offset.  Every element is one
@@ -758,7 +758,7 @@ struct ConvTapSlice : ConvSlice<TILE> {
 // blockIdx.z (one chunk, or partial results that conv_split_reduce adds), A = the kernel matrix
 // Cout x R (k contiguous), epilogue: + bias[co] (+ the old Y with accumulate), stored into
 // Y's (N, Cout, OH OW) layout.
-template <int TBM, int TBN, int VA, bool TAP>
+template <int TBM, int TBN, int VA, bool TAP, bool AHEAD>
 __global__ void __launch_bounds__(NTHREADS)
 conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const float* __restrict__ X,
                 ConvGeom g, float* __restrict__ Y, const float* __restrict__ bias, int z0,
@@ -804,7 +804,7 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     sa[1].fetch(Kn, R, m0, kb + BK, Cout, Re, tid);
     sb[1].rows(g, Re, kb + BK, rows);
     sb[1].fetch(X, g, Re, kb + BK, rows);
-    sb[0].rows(g, Re, kb + 2 * BK, rows);
+    if (AHEAD) sb[0].rows(g, Re, kb + 2 * BK, rows);
     sa[0].store(As[0], LDS_A, tid);
     sb[0].store(Bs[0], LDS_B, tid);
     __syncthreads();
@@ -827,8 +827,9 @@ conv_fwd_kernel(int Cout, int P, int R, const float* __restrict__ Kn, const floa
     auto step = [&](auto cur_c, int kt) {
         constexpr int cur = decltype(cur_c)::value;
         sa[cur].fetch(Kn, R, m0, kb + (kt + 2) * BK, Cout, Re, tid);
+        if (!AHEAD) sb[cur].rows(g, Re, kb + (kt + 2) * BK, rows);
         sb[cur].fetch(X, g, Re, kb + (kt + 2) * BK, rows);
-        sb[cur].rows(g, Re, kb + (kt + 3) * BK, rows);   // under this slice's products
+        if (AHEAD) sb[cur].rows(g, Re, kb + (kt + 3) * BK, rows);
         mma(As[cur], Bs[cur]);
         sa[cur ^ 1].store(As[cur ^ 1], LDS_A, tid);
         sb[cur ^ 1].store(Bs[cur ^ 1], LDS_B, tid);
@@ -887,12 +888,21 @@ int launch_conv(int N, int Cout, int P, int R, const float* Kn, const float* X,
     // kernel rows of any alignment by 16-byte buffer loads; longer than 32-bit offsets reach: with
     // 64-bit addresses, 16 bytes at a time where aligned
     const bool vec = R % 4 == 0 && (uintptr_t)Kn % 16 == 0;
-    auto kern = taps             ? conv_fwd_kernel<TBM, TBN, LD_BUF4, true>
-              : R <= LD_BUF_MAX  ? (R % 4 == 0 ? conv_fwd_kernel<TBM, TBN, LD_BUF4, false>
-                                               : conv_fwd_kernel<TBM, TBN, LD_BUF, false>)
-              : vec              ? conv_fwd_kernel<TBM, TBN, LD_VEC, false>
-                                 : conv_fwd_kernel<TBM, TBN, LD_SCALAR, false>;
     const int tiles = ((Cout + TBM - 1) / TBM) * ((P + TBN - 1) / TBN);
+    // rows a step ahead where more than two work-groups share a CU; with fewer the chain is the
+    // wave's own either way, and longer (8 images 16 x 28 x 28 -> 16 9.5 / 9.7 us, 4 images
+    // 28 x 14 x 14 -> 30 13.6 / 14.2)
+    const bool ahead = (long long)tiles * N * S > 2LL * num_cus();
+    auto pick = [&](auto a) {
+        constexpr bool AH = decltype(a)::value;
+        return R <= LD_BUF_MAX ? (R % 4 == 0 ? conv_fwd_kernel<TBM, TBN, LD_BUF4, false, AH>
+                                             : conv_fwd_kernel<TBM, TBN, LD_BUF, false, AH>)
+             : vec             ? conv_fwd_kernel<TBM, TBN, LD_VEC, false, AH>
+                               : conv_fwd_kernel<TBM, TBN, LD_SCALAR, false, AH>;
+    };
+    auto kern = taps  ? conv_fwd_kernel<TBM, TBN, LD_BUF4, true, false>
+              : ahead ? pick(std::true_type{})
+                      : pick(std::false_type{});
     const int nk = (R + BK - 1) / BK, kz = (nk + S - 1) / S;
     for (int z0 = 0; z0 < N; z0 += 65535) {
         const dim3 grid(tiles, N - z0 < 65535 ? N - z0 : 65535,
