@@ -397,14 +397,16 @@ __global__ void __launch_bounds__(256) bias_grad_partial(const float* __restrict
         for (int i0 = blockIdx.y + P * w; i0 < N; i0 += 4 * P * BG_ROWS) {
             float g[BG_ROWS], y[BG_ROWS];
 #pragma unroll
-            for (int r = 0; r < BG_ROWS; ++r) {
+            for (int r = 0; r < BG_ROWS; ++r) {   // past the end: row i0 again, so no branch per load
                 const long long i = i0 + 4LL * P * r;
-                g[r] = i < N ? dY[(size_t)i * out + col] : 0.f;
-                y[r] = relu && i < N ? Y[(size_t)i * out + col] : 1.f;
+                const size_t e = (size_t)(i < N ? i : i0) * out + col;
+                g[r] = dY[e];
+                y[r] = relu ? Y[e] : 1.f;
             }
 #pragma unroll
             for (int r = 0; r < BG_ROWS; ++r) {
                 const long long i = i0 + 4LL * P * r;
+                if (i >= N) break;
                 if (!(y[r] > 0.f)) {   // the reference zeroes dY where Y <= 0, in place
                     g[r] = 0.f;
                     dY[(size_t)i * out + col] = 0.f;
