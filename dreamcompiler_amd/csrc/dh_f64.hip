@@ -610,7 +610,7 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
     int G = 1;
     if (wb == 1 && !wide)
         while (G < 4 && G < nkb && tiles * G <= 2 * cus) G *= 2;
-    const double blocks_us = 7.7 + 3.7 * (double)((tiles * nkb + cus - 1) / cus);
+    const double blocks_us = 7.7 + 3.8 * (double)(tiles * nkb) / (double)cus;
     const double groups_us = G == 4 ? 5.5 + 13.2 * (double)(nkb / 4) + (nkb % 4 > 1 ? 13.2 : 3.7 * (nkb % 4))
                            : tiles <= cus ? 12.0 : 6.2 + 11.3 * (double)(nkb / 2) + (nkb % 2 ? 3.5 + 0.028 * ((K - 1) % F64_KC) : 0.0);
     const size_t pbytes = (size_t)nkb * batch * M * N * sizeof(double);
