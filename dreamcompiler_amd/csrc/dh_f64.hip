@@ -616,7 +616,7 @@ int gemm_f64_launch(int transA, int transB, int M, int N, int K, double alpha, c
     const size_t pbytes = (size_t)nkb * batch * M * N * sizeof(double);
     double* part = nullptr;
     if (nkb > 1 && nkb <= 65535 && pbytes <= ((size_t)512 << 20) &&
-        (2 * tiles <= cus || (G > 1 && blocks_us < groups_us)))
+        (2 * tiles <= cus || (G > 1 && blocks_us < groups_us && !capturing())))
         part = static_cast<double*>(dh_malloc(pbytes));   // none: the unsplit grid
     if (part) G = 1;
     const long long o = (row0 + 32 * wb - 1) / (32 * wb);   // F64_SCORES: visible tiles only

@@ -157,10 +157,10 @@ def _hip_runtime():
     return rt
 
 
-@pytest.mark.parametrize("case", ["conv_packed", "conv_split", "bf16_copy"])
+@pytest.mark.parametrize("case", ["conv_packed", "conv_split", "bf16_copy", "f64_blocks"])
 def test_calls_with_optional_scratch_under_stream_capture(case):
-    """conv2d's packed kernel and split contraction and the bf16 products' aligned copies are scratch for
-    speed: recorded with an empty pool, where a hipMalloc would end the capture, these calls
+    """conv2d's packed kernel and split contraction, the bf16 products' aligned copies and the blocks of
+    k of fp64 grids above half the CUs are scratch for speed: recorded with an empty pool, where a hipMalloc would end the capture, these calls
     run without.  Replayed three times with eager work on the outputs between; the eager call
     adds in another order, hence 1e-5 sqrt(terms) as for the kernels themselves."""
     rng = np.random.default_rng(3)
@@ -171,6 +171,12 @@ def test_calls_with_optional_scratch_under_stream_capture(case):
         out, terms = DB.empty((M, N), np.float32), K
         call = lambda: hip.load().dh_gemm_bf16(0, 0, M, N, K, bufs[0].ptr, K, bufs[1].ptr, N, 0.0,  # noqa: E731
                                                out.ptr, N)
+    elif case == "f64_blocks":
+        M, N, K = 500, 300, 1500
+        bufs = [DB.from_numpy(rng.standard_normal(s)) for s in ((M, K), (K, N))]
+        out, terms = DB.empty((M, N), np.float64), K
+        call = lambda: hip.load().dh_gemm_f64(0, 0, M, N, K, bufs[0].ptr, K, bufs[1].ptr, N, 0.0,  # noqa: E731
+                                              out.ptr, N)
     else:
         N, C, H = (20, 64, 28) if case == "conv_packed" else (2, 64, 14)
         bufs = [DB.from_numpy(rng.standard_normal(s).astype(np.float32))
@@ -179,7 +185,7 @@ def test_calls_with_optional_scratch_under_stream_capture(case):
         call = lambda: hip.load().dh_conv2d_fwd(bufs[0].ptr, bufs[1].ptr, None, out.ptr, N, C, H, H,  # noqa: E731
                                                 C, 3, 3, 1, 1)
     R, lib = _hip_runtime(), hip.load()
-    garbage = np.full(out.shape, 7.0, np.float32)
+    garbage = np.full(out.shape, 7.0, out.dtype)
     s, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
     assert R.hipStreamCreate(ctypes.byref(s)) == 0
     try:
